@@ -262,9 +262,9 @@ class Run:
         multi = " (k right-hand sides)" if self.B is not None else ""
         kname = {"spmv": ("k_mspmv" if self.B is not None else "k_spmv_plain") + multi,
                  "trsv_fwd": ("k_msweep<fwd>" if self.B is not None else
-                              "forward sweep (k_sweep_bulk + k_tail_prep + k_tail_solve)") + multi,
+                              "forward sweep (k_sweep_bulk + k_tail_rhs + k_tail_apply)") + multi,
                  "trsv_bwd": ("k_msweep<bwd>" if self.B is not None else
-                              "backward sweep (k_tail_solve + k_sweep_bulk)") + multi,
+                              "backward sweep (k_tail_rhs + k_tail_apply + k_sweep_bulk)") + multi,
                  "factor": "k_factor_round (all rounds)"}[dom]
         return kern, dom, kname, X
 

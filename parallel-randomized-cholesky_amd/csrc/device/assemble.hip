@@ -399,136 +399,6 @@ __global__ void k_pack_meta(int nchunks, const int *start, const int *cnt, const
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nchunks; c += gridDim.x * blockDim.x)
         meta[c] = make_int4(start[c], cnt[c], off[c], slices[c]);
 }
-// ---------------------------------------------------------------- tail split
-__device__ __forceinline__ int src_entry(const EllSrc &src, int b, int et, int &pos)
-{
-    const int e = src.eidx ? src.eidx[b + et] : b + et;
-    const int col = src.rowk ? src.rowk[e] : src.ind[e];
-    pos = src.colmap ? src.colmap[col] : col;
-    return e;
-}
-
-// One wave per tail row: entries with column position < tp0 and >= tp0.
-__global__ void k_tail_count(int ntail, int tp0, const int *order, EllSrc src, int *cnt_b, int *cnt_i)
-{
-    const int lane = lane_id();
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-    const int nwaves = gridDim.x * blockDim.x / kWave;
-    for (int q = wave; q < ntail; q += nwaves) {
-        const int row = order[tp0 + q];
-        const int b = src.ptr[row], len = src.ptr[row + 1] - b;
-        int nb = 0;
-        for (int t = lane; t < len; t += kWave) {
-            int pos;
-            (void)src_entry(src, b, t, pos);
-            nb += pos < tp0 ? 1 : 0;
-        }
-        for (int off = 32; off > 0; off >>= 1) nb += __shfl_xor(nb, off, kWave);
-        if (lane == 0) {
-            cnt_b[q] = nb;
-            cnt_i[q] = len - nb;
-        }
-    }
-}
-
-// One wave per tail row: stable compaction of the two parts (ballot ranks).
-template <typename TD>
-__global__ void k_tail_split(int ntail, int tp0, const int *order, EllSrc src, const int *ptr_b, const int *ptr_i,
-                             int *ind_b, TD *val_b, int *ind_i, TD *val_i)
-{
-    const int lane = lane_id();
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-    const int nwaves = gridDim.x * blockDim.x / kWave;
-    const TD *sval = (const TD *)src.val;
-    for (int q = wave; q < ntail; q += nwaves) {
-        const int row = order[tp0 + q];
-        const int b = src.ptr[row], len = src.ptr[row + 1] - b;
-        int ob = ptr_b[q], oi = ptr_i[q];
-        for (int base = 0; base < len; base += kWave) {
-            const int t = base + lane;
-            int pos = 0, e = 0;
-            if (t < len) e = src_entry(src, b, t, pos);
-            const bool isb = t < len && pos < tp0;
-            const bool isi = t < len && pos >= tp0;
-            const uint64_t mb = ballot(isb), mi = ballot(isi);
-            if (isb) {
-                const int o = ob + lanes_below(mb);
-                ind_b[o] = pos;
-                val_b[o] = sval[e];
-            }
-            if (isi) {
-                const int o = oi + lanes_below(mi);
-                ind_i[o] = pos - tp0;
-                val_i[o] = sval[e];
-            }
-            ob += __popcll(mb);
-            oi += __popcll(mi);
-        }
-    }
-}
-
-// One wave per tail level: widest internal row -> slices and block size.
-__global__ void k_tail_layout(int ntl, const int *lstart, const int *lcnt, int tp0, const int *ptr_i, int *slices,
-                              int *size)
-{
-    const int lane = lane_id();
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-    const int nwaves = gridDim.x * blockDim.x / kWave;
-    for (int L = wave; L < ntl; L += nwaves) {
-        const int q0 = lstart[L] - tp0, cnt = lcnt[L];
-        int w = 0;
-        for (int i = lane; i < cnt; i += kWave) {
-            const int len = ptr_i[q0 + i + 1] - ptr_i[q0 + i];
-            w = len > w ? len : w;
-        }
-        for (int off = 32; off > 0; off >>= 1) {
-            const int o = __shfl_xor(w, off, kWave);
-            w = o > w ? o : w;
-        }
-        if (lane == 0) {
-            const int G = tail_group(cnt);
-            const int sl = (w + G - 1) / G;
-            slices[L] = sl;
-            size[L] = (sl + kTailBlock - 1) / kTailBlock * kTailBlock * sweep_rows_pow2(cnt) * G;
-        }
-    }
-}
-
-template <typename TD>
-__global__ void k_tail_fill(int ntl, const int *lstart, const int *lcnt, int tp0, const int *ptr_i, const int *ind_i,
-                            const TD *val_i, const int *off, const int *slices, int pad_ind, int *ell_ind, TD *ell_val)
-{
-    const int lane = lane_id();
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-    const int nwaves = gridDim.x * blockDim.x / kWave;
-    for (int L = wave; L < ntl; L += nwaves) {
-        const int cnt = lcnt[L], q0 = lstart[L] - tp0;
-        const int P = sweep_rows_pow2(cnt), G = tail_group(cnt);
-        const int stride = P * G, o = off[L];
-        const int blk = stride * kTailBlock;
-        const int total = (slices[L] + kTailBlock - 1) / kTailBlock * blk;
-        for (int idx = lane; idx < total; idx += kWave) {
-            // idx = block * blk + lane slot * kTailBlock + u: slice block * kTailBlock + u
-            const int b0 = idx / blk, r0 = idx - b0 * blk;
-            const int t = r0 / kTailBlock, u = r0 - t * kTailBlock;
-            const int sl = b0 * kTailBlock + u;
-            const int i = t / G, g = t - i * G;
-            const int et = sl * G + g;
-            int ind = pad_ind;
-            TD v = (TD)0;
-            if (i < cnt) {
-                const int b = ptr_i[q0 + i];
-                if (et < ptr_i[q0 + i + 1] - b) {
-                    ind = ind_i[b + et];
-                    v = val_i[b + et];
-                }
-            }
-            ell_ind[o + idx] = ind;
-            ell_val[o + idx] = v;
-        }
-    }
-}
-
 __global__ void k_sweep_layout(int nchunks, const int *cnt, const int *width, int *slices, int *size)
 {
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nchunks; c += gridDim.x * blockDim.x) {
@@ -763,46 +633,6 @@ void launch_pack_meta(int nchunks, const int *start, const int *cnt, const int *
 {
     hipLaunchKernelGGL(k_pack_meta, dim3(1024), dim3(256), 0, s, nchunks, start, cnt, off, slices, meta);
 }
-
-static int waves_grid(int items)
-{
-    int g = (items + 3) / 4;
-    if (g > 16384) g = 16384;
-    return g < 1 ? 1 : g;
-}
-void launch_tail_count(int ntail, int tp0, const int *order, EllSrc src, int *cnt_b, int *cnt_i, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_tail_count, dim3(waves_grid(ntail)), dim3(256), 0, s, ntail, tp0, order, src, cnt_b, cnt_i);
-}
-template <typename TD>
-void launch_tail_split(int ntail, int tp0, const int *order, EllSrc src, const int *ptr_b, const int *ptr_i,
-                       int *ind_b, TD *val_b, int *ind_i, TD *val_i, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_tail_split<TD>, dim3(waves_grid(ntail)), dim3(256), 0, s, ntail, tp0, order, src, ptr_b,
-                       ptr_i, ind_b, val_b, ind_i, val_i);
-}
-void launch_tail_layout(int ntl, const int *lstart, const int *lcnt, int tp0, const int *ptr_i, int *slices,
-                        int *size, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_tail_layout, dim3(waves_grid(ntl)), dim3(256), 0, s, ntl, lstart, lcnt, tp0, ptr_i, slices,
-                       size);
-}
-template <typename TD>
-void launch_tail_fill(int ntl, const int *lstart, const int *lcnt, int tp0, const int *ptr_i, const int *ind_i,
-                      const TD *val_i, const int *off, const int *slices, int pad_ind, int *ell_ind, TD *ell_val,
-                      hipStream_t s)
-{
-    hipLaunchKernelGGL(k_tail_fill<TD>, dim3(waves_grid(ntl)), dim3(256), 0, s, ntl, lstart, lcnt, tp0, ptr_i, ind_i,
-                       val_i, off, slices, pad_ind, ell_ind, ell_val);
-}
-template void launch_tail_split<float>(int, int, const int *, EllSrc, const int *, const int *, int *, float *, int *,
-                                       float *, hipStream_t);
-template void launch_tail_split<double>(int, int, const int *, EllSrc, const int *, const int *, int *, double *,
-                                        int *, double *, hipStream_t);
-template void launch_tail_fill<float>(int, const int *, const int *, int, const int *, const int *, const float *,
-                                      const int *, const int *, int, int *, float *, hipStream_t);
-template void launch_tail_fill<double>(int, const int *, const int *, int, const int *, const int *, const double *,
-                                       const int *, const int *, int, int *, double *, hipStream_t);
 
 template void launch_lt_fill<float>(const AssembleArgs &, const int *, int *, float *, float *, hipStream_t);
 template void launch_lt_fill<double>(const AssembleArgs &, const int *, int *, double *, double *, hipStream_t);

@@ -112,6 +112,37 @@ __device__ __forceinline__ void st_relaxed_val(float *p, float v)
 __device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 __device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
 
+// Sum over the G lanes of a row group (G a power of two <= 64, groups aligned
+// inside the wave), valid in the group's LAST lane: a shift-and-add scan over
+// DPP row shifts (1, 2, 4, 8 lanes inside 16-lane rows) and row broadcasts
+// (lane 15 to the next row, lane 31 to the upper half).  The lanes move data
+// through the VALU, not through LDS like a shuffle; the order is fixed, so the
+// result is deterministic.  Every lane of the wave must be active.
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ float dpp_move(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, kRowMask, 0xF, true));
+}
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ double dpp_move(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), kCtrl, kRowMask, 0xF, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), kCtrl, kRowMask, 0xF, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+template <typename T>
+__device__ __forceinline__ T group_sum(T v, int G)
+{
+    if (G >= 2) v += dpp_move<0x111, 0xF>(v);     // row_shr:1
+    if (G >= 4) v += dpp_move<0x112, 0xF>(v);     // row_shr:2
+    if (G >= 8) v += dpp_move<0x114, 0xF>(v);     // row_shr:4
+    if (G >= 16) v += dpp_move<0x118, 0xF>(v);    // row_shr:8
+    if (G >= 32) v += dpp_move<0x142, 0xA>(v);    // row_bcast:15 into rows 1 and 3
+    if (G >= 64) v += dpp_move<0x143, 0xC>(v);    // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
 // Bounded waits: a wave that waits longer than this many wall-clock ticks
 // (100 MHz constant clock) gives up, raises kStatusTimeout and exits.
 constexpr long long kSpinTicks = 2000000000ll;   // 20 s

@@ -211,7 +211,6 @@ void launch_mul64(const int *in, int *out, int n, hipStream_t s);
 // s = t / G at off[c] + s * P * G + i * G + (t % G).  slices[c] =
 // ceil(width[c] / G); size[c] = slices[c] * P * G.
 constexpr int kSweepThreads = 256;
-constexpr int kTailThreads = 512;           // 8 waves: fewer idle waves per narrow level than 16
 __host__ __device__ inline int sweep_rows_pow2(int cnt)
 {
     return cnt <= 1 ? 1 : 1 << (32 - __builtin_clz((unsigned)(cnt - 1)));
@@ -224,47 +223,36 @@ __host__ __device__ inline int sweep_group(int cnt)
 void launch_sweep_layout(int nchunks, const int *cnt, const int *width, int *slices, int *size, hipStream_t s);
 
 // Tail of the level order: the rows at positions [tp0, ns) (the narrow
-// trailing levels) are solved by one kTailThreads workgroup whose LDS holds
-// their values.  The entries of each tail row's source row (a row of L for the
-// forward sweep, of L^T for the backward sweep) are split by column position:
-// below tp0 ("bulk part": final before the tail starts, folded in by a wide
-// kernel) or at/after tp0 ("internal": read from LDS, column stored as
-// position - tp0).  A tail level of cnt <= kTailMaxRows rows is one group
-// with G = tail_group(cnt) lanes per row (P = next power of two >= cnt,
-// lane slot i * G + g of the level's P * G) and slices = ceil(width / G)
-// entries per lane slot, stored lane-major in blocks of kTailBlock: entry t
-// of level row i (slice s = t / G, g = t % G) lives at
-//   off[L] + (s / kTailBlock) * P * G * kTailBlock + (i * G + g) * kTailBlock + s % kTailBlock,
-// so a lane loads a block's entries with a few 16-byte loads.  Unused entries
-// are padding (index ntail, value 0); one more block of padding at off[ntl] is
-// what lanes without a slot load.  The workgroup's LDS holds 0 at value slot
-// ntail, so a padded contribution is -0 * 0 and needs no arithmetic mask.
-constexpr int kTailMaxRows = kTailThreads;
-constexpr int kTailBlock = 8;
-__host__ __device__ inline int tail_group(int cnt)
-{
-    int g = kTailThreads / sweep_rows_pow2(cnt);
-    return g > 64 ? 64 : (g < 1 ? 1 : g);
-}
-// LDS of the tail workgroup: ntail + 1 values (16-byte padded), then one
-// int4 descriptor per tail level and one empty descriptor after them.
+// trailing levels) are cut into blocks of m consecutive positions.  A block's
+// own unit lower triangle is inverted at assembly (dense, m x m), so a sweep
+// solves the block with two launches whatever its number of levels: the
+// entries outside the block are folded into its right-hand side, then the
+// inverse is applied.  Blocks hold at most kTailBlock rows.
+constexpr int kTailBlock = 2048;
+constexpr int kTailTile = 64;               // base block of the inversion; m is a multiple of it
+constexpr int kTailMaxRows = 16 * kTailBlock;
+struct TailBuild {
+    int ntail, tp0, m, nb;                  // rows, first position, rows per block, blocks
+    const int *order;
+};
+// Entries of tail row q outside its block: cnt[q] (forward: rows of L, columns
+// before the block; backward: rows of L^T, columns after it).  The backward
+// count also sets *flag if a column of L has an absolute sum above 1.001 (or
+// not a number): the inverse's entries are bounded by 1 only for
+// such factors (every randomized factor is one; a loaded one need not be).
 template <typename T>
-__host__ __device__ inline int tail_value_bytes(int ntail)
-{
-    return (int)((((long long)ntail + 1) * (long long)sizeof(T) + 15) / 16 * 16);
-}
-void launch_tail_count(int ntail, int tp0, const int *order, EllSrc src, int *cnt_b, int *cnt_i, hipStream_t s);
-template <typename TD>
-void launch_tail_split(int ntail, int tp0, const int *order, EllSrc src, const int *ptr_b, const int *ptr_i,
-                       int *ind_b, TD *val_b, int *ind_i, TD *val_i, hipStream_t s);
-// slices[L] = ceil(max internal row length of level L / G),
-// size[L] = ceil(slices / kTailBlock) * kTailBlock * P * G
-void launch_tail_layout(int ntl, const int *lstart, const int *lcnt, int tp0, const int *ptr_i, int *slices,
-                        int *size, hipStream_t s);
-template <typename TD>
-void launch_tail_fill(int ntl, const int *lstart, const int *lcnt, int tp0, const int *ptr_i, const int *ind_i,
-                      const TD *val_i, const int *off, const int *slices, int pad_ind, int *ell_ind, TD *ell_val,
-                      hipStream_t s);
+void launch_tail_count(const TailBuild &t, bool fwd, EllSrc src, int *cnt, int *flag, hipStream_t s);
+// CSR (absolute positions) of those entries; forward: the block's own entries
+// go to the dense matrices D (nb x m x m, row-major, zeroed by the caller).
+template <typename T>
+void launch_tail_split(const TailBuild &t, bool fwd, EllSrc src, const int *ptr, int *ind, T *val, double *D,
+                       hipStream_t s);
+// D <- inverse of every block's unit lower triangle, in FP64; E: scratch of
+// the same size.
+void launch_tail_invert(const TailBuild &t, double *D, double *E, hipStream_t s);
+// Wf = D in precision T and Wb = its transpose (FP64: Wf may be D and Wb may be E).
+template <typename T>
+void launch_tail_store(const TailBuild &t, const double *D, T *Wf, T *Wb, hipStream_t s);
 template <typename TS, typename TD>
 void launch_sweep_fill(int nchunks, const int *start, const int *cnt, const int *order, EllSrc src, const int *off,
                        const int *slices, int pad_ind, TD pad_val, int *ell_ind, TD *ell_val, hipStream_t s);
@@ -325,18 +313,14 @@ struct SolveArgs {
     // level split: chunks [0, bulk_chunks) belong to the wide levels and run
     // on the persistent grid; levels [tail_level, nlevels) form the tail
     int bulk_chunks, tail_level, nlevels;
-    // tail (see launch_tail_*): rows [tail_pos0, n), ntail_levels levels with
-    // absolute start positions tl_start and row counts tl_cnt; internal ELL of
-    // the forward (tf_*) and backward (tb_*) sweeps; CSR (tp_*) of the
-    // forward bulk part (absolute column positions); tacc = bulk-folded
-    // right-hand side of the tail rows (precision of the factor)
-    int tail_pos0, ntail, ntail_levels, tail_lds_bytes;
-    const int *tl_start, *tl_cnt;
-    const int *tf_off, *tf_slices, *tf_ind;
-    const int *tb_off, *tb_slices, *tb_ind;
-    const void *tf_val, *tb_val;
-    const int *tp_ptr, *tp_ind;
-    const void *tp_val;
+    // tail (see launch_tail_*): rows [tail_pos0, n) in tail_nb blocks of
+    // tail_m rows; CSR of the entries outside a row's block (absolute column
+    // positions, tf_*: rows of L, tb_*: rows of L^T), the blocks' inverses by
+    // rows (tail_wf) and by columns (tail_wb), tacc = right-hand side of the
+    // block being solved (precision of the factor)
+    int tail_pos0, ntail, tail_nb, tail_m;
+    const int *tf_ptr, *tf_ind, *tb_ptr, *tb_ind;
+    const void *tf_val, *tb_val, *tail_wf, *tail_wb;
     void *tacc;
     long long spin_ticks;
     const double *b;
@@ -348,8 +332,9 @@ struct SolveArgs {
     const double *alpha_sys;
 };
 int sweep_occupancy_blocks(int device);
-// Largest dynamic LDS (bytes) the tail workgroup may use on this device.
-int tail_lds_limit(int device);
+// Tail part of the sweeps (nothing when ntail == 0).
+template <typename T> void launch_tail_fwd(const SolveArgs &a, const double *p_cur, int update_rx, hipStream_t s);
+template <typename T> void launch_tail_bwd(const SolveArgs &a, hipStream_t s);
 
 template <typename T> void launch_fill_sentinel(T *v, int n, hipStream_t s);
 template <typename T> void launch_pcg_init(const SolveArgs &a, hipStream_t s);

@@ -11,7 +11,8 @@
 //      block partials of p'Ap; the last block computes alpha;
 //   K2 fwd    r -= alpha Ap and x += alpha p on the row being solved, then the
 //             forward sweep y = L^-1 r: persistent chunks over the wide levels,
-//             then the narrow trailing levels in one LDS-resident workgroup;
+//             then the narrow trailing levels by dense block inverses
+//             (dense_tail.hip);
 //   K3 bwd    z = L^-T (D+ y): the trailing levels first, then the wide ones;
 //   K4 dot    r'z block partials, last block computes beta and the stop test.
 // All vectors live in the level-order position numbering, so a chunk of the
@@ -145,37 +146,6 @@ __device__ __forceinline__ T grouped_row_solve_pref(const int *jp, const T *lp, 
         acc = grouped_row_solve<T>(ind + kBulkPref * stride, val + kBulkPref * stride, nsl - kBulkPref, stride, vec,
                                    acc, spin, sc, nap_max);
     return acc;
-}
-
-// Sum over the G lanes of a row group (G a power of two <= 64, groups aligned
-// inside the wave), valid in the group's LAST lane: a shift-and-add scan over
-// DPP row shifts (1, 2, 4, 8 lanes inside 16-lane rows) and row broadcasts
-// (lane 15 to the next row, lane 31 to the upper half).  The lanes move data
-// through the VALU, not through LDS like a shuffle; the order is fixed, so the
-// result is deterministic.  Every lane of the wave must be active.
-template <int kCtrl, int kRowMask>
-__device__ __forceinline__ float dpp_move(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, kRowMask, 0xF, true));
-}
-template <int kCtrl, int kRowMask>
-__device__ __forceinline__ double dpp_move(double v)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffll), kCtrl, kRowMask, 0xF, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), kCtrl, kRowMask, 0xF, true);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-template <typename T>
-__device__ __forceinline__ T group_sum(T v, int G)
-{
-    if (G >= 2) v += dpp_move<0x111, 0xF>(v);     // row_shr:1
-    if (G >= 4) v += dpp_move<0x112, 0xF>(v);     // row_shr:2
-    if (G >= 8) v += dpp_move<0x114, 0xF>(v);     // row_shr:4
-    if (G >= 16) v += dpp_move<0x118, 0xF>(v);    // row_shr:8
-    if (G >= 32) v += dpp_move<0x142, 0xA>(v);    // row_bcast:15 into rows 1 and 3
-    if (G >= 64) v += dpp_move<0x143, 0xC>(v);    // row_bcast:31 into rows 2 and 3
-    return v;
 }
 
 // Thread range of a grid-stride loop over the ordered SpMV tiles in which
@@ -490,208 +460,6 @@ __global__ void __launch_bounds__(kSweepThreads) k_sweep_bulk(SolveArgs a, const
     }
 }
 
-// ---------------------------------------------------------------- tail
-// The narrow trailing levels (rows [tail_pos0, n)) run in one kTailThreads
-// workgroup whose LDS holds the tail's solution values, so the level-to-level
-// dependency chain goes through LDS and a barrier, not through HBM.
-// Forward: k_tail_prep folds every tail row's entries in the wide levels
-// (final once the bulk sweep has ended) into tacc with one wave per row, and
-// applies the row's r/x update; k_tail_solve then walks the tail levels.
-// Backward: the tail levels come first and depend only on each other.
-template <typename T>
-__global__ void __launch_bounds__(kRedBlock) k_tail_prep(SolveArgs a, const double *p_cur, int update_rx)
-{
-    PcgScalars *sc = a.sc;
-    if (sc->done) return;
-    const double alpha0 = update_rx ? sc->alpha : 0.0;
-    const T *val = (const T *)a.tp_val;
-    const T *y = (const T *)a.y;
-    T *tacc = (T *)a.tacc;
-    const int lane = lane_id();
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-    const int nwaves = gridDim.x * blockDim.x / kWave;
-    for (int q = wave; q < a.ntail; q += nwaves) {
-        T acc = (T)0;
-        for (int e = a.tp_ptr[q] + lane; e < a.tp_ptr[q + 1]; e += kWave) acc = fma_t(-val[e], y[a.tp_ind[e]], acc);
-        acc = group_sum(acc, kWave);
-        if (lane == kWave - 1) {
-            const int k = a.tail_pos0 + q;
-            double rk = a.r[k];
-            if (update_rx) {
-                const double al = a.alpha_sys ? a.alpha_sys[a.sys_of[k]] : alpha0;
-                rk = fma_t(-al, a.ap[k], rk);
-                a.r[k] = rk;
-                a.x[k] = fma_t(al, p_cur[k], a.x[k]);
-            }
-            tacc[q] = (T)rk + acc;
-        }
-    }
-}
-
-// Waits for this wave's LDS operations, then the workgroup barrier; global
-// loads in flight (the next level's indices) are not waited for.
-__device__ __forceinline__ void lds_barrier()
-{
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-
-constexpr int kTailPref = kTailBlock;    // slices per lane loaded before the LDS reads
-
-// The kTailBlock consecutive entries of a lane slot (16-byte aligned: every
-// level's block size is a multiple of kTailBlock entries).
-template <typename T>
-__device__ __forceinline__ void tail_block_load(const int *ind, const T *val, int base, int *j, T *l)
-{
-    static_assert(kTailBlock == 8, "two 16-byte index loads per block");
-    const int4 *pi = reinterpret_cast<const int4 *>(ind + base);
-    const int4 i0 = pi[0], i1 = pi[1];
-    j[0] = i0.x; j[1] = i0.y; j[2] = i0.z; j[3] = i0.w;
-    j[4] = i1.x; j[5] = i1.y; j[6] = i1.z; j[7] = i1.w;
-    if constexpr (sizeof(T) == 4) {
-        const float4 *pv = reinterpret_cast<const float4 *>(val + base);
-        const float4 v0 = pv[0], v1 = pv[1];
-        l[0] = v0.x; l[1] = v0.y; l[2] = v0.z; l[3] = v0.w;
-        l[4] = v1.x; l[5] = v1.y; l[6] = v1.z; l[7] = v1.w;
-    } else {
-        const double2 *pv = reinterpret_cast<const double2 *>(val + base);
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-            const double2 v = pv[h];
-            l[2 * h] = v.x;
-            l[2 * h + 1] = v.y;
-        }
-    }
-}
-
-template <typename T, bool kFwd>
-__global__ void __launch_bounds__(kTailThreads) k_tail_solve(SolveArgs a)
-{
-    extern __shared__ double tail_lds_d[];
-    T *v = reinterpret_cast<T *>(tail_lds_d);
-    PcgScalars *sc = a.sc;
-    if (sc->done) return;
-    const int t = threadIdx.x;
-    const int nt = a.ntail, tp0 = a.tail_pos0;
-    T *y = (T *)a.y;
-    T *z = (T *)a.z;
-    const int *off = kFwd ? a.tf_off : a.tb_off;
-    const int *slices = kFwd ? a.tf_slices : a.tb_slices;
-    const int *ind = kFwd ? a.tf_ind : a.tb_ind;
-    const T *val = (const T *)(kFwd ? a.tf_val : a.tb_val);
-    // initial values: forward = bulk-folded right-hand side; backward = D+ y
-    // (solver.hpp:64-84), with y reset to the sentinel for the next sweep
-    for (int q = t; q < nt; q += kTailThreads) {
-        T init;
-        if (kFwd) {
-            init = ((const T *)a.tacc)[q];
-        } else {
-            const int k = tp0 + q;
-            T yk = y[k];
-            y[k] = sent_value(T());
-            const T dk = ((const T *)a.diag)[k];
-            if (dk != (T)0) yk = yk / dk;
-            init = yk;
-        }
-        v[q] = init;
-    }
-    if (t == 0) v[nt] = (T)0;        // slot of the padding entries
-    // level descriptors {start, cnt, ELL offset, slices} after the values
-    const int ntl = a.ntail_levels;
-    const int ze = off[ntl];          // the padding block after the last level
-    int4 *tm = reinterpret_cast<int4 *>(reinterpret_cast<char *>(tail_lds_d) + tail_value_bytes<T>(nt));
-    for (int L = t; L < ntl; L += kTailThreads) tm[L] = make_int4(a.tl_start[L], a.tl_cnt[L], off[L], slices[L]);
-    // an empty level (no rows, no slices) after the last one: the loop below
-    // solves whole groups of three levels, the ones past the end being empty
-    if (t == 0) tm[ntl] = make_int4(tp0, 0, ze, 0);
-    __syncthreads();
-    // Software pipeline over three register sets (A, B, C): this lane's first
-    // kTailPref index/value slices of level s + 2 are loaded while level s is
-    // solved (two levels of latency cover one global round trip); the loop
-    // is unrolled by three so that no register copy (and no wait) sits
-    // between the loads and their use.  Level descriptors are read from LDS
-    // one fetch ahead (dn), so a fetch starts without an LDS round trip; the
-    // lane term (a.zero is 0) keeps the read a per-lane one, so the compiler
-    // does not make it uniform (and wait for it) at the read but at its use.
-    auto desc = [&](int s) { return tm[(s < ntl ? (kFwd ? s : ntl - 1 - s) : ntl) + (t & (kWave - 1)) * a.zero]; };
-    auto fetch = [&](const int4 &dsrc, int4 &d, int *j, T *l) {
-        d = make_int4(__builtin_amdgcn_readfirstlane(dsrc.x), __builtin_amdgcn_readfirstlane(dsrc.y),
-                      __builtin_amdgcn_readfirstlane(dsrc.z), __builtin_amdgcn_readfirstlane(dsrc.w));
-        const int stride = sweep_rows_pow2(d.y) * tail_group(d.y);
-        // every lane loads (the padding block when it has no slot), so the
-        // loads are never predicated away, and nothing is computed from the
-        // loaded values before their level is solved (a mask applied here
-        // would make the compiler wait for these loads at once); slices past
-        // the level's own are padding in the layout.  A level without
-        // internal entries (d.w = 0, also the empty one past the end) has no
-        // block of its own.
-        tail_block_load<T>(ind, val, (t < stride && d.w > 0) ? d.z + t * kTailBlock : ze, j, l);
-    };
-    auto solve = [&](const int4 &d, const int *j, const T *l) {
-        const int G = tail_group(d.y);
-        const int stride = sweep_rows_pow2(d.y) * G;
-        const int i = t / G, g = t - i * G;
-        const bool lead = t < stride && i < d.y && g == G - 1;
-        const int q = d.x - tp0 + i;
-        T acc = (T)0;
-        // a wave with no slot of this level skips its LDS work (its loads of
-        // the padding block were issued all the same, see fetch)
-        if ((t & ~(kWave - 1)) < stride) {
-            // the row's own value is read with the gathers (it is written only
-            // at the end of the level), not after the sum: one LDS round trip
-            // less on the level's critical path; other lanes read the zero slot
-            const T own = v[lead ? q : nt];
-#pragma unroll
-            for (int u = 0; u < kTailPref; ++u) acc = fma_t(-l[u], v[j[u]], acc);
-            if (t < stride) {
-                // blocks past the prefetched one (long rows); a padded entry
-                // adds -0 * 0 = -0, which leaves acc unchanged
-                for (int sl = kTailPref; sl < d.w; sl += kTailBlock) {
-                    int jj[kTailBlock];
-                    T ll[kTailBlock];
-                    tail_block_load<T>(ind, val, d.z + sl * stride + t * kTailBlock, jj, ll);
-#pragma unroll
-                    for (int u = 0; u < kTailBlock; ++u) acc = fma_t(-ll[u], v[jj[u]], acc);
-                }
-            }
-            if (lead) acc += own;
-            acc = group_sum(acc, G);
-            if (lead) v[q] = acc;
-        }
-        lds_barrier();
-    };
-    int4 dA = make_int4(0, 0, 0, 0), dB = dA, dC = dA;
-    int jA[kTailPref], jB[kTailPref], jC[kTailPref];
-    T lA[kTailPref], lB[kTailPref], lC[kTailPref];
-    int4 dn = dA;
-    if (ntl > 0) {
-        fetch(desc(0), dA, jA, lA);
-        fetch(desc(1), dB, jB, lB);
-        dn = desc(2);
-    }
-    // no exits inside the group: an exit path would carry the newest loads
-    // to the loop header, where the compiler then waits for them every level
-    for (int s = 0; s < ntl; s += 3) {
-        fetch(dn, dC, jC, lC);
-        dn = desc(s + 3);
-        solve(dA, jA, lA);
-        fetch(dn, dA, jA, lA);
-        dn = desc(s + 4);
-        solve(dB, jB, lB);
-        fetch(dn, dB, jB, lB);
-        dn = desc(s + 5);
-        solve(dC, jC, lC);
-    }
-    for (int q = t; q < nt; q += kTailThreads) {
-        const int k = tp0 + q;
-        if (kFwd) {
-            y[k] = unsent(v[q]);
-            z[k] = sent_value(T());
-        } else {
-            z[k] = unsent(v[q]);
-        }
-    }
-}
-
 // ---------------------------------------------------------------- K4
 template <typename T>
 __global__ void __launch_bounds__(kRedBlock) k_dot(SolveArgs a, int init)
@@ -850,19 +618,13 @@ void launch_fwd(const SolveArgs &a, const double *p_cur, int update_rx, hipStrea
     if (a.bulk_chunks > 0)
         hipLaunchKernelGGL((k_sweep_bulk<T, true>), dim3(sweep_blocks(a)), dim3(kSweepThreads), 0, s, a, p_cur,
                            update_rx);
-    if (a.ntail > 0) {
-        int g = (a.ntail + 3) / 4;
-        if (g > 4096) g = 4096;
-        hipLaunchKernelGGL(k_tail_prep<T>, dim3(g), dim3(kRedBlock), 0, s, a, p_cur, update_rx);
-        hipLaunchKernelGGL((k_tail_solve<T, true>), dim3(1), dim3(kTailThreads), a.tail_lds_bytes, s, a);
-    }
+    launch_tail_fwd<T>(a, p_cur, update_rx, s);
 }
 
 template <typename T>
 void launch_bwd(const SolveArgs &a, hipStream_t s)
 {
-    if (a.ntail > 0)
-        hipLaunchKernelGGL((k_tail_solve<T, false>), dim3(1), dim3(kTailThreads), a.tail_lds_bytes, s, a);
+    launch_tail_bwd<T>(a, s);
     if (a.bulk_chunks > 0)
         hipLaunchKernelGGL((k_sweep_bulk<T, false>), dim3(sweep_blocks(a)), dim3(kSweepThreads), 0, s, a,
                            (const double *)nullptr, 0);
@@ -1100,20 +862,6 @@ template <typename T>
 void launch_trsv_bwd_only(const SolveArgs &a, hipStream_t s)
 {
     launch_bwd<T>(a, s);
-}
-
-int tail_lds_limit(int device)
-{
-    int lim = 0;
-    if (hipDeviceGetAttribute(&lim, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess || lim <= 0)
-        lim = 64 * 1024;
-    if (lim > 160 * 1024) lim = 160 * 1024;
-    (void)hipFuncSetAttribute((const void *)k_tail_solve<float, true>, hipFuncAttributeMaxDynamicSharedMemorySize, lim);
-    (void)hipFuncSetAttribute((const void *)k_tail_solve<float, false>, hipFuncAttributeMaxDynamicSharedMemorySize, lim);
-    (void)hipFuncSetAttribute((const void *)k_tail_solve<double, true>, hipFuncAttributeMaxDynamicSharedMemorySize, lim);
-    (void)hipFuncSetAttribute((const void *)k_tail_solve<double, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              lim);
-    return lim;
 }
 
 int sweep_occupancy_blocks(int device)

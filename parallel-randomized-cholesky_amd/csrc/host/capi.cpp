@@ -112,7 +112,7 @@ static int rc_create_impl(rc_handle_t *out, const rc_options *opt)
         if (lo) h->level_order_set = true;
         const char *nm = std::getenv("RCHOL_NAP_MAX");          // polling back-off cap (1..64)
         if (nm) h->nap_max = std::max(1, std::min(64, std::atoi(nm)));
-        const char *tr = std::getenv("RCHOL_TAIL_ROWS");        // tail level width limit (1..kTailMaxRows + 1)
+        const char *tr = std::getenv("RCHOL_TAIL_ROWS");        // tail level width limit (1: no tail)
         if (tr) h->tail_max_rows = std::max(1, std::min(kTailMaxRows + 1, std::atoi(tr)));
         const char *sc = std::getenv("RCHOL_LIST_SEG_CAP");     // ready-list segment capacity limit (>= 1)
         if (sc) h->seg_cap_limit = std::max(1, std::atoi(sc));
@@ -850,8 +850,43 @@ static int bit_width(int64_t v)
     return b;
 }
 
+// First level of the tail (see dense_tail.hip).  With a width limit, the
+// trailing run of narrower levels; limit < 0: the split with the least
+// estimated sweep time.  A level of the dataflow sweep costs one store ->
+// poll round trip through device-scope memory (2.2 us, measured), a tail block
+// two launches and their memory round trips (about 9 us, its share of the
+// inversion included) and the bytes of its triangle (3 TB/s).  Returns the widest tail
+// level + 1 in *width.
+static int tail_start(int limit, const std::vector<int> &hl, int nl, int vbytes, int *width)
+{
+    constexpr double kLevelUs = 2.2, kBulkUs = 6.0, kBlockUs = 9.0, kBytesPerUs = 3.0e6;
+    const int ns = nl > 0 ? hl[(size_t)nl] : 0;
+    int best = nl, widest = 0;
+    double best_us = nl * kLevelUs + (nl > 0 ? kBulkUs : 0.0);
+    for (int tl = nl - 1; tl >= 0; --tl) {
+        const int rows = ns - hl[(size_t)tl];
+        const int w = hl[(size_t)tl + 1] - hl[(size_t)tl];
+        if (rows > kTailMaxRows) break;
+        if (limit >= 0) {
+            if (w >= limit) break;
+            best = tl;
+            continue;
+        }
+        const int nb = (rows + kTailBlock - 1) / kTailBlock;
+        const double us = tl * kLevelUs + (tl > 0 ? kBulkUs : 0.0) + nb * kBlockUs +
+                          0.5 * rows * ((double)rows / nb) * vbytes / kBytesPerUs;
+        if (us < best_us) {
+            best_us = us;
+            best = tl;
+        }
+    }
+    for (int tl = best; tl < nl; ++tl) widest = std::max(widest, hl[(size_t)tl + 1] - hl[(size_t)tl]);
+    *width = best < nl ? widest + 1 : 0;
+    return best;
+}
+
 template <typename T>
-static int assemble(rc_handle_t h, double *ms_out)
+static int assemble(rc_handle_t h, double *ms_out, bool tail = true)
 {
     h->multi_ready = false;
     hipStream_t s = h->stream;
@@ -1019,8 +1054,7 @@ static int assemble(rc_handle_t h, double *ms_out)
     RC_HIP(h->chunk_cnt.ensure((size_t)std::max(nchunks, 1) * sizeof(int)));
     launch_chunk_fill(nchunks, nseg, lptr, cptr, h->lvl_w.as<int>(), h->sweep_gmin, h->chunk_start.as<int>(),
                       h->chunk_cnt.as<int>(), s);
-    // level split: the trailing run of levels with fewer than tail_max_rows
-    // rows, as long as their rows fit the tail workgroup's LDS, is the tail
+    // level split: the trailing levels [tail_level, nl) form the tail
     std::vector<int> hl(nlsz), hc(nlsz);
     {
         std::vector<int> hs(nssz), hcs(nssz);
@@ -1031,23 +1065,13 @@ static int assemble(rc_handle_t h, double *ms_out)
             hl[L] = hs[L * (size_t)per_level];
             hc[L] = hcs[L * (size_t)per_level];
         }
-        if (h->tail_lds_cap < 0) h->tail_lds_cap = tail_lds_limit(h->opt.device);
-        int tl = nl;
-        int64_t rows = 0;
-        while (tl > 0) {
-            const int c = hl[(size_t)tl] - hl[(size_t)tl - 1];
-            // values + one descriptor per tail level + the empty descriptor
-            const int64_t bytes = ((rows + c + 1) * (int64_t)sizeof(T) + 15) / 16 * 16 + 16 * (int64_t)(nl - tl + 2);
-            if (c >= h->tail_max_rows || bytes > (int64_t)h->tail_lds_cap) break;
-            rows += c;
-            --tl;
-        }
-        h->tail_level = tl;
-        h->bulk_chunks = nl > 0 ? hc[(size_t)tl] : 0;
+        h->tail_level = tail ? tail_start(h->tail_max_rows, hl, nl, (int)sizeof(T), &h->tail_width) : nl;
+        h->bulk_chunks = nl > 0 ? hc[(size_t)h->tail_level] : 0;
     }
+    const int nbulk = h->bulk_chunks;             // chunks of the tail levels have no sweep layout
 
     // 4. sliced ELL of L (forward) and L^T (backward) over the chunks
-    const size_t csz = (size_t)nchunks + 1;
+    const size_t csz = (size_t)nbulk + 1;
     RC_HIP(h->lf_width.ensure(csz * sizeof(int)));
     RC_HIP(h->lf_off.ensure(csz * sizeof(int)));
     RC_HIP(h->lb_width.ensure(csz * sizeof(int)));
@@ -1063,12 +1087,12 @@ static int assemble(rc_handle_t h, double *ms_out)
     };
     // grouped layout: width -> slice count in place, slice block sizes -> offsets
     auto sweep_offsets = [&](const int *ptr, int *slices, int *off, int64_t &total) -> int {
-        launch_ell_width(nchunks, h->chunk_start.as<int>(), h->chunk_cnt.as<int>(), h->order.as<int>(), ns, ptr,
+        launch_ell_width(nbulk, h->chunk_start.as<int>(), h->chunk_cnt.as<int>(), h->order.as<int>(), ns, ptr,
                          slices, s);
-        launch_sweep_layout(nchunks, h->chunk_cnt.as<int>(), slices, slices, h->tmp_a.as<int>(), s);
-        scan_exclusive(h->tmp_a.as<int>(), off, nchunks, h->tmp_scan.as<int>(), s);
+        launch_sweep_layout(nbulk, h->chunk_cnt.as<int>(), slices, slices, h->tmp_a.as<int>(), s);
+        scan_exclusive(h->tmp_a.as<int>(), off, nbulk, h->tmp_scan.as<int>(), s);
         int t = 0;
-        RC_HIP(hipMemcpyAsync(&t, off + nchunks, sizeof(int), hipMemcpyDeviceToHost, s));
+        RC_HIP(hipMemcpyAsync(&t, off + nbulk, sizeof(int), hipMemcpyDeviceToHost, s));
         RC_HIP(hipStreamSynchronize(s));
         total = t;
         return RC_OK;
@@ -1092,100 +1116,76 @@ static int assemble(rc_handle_t h, double *ms_out)
         RC_HIP(hipStreamSynchronize(s));
     }
     EllSrc fs{h->l_ptr.as<int>(), nullptr, h->lt_val.p, h->vals0.as<int>(), h->rowk.as<int>(), nullptr};
-    launch_sweep_fill<T, T>(nchunks, h->chunk_start.as<int>(), h->chunk_cnt.as<int>(), h->order.as<int>(), fs,
+    launch_sweep_fill<T, T>(nbulk, h->chunk_start.as<int>(), h->chunk_cnt.as<int>(), h->order.as<int>(), fs,
                             h->lf_off.as<int>(), h->lf_width.as<int>(), ns, (T)0, h->lf_ind.as<int>(), h->lf_val.as<T>(),
                             s);
     EllSrc bs{h->lt_ptr.as<int>(), h->lt_ind.as<int>(), h->lt_val.p, nullptr, nullptr, h->pos_of.as<int>()};
-    launch_sweep_fill<T, T>(nchunks, h->chunk_start.as<int>(), h->chunk_cnt.as<int>(), h->order.as<int>(), bs,
+    launch_sweep_fill<T, T>(nbulk, h->chunk_start.as<int>(), h->chunk_cnt.as<int>(), h->order.as<int>(), bs,
                             h->lb_off.as<int>(), h->lb_width.as<int>(), ns, (T)0, h->lb_ind.as<int>(), h->lb_val.as<T>(),
                             s);
     RC_HIP(h->diagP.ensure((size_t)std::max(ns, 1) * sizeof(T)));
     launch_gather_t<T>(h->diagT.as<T>(), h->order.as<int>(), h->diagP.as<T>(), ns, s);
-    RC_HIP(h->cm_f.ensure((size_t)std::max(nchunks, 1) * sizeof(int4)));
-    RC_HIP(h->cm_b.ensure((size_t)std::max(nchunks, 1) * sizeof(int4)));
-    launch_pack_meta(nchunks, h->chunk_start.as<int>(), h->chunk_cnt.as<int>(), h->lf_off.as<int>(),
+    RC_HIP(h->cm_f.ensure((size_t)std::max(nbulk, 1) * sizeof(int4)));
+    RC_HIP(h->cm_b.ensure((size_t)std::max(nbulk, 1) * sizeof(int4)));
+    launch_pack_meta(nbulk, h->chunk_start.as<int>(), h->chunk_cnt.as<int>(), h->lf_off.as<int>(),
                      h->lf_width.as<int>(), h->cm_f.as<int4>(), s);
-    launch_pack_meta(nchunks, h->chunk_start.as<int>(), h->chunk_cnt.as<int>(), h->lb_off.as<int>(),
+    launch_pack_meta(nbulk, h->chunk_start.as<int>(), h->chunk_cnt.as<int>(), h->lb_off.as<int>(),
                      h->lb_width.as<int>(), h->cm_b.as<int4>(), s);
 
-    // 4b. the tail: level table, forward bulk-part CSR, internal ELL per direction
-    h->ntail_levels = nl - h->tail_level;
+    // 4b. the tail: entries outside the rows' blocks, inverses of the blocks
     h->tail_pos0 = nl > 0 ? hl[(size_t)h->tail_level] : ns;
     h->ntail = ns - h->tail_pos0;
-    h->tail_lds_bytes = tail_value_bytes<T>(h->ntail) + 16 * (h->ntail_levels + 1);
+    h->tail_nb = (h->ntail + kTailBlock - 1) / kTailBlock;
     if (h->ntail > 0) {
-        const int ntl = h->ntail_levels, tp0 = h->tail_pos0, nt = h->ntail;
-        std::vector<int> ls((size_t)ntl), lc((size_t)ntl);
-        for (int L = 0; L < ntl; ++L) {
-            ls[(size_t)L] = hl[(size_t)(h->tail_level + L)];
-            lc[(size_t)L] = hl[(size_t)(h->tail_level + L + 1)] - ls[(size_t)L];
+        TailBuild tb;
+        tb.ntail = h->ntail;
+        tb.tp0 = h->tail_pos0;
+        tb.nb = h->tail_nb;
+        // blocks of equal size, a multiple of the inversion's tile
+        tb.m = ((h->ntail + tb.nb - 1) / tb.nb + kTailTile - 1) / kTailTile * kTailTile;
+        tb.order = h->order.as<int>();
+        h->tail_m = tb.m;
+        const size_t nt = (size_t)tb.ntail, dense = (size_t)tb.nb * (size_t)tb.m * (size_t)tb.m;
+        RC_HIP(h->tacc.ensure((size_t)tb.m * sizeof(T)));
+        RC_HIP(h->tf_ptr.ensure((nt + 1) * sizeof(int)));
+        RC_HIP(h->tb_ptr.ensure((nt + 1) * sizeof(int)));
+        RC_HIP(h->tail_d.ensure(dense * sizeof(double)));
+        RC_HIP(h->tail_e.ensure(dense * sizeof(double)));
+        int *cnt_f = h->tmp_a.as<int>(), *cnt_b = cnt_f + nt + 1, *flag = cnt_b + nt + 1;
+        RC_HIP(hipMemsetAsync(flag, 0, sizeof(int), s));
+        launch_tail_count<T>(tb, true, fs, cnt_f, flag, s);
+        launch_tail_count<T>(tb, false, bs, cnt_b, flag, s);
+        scan_exclusive(cnt_f, h->tf_ptr.as<int>(), tb.ntail, h->tmp_scan.as<int>(), s);
+        scan_exclusive(cnt_b, h->tb_ptr.as<int>(), tb.ntail, h->tmp_scan.as<int>(), s);
+        int tot[3] = {0, 0, 0};
+        RC_HIP(hipMemcpyAsync(&tot[0], h->tf_ptr.as<int>() + nt, sizeof(int), hipMemcpyDeviceToHost, s));
+        RC_HIP(hipMemcpyAsync(&tot[1], h->tb_ptr.as<int>() + nt, sizeof(int), hipMemcpyDeviceToHost, s));
+        RC_HIP(hipMemcpyAsync(&tot[2], flag, sizeof(int), hipMemcpyDeviceToHost, s));
+        RC_HIP(hipMemsetAsync(h->tail_d.p, 0, dense * sizeof(double), s));
+        RC_HIP(hipStreamSynchronize(s));
+        if (tot[2] != 0) {
+            // a loaded factor whose columns are not bounded: every level is
+            // solved by substitution
+            (void)hipEventDestroy(e0);
+            (void)hipEventDestroy(e1);
+            return assemble<T>(h, ms_out, false);
         }
-        RC_HIP(h->tl_start.ensure((size_t)ntl * sizeof(int)));
-        RC_HIP(h->tl_cnt.ensure((size_t)ntl * sizeof(int)));
-        RC_HIP(hipMemcpyAsync(h->tl_start.p, ls.data(), (size_t)ntl * sizeof(int), hipMemcpyHostToDevice, s));
-        RC_HIP(hipMemcpyAsync(h->tl_cnt.p, lc.data(), (size_t)ntl * sizeof(int), hipMemcpyHostToDevice, s));
-        RC_HIP(h->tacc.ensure((size_t)nt * sizeof(T)));
-        RC_HIP(h->ti_ptr.ensure(((size_t)nt + 1) * sizeof(int)));
-        int *cnt_b = h->tmp_a.as<int>(), *cnt_i = cnt_b + nt + 1;
-        auto build = [&](const EllSrc &src, bool fwd, DevVec &off, DevVec &slices, DevVec &ind, DevVec &val) -> int {
-            launch_tail_count(nt, tp0, h->order.as<int>(), src, cnt_b, cnt_i, s);
-            if (fwd) RC_HIP(h->tp_ptr.ensure(((size_t)nt + 1) * sizeof(int)));
-            int nb = 0, ni = 0;
-            if (fwd) {
-                scan_exclusive(cnt_b, h->tp_ptr.as<int>(), nt, h->tmp_scan.as<int>(), s);
-                RC_HIP(hipMemcpyAsync(&nb, h->tp_ptr.as<int>() + nt, sizeof(int), hipMemcpyDeviceToHost, s));
-            }
-            scan_exclusive(cnt_i, h->ti_ptr.as<int>(), nt, h->tmp_scan.as<int>(), s);
-            RC_HIP(hipMemcpyAsync(&ni, h->ti_ptr.as<int>() + nt, sizeof(int), hipMemcpyDeviceToHost, s));
-            RC_HIP(hipStreamSynchronize(s));
-            if (!fwd) {
-                // a backward dependency always lies in a deeper level, so the
-                // backward tail has no bulk part
-                int64_t tot = 0;
-                std::vector<int> hb((size_t)nt);
-                RC_HIP(hipMemcpy(hb.data(), cnt_b, (size_t)nt * sizeof(int), hipMemcpyDeviceToHost));
-                for (int v : hb) tot += v;
-                if (tot != 0) return fail(h, RC_ERR_STATE, "backward tail row depends on a wider level");
-            }
-            if (fwd) {
-                RC_HIP(h->tp_ind.ensure((size_t)std::max(nb, 1) * sizeof(int)));
-                RC_HIP(h->tp_val.ensure((size_t)std::max(nb, 1) * sizeof(T)));
-            }
-            RC_HIP(h->ti_ind.ensure((size_t)std::max(ni, 1) * sizeof(int)));
-            RC_HIP(h->ti_val.ensure((size_t)std::max(ni, 1) * sizeof(T)));
-            launch_tail_split<T>(nt, tp0, h->order.as<int>(), src, fwd ? h->tp_ptr.as<int>() : cnt_b,
-                                 h->ti_ptr.as<int>(), fwd ? h->tp_ind.as<int>() : nullptr,
-                                 fwd ? h->tp_val.as<T>() : nullptr, h->ti_ind.as<int>(), h->ti_val.as<T>(), s);
-            RC_HIP(slices.ensure((size_t)ntl * sizeof(int)));
-            RC_HIP(off.ensure(((size_t)ntl + 1) * sizeof(int)));
-            int *size = cnt_b;        // reuse: ntl <= nt
-            launch_tail_layout(ntl, h->tl_start.as<int>(), h->tl_cnt.as<int>(), tp0, h->ti_ptr.as<int>(),
-                               slices.as<int>(), size, s);
-            scan_exclusive(size, off.as<int>(), ntl, h->tmp_scan.as<int>(), s);
-            int total = 0;
-            RC_HIP(hipMemcpyAsync(&total, off.as<int>() + ntl, sizeof(int), hipMemcpyDeviceToHost, s));
-            RC_HIP(hipStreamSynchronize(s));
-            // one more block after the levels: the padding lanes without a slot load
-            RC_HIP(ind.ensure(((size_t)total + kTailBlock) * sizeof(int)));
-            RC_HIP(val.ensure(((size_t)total + kTailBlock) * sizeof(T)));
-            launch_tail_fill<T>(ntl, h->tl_start.as<int>(), h->tl_cnt.as<int>(), tp0, h->ti_ptr.as<int>(),
-                                h->ti_ind.as<int>(), h->ti_val.as<T>(), off.as<int>(), slices.as<int>(), nt,
-                                ind.as<int>(), val.as<T>(), s);
-            int pad_ind[kTailBlock];
-            T pad_val[kTailBlock];
-            for (int u = 0; u < kTailBlock; ++u) {
-                pad_ind[u] = nt;
-                pad_val[u] = (T)0;
-            }
-            RC_HIP(hipMemcpyAsync(ind.as<int>() + total, pad_ind, sizeof(pad_ind), hipMemcpyHostToDevice, s));
-            RC_HIP(hipMemcpyAsync(val.as<T>() + total, pad_val, sizeof(pad_val), hipMemcpyHostToDevice, s));
-            RC_HIP(hipStreamSynchronize(s));
-            return RC_OK;
-        };
-        rc = build(fs, true, h->tf_off, h->tf_slices, h->tf_ind, h->tf_val);
-        if (rc != RC_OK) return rc;
-        rc = build(bs, false, h->tb_off, h->tb_slices, h->tb_ind, h->tb_val);
-        if (rc != RC_OK) return rc;
+        RC_HIP(h->tf_ind.ensure((size_t)std::max(tot[0], 1) * sizeof(int)));
+        RC_HIP(h->tf_val.ensure((size_t)std::max(tot[0], 1) * sizeof(T)));
+        RC_HIP(h->tb_ind.ensure((size_t)std::max(tot[1], 1) * sizeof(int)));
+        RC_HIP(h->tb_val.ensure((size_t)std::max(tot[1], 1) * sizeof(T)));
+        launch_tail_split<T>(tb, true, fs, h->tf_ptr.as<int>(), h->tf_ind.as<int>(), h->tf_val.as<T>(),
+                             h->tail_d.as<double>(), s);
+        launch_tail_split<T>(tb, false, bs, h->tb_ptr.as<int>(), h->tb_ind.as<int>(), h->tb_val.as<T>(),
+                             h->tail_d.as<double>(), s);
+        launch_tail_invert(tb, h->tail_d.as<double>(), h->tail_e.as<double>(), s);
+        if constexpr (sizeof(T) == 4) {
+            RC_HIP(h->tail_wf.ensure(dense * sizeof(T)));
+            RC_HIP(h->tail_wb.ensure(dense * sizeof(T)));
+            launch_tail_store<T>(tb, h->tail_d.as<double>(), h->tail_wf.as<T>(), h->tail_wb.as<T>(), s);
+        } else {
+            launch_tail_store<T>(tb, h->tail_d.as<double>(), nullptr, h->tail_e.as<T>(), s);
+        }
     }
 
     // 5. A in position numbering, sliced ELL over 64-position tiles
@@ -1639,21 +1639,16 @@ SolveArgs solve_args(rc_handle_t h)
     a.tail_level = h->tail_level;
     a.tail_pos0 = h->tail_pos0;
     a.ntail = h->ntail;
-    a.ntail_levels = h->ntail_levels;
-    a.tail_lds_bytes = h->tail_lds_bytes;
-    a.tl_start = h->tl_start.as<int>();
-    a.tl_cnt = h->tl_cnt.as<int>();
-    a.tf_off = h->tf_off.as<int>();
-    a.tf_slices = h->tf_slices.as<int>();
+    a.tail_nb = h->tail_nb;
+    a.tail_m = h->tail_m;
+    a.tf_ptr = h->tf_ptr.as<int>();
     a.tf_ind = h->tf_ind.as<int>();
     a.tf_val = h->tf_val.p;
-    a.tb_off = h->tb_off.as<int>();
-    a.tb_slices = h->tb_slices.as<int>();
+    a.tb_ptr = h->tb_ptr.as<int>();
     a.tb_ind = h->tb_ind.as<int>();
     a.tb_val = h->tb_val.p;
-    a.tp_ptr = h->tp_ptr.as<int>();
-    a.tp_ind = h->tp_ind.as<int>();
-    a.tp_val = h->tp_val.p;
+    a.tail_wf = h->prec == 32 ? h->tail_wf.p : h->tail_d.p;
+    a.tail_wb = h->prec == 32 ? h->tail_wb.p : h->tail_e.p;
     a.tacc = h->tacc.p;
     a.nlevels = h->nlevels;
     a.spin_ticks = h->spin_ticks;
@@ -2614,7 +2609,7 @@ static int rc_autotune_impl(rc_handle_t h, int reps, rc_tune_stats *st)
     if (!h->factored || !h->rhs_set) return fail(h, RC_ERR_STATE, "factor and rc_set_rhs must precede rc_autotune");
     if (reps <= 0) reps = 5;
     RC_HIP(hipSetDevice(h->opt.device));
-    const int tails[] = {0, 64, 128, 256, kTailMaxRows + 1};
+    const int tails[] = {-1, 0, 64, 256, 1024};        // -1: the rule (tail_start)
     const int grids[] = {h->sweep_blocks_max, h->sweep_blocks_max / 2, h->sweep_blocks_max / 4};
     auto reassemble = [&](int tail) -> int {
         h->tail_max_rows = tail;
@@ -2654,7 +2649,7 @@ static int rc_autotune_impl(rc_handle_t h, int reps, rc_tune_stats *st)
     if (rc != RC_OK) return rc;
     h->fstats.nlevels = h->nlevels;
     if (st) {
-        st->tail_max_rows = best_tail;
+        st->tail_max_rows = h->tail_width;
         st->sweep_blocks = best_grid;
         st->configs_tried = tried;
         st->sweeps_ms_before = base;

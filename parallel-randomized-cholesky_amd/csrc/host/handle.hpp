@@ -126,13 +126,13 @@ struct rc_handle_s {
     bool level_order_set = false;   // RCHOL_LEVEL_ORDER given
     int level_order = 1;            // 0 length, 1 spatial (default), 2 spatial within length buckets,
                                     // 3 spatial within sweep-group classes
-    // tail of the level order (LDS-resident solve)
-    int tail_max_rows = 256, tail_lds_cap = -1;
+    // tail of the level order (dense block inverses)
+    int tail_max_rows = -1;         // width limit of its levels; -1: chosen by estimated time, 0: no tail
+    int tail_width = 0;             // widest tail level of the current factor + 1 (0: no tail)
     int nap_max = 1;                // measured best: poll again after one s_sleep 2
     int seg_cap_limit = 0;          // > 0: ready-list segments hold at most this many entries (exercises the overflow region)
-    int tail_pos0 = 0, ntail = 0, ntail_levels = 0, tail_lds_bytes = 0;
-    DevVec tl_start, tl_cnt, tp_ptr, tp_ind, tp_val, tf_off, tf_slices, tf_ind, tf_val, tb_off, tb_slices, tb_ind,
-        tb_val, ti_ptr, ti_ind, ti_val, tacc;
+    int tail_pos0 = 0, ntail = 0, tail_nb = 0, tail_m = 0;
+    DevVec tf_ptr, tf_ind, tf_val, tb_ptr, tb_ind, tb_val, tacc, tail_d, tail_e, tail_wf, tail_wb;
     rc_factor_stats fstats{};
 
     // PCG
