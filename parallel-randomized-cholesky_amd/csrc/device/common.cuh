@@ -44,6 +44,13 @@ __device__ __forceinline__ void fence_release() { __builtin_amdgcn_fence(__ATOMI
 __device__ __forceinline__ void fence_acquire() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
 __device__ __forceinline__ void fence_acq_rel() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "agent"); }
 
+// Waits until this wave's stores are complete.  Agent-scope (`sc1`) stores are
+// written through to the point where every XCD sees them, so values that are
+// only ever written and read with agent-scope accesses need no release fence
+// (an L2 write-back, several us when every workgroup of a launch issues one)
+// before an arrival counter is raised: this wait orders them.
+__device__ __forceinline__ void drain_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // ---------------------------------------------------------------- wave ops
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
 

@@ -394,8 +394,17 @@ struct MultiArgs {
     const int *row_ord;           // position of every input-numbered row (the SpMV's visiting order)
     const int *l_ptr, *l_ind, *lt_ptr, *lt_ind;
     const void *l_val, *lt_val, *diag;
+    // chunks of the levels before the tail, {first row, rows, first entry,
+    // entries} per sweep (launch_mchunk_fill)
     int nchunks;
-    const int *chunk_start, *chunk_cnt;
+    const int4 *cm_f, *cm_b;
+    // tail: as in SolveArgs; tacc: tail_m x K; tail_part: kMTailParts partial
+    // results of a block; tail_arrive: arrivals per row tile (zero between launches)
+    int tail_pos0, ntail, tail_nb, tail_m;
+    const int *tf_ptr, *tf_ind, *tb_ptr, *tb_ind;
+    const void *tf_val, *tb_val, *tail_wf, *tail_wb;
+    void *tacc, *tail_part;
+    unsigned int *tail_arrive;
     double *x, *r, *ap, *p0, *p1;
     void *y, *z;
     const double *b;
@@ -405,6 +414,23 @@ struct MultiArgs {
     int reduce_blocks, sweep_blocks;
     long long spin_ticks;
 };
+
+// Geometry of the sweeps: 256-thread workgroups; a chunk's first 512 entries
+// pass through LDS; V right-hand sides per lane.
+constexpr int kMSweepThreads = 256, kMSweepBits = 8;
+constexpr int kMChunkEntries = 512;
+constexpr int kMTailCols = 512;             // columns of a block's triangle per workgroup
+constexpr int kMTailParts = kTailBlock / kMTailCols;
+inline int multi_lane_rhs(int K, int vbytes)
+{
+    const int v = 16 / vbytes;
+    return K >= v ? v : K;
+}
+// Chunks of nseg level segments [seg_ptr[g], seg_ptr[g + 1]) whose widest rows
+// have width[g] entries; L = K / V lanes hold a row's right-hand sides.
+void launch_mchunk_count(int nseg, const int *seg_ptr, const int *width, int L, int *cnt, hipStream_t s);
+void launch_mchunk_fill(int nchunks, int nseg, const int *seg_ptr, const int *chunk_ptr, const int *width, int L,
+                        const int *l_ptr, const int *lt_ptr, int4 *cm_f, int4 *cm_b, hipStream_t s);
 
 template <typename T> void launch_multi_init(const MultiArgs &a, hipStream_t s);
 template <typename T> void launch_multi_iteration(const MultiArgs &a, int parity, hipStream_t s);

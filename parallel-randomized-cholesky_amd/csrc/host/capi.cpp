@@ -889,6 +889,7 @@ template <typename T>
 static int assemble(rc_handle_t h, double *ms_out, bool tail = true)
 {
     h->multi_ready = false;
+    h->m_chunk_K = 0;
     hipStream_t s = h->stream;
     hipEvent_t e0, e1;
     RC_HIP(hipEventCreate(&e0));
@@ -1067,6 +1068,7 @@ static int assemble(rc_handle_t h, double *ms_out, bool tail = true)
         }
         h->tail_level = tail ? tail_start(h->tail_max_rows, hl, nl, (int)sizeof(T), &h->tail_width) : nl;
         h->bulk_chunks = nl > 0 ? hc[(size_t)h->tail_level] : 0;
+        h->bulk_segs = h->tail_level * per_level;
     }
     const int nbulk = h->bulk_chunks;             // chunks of the tail levels have no sweep layout
 
@@ -1861,8 +1863,9 @@ static int build_multi(rc_handle_t h)
         int nnz = 0;
         RC_HIP(hipMemcpyAsync(&nnz, ptr.as<int>() + ns, sizeof(int), hipMemcpyDeviceToHost, s));
         RC_HIP(hipStreamSynchronize(s));
-        RC_HIP(ind.ensure((size_t)std::max(nnz, 1) * sizeof(int)));
-        RC_HIP(val.ensure((size_t)std::max(nnz, 1) * vbytes));
+        // one more entry: a chunk of empty rows at the end loads (and ignores) it
+        RC_HIP(ind.ensure(((size_t)nnz + 1) * sizeof(int)));
+        RC_HIP(val.ensure(((size_t)nnz + 1) * vbytes));
         return RC_OK;
     };
     EllSrc as{h->a_ptr.as<int>(), h->a_ind.as<int>(), h->a_val.p, nullptr, nullptr, h->pos_of.as<int>()};
@@ -1888,6 +1891,7 @@ static int build_multi(rc_handle_t h)
 
 extern "C" {
 
+// (build_multi must have run for this factor)
 static int multi_args(rc_handle_t h, int k, MultiArgs &a)
 {
     int K = 1;
@@ -1907,6 +1911,32 @@ static int multi_args(rc_handle_t h, int k, MultiArgs &a)
     RC_HIP(h->m_part.ensure((size_t)h->reduce_blocks * 2 * K * sizeof(double)));
     RC_HIP(h->ctrs.ensure(kClaimWords * sizeof(unsigned int)));
     RC_HIP(h->pos_of_user.ensure((n + 1) * sizeof(int)));
+    {
+        const size_t tm = h->ntail > 0 ? (size_t)h->tail_m : 1;
+        RC_HIP(h->m_tacc.ensure(tm * (size_t)K * sz));
+        RC_HIP(h->m_tpart.ensure((size_t)kMTailParts * tm * (size_t)K * sz));
+        if (!h->m_tarr.p) {
+            RC_HIP(h->m_tarr.ensure(kTailBlock / 16 * sizeof(unsigned int)));
+            RC_HIP(hipMemsetAsync(h->m_tarr.p, 0, kTailBlock / 16 * sizeof(unsigned int), h->stream));
+        }
+    }
+    if (h->m_chunk_K != K) {              // chunks of the wide levels for this many right-hand sides
+        const int L = K / multi_lane_rhs(K, (int)sz), ng = h->bulk_segs;
+        const int *seg = h->seg_work.as<int>();
+        RC_HIP(h->m_ccnt.ensure(((size_t)ng + 1) * sizeof(int)));
+        RC_HIP(h->m_cptr.ensure(((size_t)ng + 1) * sizeof(int)));
+        launch_mchunk_count(ng, seg, h->lvl_w.as<int>(), L, h->m_ccnt.as<int>(), h->stream);
+        scan_exclusive(h->m_ccnt.as<int>(), h->m_cptr.as<int>(), ng, h->tmp_scan.as<int>(), h->stream);
+        int nc = 0;
+        RC_HIP(hipMemcpyAsync(&nc, h->m_cptr.as<int>() + ng, sizeof(int), hipMemcpyDeviceToHost, h->stream));
+        RC_HIP(hipStreamSynchronize(h->stream));
+        RC_HIP(h->m_cmf.ensure((size_t)std::max(nc, 1) * sizeof(int4)));
+        RC_HIP(h->m_cmb.ensure((size_t)std::max(nc, 1) * sizeof(int4)));
+        launch_mchunk_fill(nc, ng, seg, h->m_cptr.as<int>(), h->lvl_w.as<int>(), L, h->m_lptr.as<int>(),
+                           h->m_ltptr.as<int>(), h->m_cmf.as<int4>(), h->m_cmb.as<int4>(), h->stream);
+        h->m_nchunks = nc;
+        h->m_chunk_K = K;
+    }
     launch_inverse_perm((int)n, h->idx_user.as<int>(), h->pos_of_user.as<int>(), h->stream);
     a.n = (int)n;
     a.K = K;
@@ -1922,9 +1952,24 @@ static int multi_args(rc_handle_t h, int k, MultiArgs &a)
     a.l_val = h->m_lval.p;
     a.lt_val = h->m_ltval.p;
     a.diag = h->diagP.p;
-    a.nchunks = h->nchunks;
-    a.chunk_start = h->chunk_start.as<int>();
-    a.chunk_cnt = h->chunk_cnt.as<int>();
+    a.nchunks = h->m_nchunks;
+    a.cm_f = h->m_cmf.as<int4>();
+    a.cm_b = h->m_cmb.as<int4>();
+    a.tail_pos0 = h->tail_pos0;
+    a.ntail = h->ntail;
+    a.tail_nb = h->tail_nb;
+    a.tail_m = h->tail_m;
+    a.tf_ptr = h->tf_ptr.as<int>();
+    a.tf_ind = h->tf_ind.as<int>();
+    a.tf_val = h->tf_val.p;
+    a.tb_ptr = h->tb_ptr.as<int>();
+    a.tb_ind = h->tb_ind.as<int>();
+    a.tb_val = h->tb_val.p;
+    a.tail_wf = h->prec == 32 ? h->tail_wf.p : h->tail_d.p;
+    a.tail_wb = h->prec == 32 ? h->tail_wb.p : h->tail_e.p;
+    a.tacc = h->m_tacc.p;
+    a.tail_part = h->m_tpart.p;
+    a.tail_arrive = h->m_tarr.as<unsigned int>();
     a.x = h->m_x.as<double>();
     a.r = h->m_r.as<double>();
     a.ap = h->m_ap.as<double>();

@@ -122,7 +122,7 @@ struct rc_handle_s {
     DevVec tmp_a, tmp_b, tmp_scan, keys0, keys1, vals0, vals1, rowk, l_ptr;
     int64_t nnz_lt = 0, ell_l = 0, ell_u = 0, ell_a = 0;
     int nlevels = 0, nchunks = 0, ntiles = 0;
-    int tail_level = 0, bulk_chunks = 0;
+    int tail_level = 0, bulk_chunks = 0, bulk_segs = 0;   // bulk_segs: level segments before the tail
     bool level_order_set = false;   // RCHOL_LEVEL_ORDER given
     int level_order = 1;            // 0 length, 1 spatial (default), 2 spatial within length buckets,
                                     // 3 spatial within sweep-group classes
@@ -172,6 +172,8 @@ struct rc_handle_s {
     // multi-RHS: CSRs in position numbering (built lazily per factor) + vectors
     bool multi_ready = false;
     DevVec m_aptr, m_aind, m_aval, m_lptr, m_lind, m_lval, m_ltptr, m_ltind, m_ltval;
+    DevVec m_ccnt, m_cptr, m_cmf, m_cmb, m_tacc, m_tpart, m_tarr;
+    int m_chunk_K = 0, m_nchunks = 0;      // sweep chunks built for m_chunk_K lanes (0: not built for this factor)
     DevVec m_x, m_r, m_ap, m_p0, m_p1, m_y, m_z, m_b, m_B, m_X, m_sc, m_part;
     int m_k = 0;                    // right-hand sides held in m_B (user order, column-major)
     int m_n = 0;                    // rows of every right-hand side in m_B

@@ -82,3 +82,55 @@ def test_loaded_factor_with_unbounded_columns_is_solved_by_substitution(rc, wl, 
     got = x * (z @ z) / (x @ z)
     assert np.linalg.norm(got - z) <= n * 2.0 ** -52 * np.linalg.cond(L) ** 2 * np.linalg.norm(z)
     s.close()
+
+
+def _one_step_bound(a, f, b, x, prec):
+    """Componentwise rounding bound of one PCG step x = alpha z, z = L^-T D+ L^-1 b,
+    for two computations of it.  A triangular solve in any order of sums gives
+    (L + E) y = b with |E| <= g |L|, g = n eps, and here L^-1 >= 0, |L| = 2I - L,
+    so |dy| <= 2 g L^-1 |y| <= 2 g L^-2 |b|; the products of alpha = r'z / z'Az
+    add their own sums' errors."""
+    n = a.n
+    eps = 2.0 ** -53 if prec == 64 else 2.0 ** -24
+    g = n * eps
+    inv = np.linalg.inv(f.dense_L())
+    dp = np.where(f.diag != 0, 1.0 / np.where(f.diag != 0, f.diag, 1.0), 1.0)
+    yb = inv @ np.abs(b)
+    zb = inv.T @ (dp * yb)
+    dz = 2 * g * (inv.T @ (dp * (inv @ yb)) + inv.T @ zb) + 3 * eps * zb
+    A = a.dense()
+    z = inv.T @ (dp * (inv @ b))
+    rz, zaz = b @ z, z @ A @ z
+    h = n * 2.0 ** -53
+    dalpha = (h * (np.abs(b) @ np.abs(z)) + np.abs(b) @ dz) / rz
+    dalpha += (h * (np.abs(z) @ np.abs(A) @ np.abs(z)) + 2 * dz @ np.abs(A) @ np.abs(z)) / zaz
+    return 2 * (abs(rz / zaz) * dz + np.abs(x) * dalpha)
+
+
+@pytest.mark.parametrize("prec", [64, 32])
+@pytest.mark.parametrize("tail", ["1", "1000000"])
+@pytest.mark.parametrize("k", [1, 2, 5, 32, 64])
+def test_multi_rhs_sweeps_apply_the_preconditioner(rc, orc, wl, k, tail, prec, monkeypatch):
+    """k right-hand sides, one step: without a tail (a complete graph's rows of
+    up to 259 entries exceed the entries a chunk keeps in LDS, a grid's do not)
+    and with the whole system in the tail (more than one part per row tile)."""
+    monkeypatch.setenv("RCHOL_TAIL_ROWS", tail)
+    n = 260
+    iu, ju = np.triu_indices(n, 1)
+    w = np.random.default_rng(5).uniform(0.5, 2.0, len(iu))
+    for data in (wl.laplacian_triplets(n, iu, ju, w), wl.grid_laplacian((29, 31), "uniform_0.5_2", seed=3)):
+        n = data[0]
+        print(f"[gpu] multi tail={tail} n={n} k={k} prec={prec}", flush=True)
+        s = rc.Solver(device=0, seed=5, precision=prec, maxit=1)
+        s.set_triplets(*data)
+        s.order(rc.ORDER_NNZ_SORT, 1)
+        s.factor()
+        fac, sys_, perm, _ = orc.prepare_system(*data, order="nnz-sort", order_seed=1)
+        f = orc.factor(fac, seed=5)
+        B = np.random.default_rng(1).standard_normal((n, k))
+        B -= B.mean(axis=0)
+        X, _ = s.solve_multi(B, tol=0.0)
+        for q in range(k):
+            xo, _ = orc.pcg(sys_, f, B[perm, q], tol=0.0, maxit=1, precision=prec)
+            assert np.all(np.abs(X[perm, q] - xo) <= _one_step_bound(sys_, f, B[perm, q], xo, prec))
+        s.close()
