@@ -33,8 +33,14 @@ namespace rc {
 
 namespace {
 
-constexpr int kRedBlock = 256;
+// Workgroups of the kernels that end in a reduction: few and large.  Every
+// workgroup adds itself to one arrival counter (returning atomics on one
+// address retire about 11 ns apart) and the last one adds their partials:
+// with 1024 workgroups of 256 threads and a release fence each, k_dot took
+// 19 us on 4096 rows.
+constexpr int kRedBlock = 1024;
 
+// Sum over the workgroup in a fixed order, valid in wave 0.
 __device__ __forceinline__ double block_sum(double v, double *lds)
 {
     v = wave_sum(v);
@@ -42,10 +48,12 @@ __device__ __forceinline__ double block_sum(double v, double *lds)
     if (lane_id() == 0) lds[wid] = v;
     __syncthreads();
     double t = 0.0;
-    if (threadIdx.x == 0)
-        for (int w = 0; w < (int)(blockDim.x / kWave); ++w) t += lds[w];
+    if (wid == 0) {
+        t = lane_id() < (int)(blockDim.x / kWave) ? lds[lane_id()] : 0.0;
+        t = wave_sum(t);
+    }
     __syncthreads();
-    return t;   // valid in thread 0
+    return t;
 }
 
 // Sum of partials[0..m) by one block in a fixed order; valid in thread 0.
@@ -56,15 +64,15 @@ __device__ __forceinline__ double reduce_partials(const double *partials, int m,
     return block_sum(v, lds);
 }
 
-// Returns true in every thread of the block that arrived last.
+// Returns true in every thread of the block that arrived last.  Thread 0 wrote
+// the block's partials with agent-scope stores, and they are read the same way.
 __device__ __forceinline__ bool last_block(unsigned int *arrive, int *lds_flag)
 {
     __syncthreads();
     if (threadIdx.x == 0) {
-        fence_release();
+        drain_stores();
         unsigned int old = atomicAdd(arrive, 1u);
         *lds_flag = (old == gridDim.x - 1) ? 1 : 0;
-        if (*lds_flag) fence_acquire();
     }
     __syncthreads();
     return *lds_flag != 0;
@@ -175,12 +183,39 @@ __device__ __forceinline__ TileRange xcd_tile_range(int ntiles)
     return r;
 }
 
+// Row sum of a tile (lane = row) in entry order, eight entries in flight: the
+// tile's width is uniform, so loads past it repeat the last entry (one line)
+// and their products are left out.  (Batches of four with a scalar remainder
+// cost a 7-point row four dependent round trips.)
+template <typename F>
+__device__ __forceinline__ double tile_row(const int *ind, const double *val, int w, F load)
+{
+    constexpr int B = 8;
+    double acc = 0.0;
+    for (int t = 0; t < w; t += B) {
+        int j[B];
+        double v[B], x[B];
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+            const int e = (t + u < w ? t + u : w - 1) * kWave;
+            j[u] = ind[e];
+            v[u] = val[e];
+        }
+#pragma unroll
+        for (int u = 0; u < B; ++u) x[u] = load(j[u]);
+#pragma unroll
+        for (int u = 0; u < B; ++u)
+            if (t + u < w) acc = fma_t(v[u], x[u], acc);
+    }
+    return acc;
+}
+
 // ---------------------------------------------------------------- K1
 // p_new = z + beta p_old (streaming), then Ap = A p_new with block partials of
 // p'Ap; the last block computes alpha.  (Forming p_new inside the SpMV gather
 // would recompute it once per matrix entry.)
 template <typename T>
-__global__ void __launch_bounds__(kRedBlock) k_pupdate(SolveArgs a, const double *p_old, double *p_new)
+__global__ void __launch_bounds__(256) k_pupdate(SolveArgs a, const double *p_old, double *p_new)
 {
     PcgScalars *sc = a.sc;
     if (sc->done) return;
@@ -207,19 +242,7 @@ __global__ void __launch_bounds__(kRedBlock) k_spmv(SolveArgs a, const double *p
         const int w = a.a_width[tile];
         const int *ind = a.a_ind + a.a_off[tile] + lane;
         const double *val = a.a_val + a.a_off[tile] + lane;
-        double acc = 0.0;
-        int t = 0;
-        for (; t + 4 <= w; t += 4) {
-            int j[4];
-            double v[4], pj[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) { j[u] = ind[(t + u) * kWave]; v[u] = val[(t + u) * kWave]; }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) pj[u] = p[j[u]];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) acc = fma_t(v[u], pj[u], acc);
-        }
-        for (; t < w; ++t) acc = fma_t(val[t * kWave], p[ind[t * kWave]], acc);
+        const double acc = tile_row(ind, val, w, [&](int j) { return p[j]; });
         if (q < a.n) {
             a.ap[q] = acc;
             acc_dot += p[q] * acc;
@@ -254,19 +277,7 @@ __global__ void __launch_bounds__(kRedBlock) k_spmv_plain(SolveArgs a, const dou
         const int w = a.a_width[tile];
         const int *ind = a.a_ind + a.a_off[tile] + lane;
         const double *val = a.a_val + a.a_off[tile] + lane;
-        double acc = 0.0;
-        int t = 0;
-        for (; t + 4 <= w; t += 4) {
-            int j[4];
-            double v[4], xj[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) { j[u] = ind[(t + u) * kWave]; v[u] = val[(t + u) * kWave]; }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) xj[u] = x[j[u]];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) acc = fma_t(v[u], xj[u], acc);
-        }
-        for (; t < w; ++t) acc = fma_t(val[t * kWave], x[ind[t * kWave]], acc);
+        const double acc = tile_row(ind, val, w, [&](int j) { return x[j]; });
         if (p < a.n) y[p] = acc;
     }
 }
@@ -523,8 +534,7 @@ __global__ void __launch_bounds__(kRedBlock) k_residual(SolveArgs a)
         const int w = a.a_width[tile];
         const int *ind = a.a_ind + a.a_off[tile] + lane;
         const double *val = a.a_val + a.a_off[tile] + lane;
-        double s = 0.0;
-        for (int t = 0; t < w; ++t) s = fma_t(val[t * kWave], a.x[ind[t * kWave]], s);
+        const double s = tile_row(ind, val, w, [&](int j) { return a.x[j]; });
         if (p < a.n) {
             double d = s - a.b[p];
             acc += d * d;
@@ -637,12 +647,13 @@ void launch_bwd(const SolveArgs &a, hipStream_t s)
 // sys_of, and the per-system dot products are segmented reductions over the
 // system-major position list (see BatchArgs).  A converged system is frozen:
 // its alpha and beta are zero, so x and r keep their values and p stays z.
+constexpr int kSegBlock = 256;     // one workgroup per kBatchRows rows of a system
 enum { kOpPap = 0, kOpRz = 1, kOpBnorm = 2, kOpRes = 3 };
 
 // p_new = z + beta_sys p_old per row (streaming; the system's beta is looked
 // up once per row instead of once per matrix entry in the SpMV gather).
 template <typename T>
-__global__ void __launch_bounds__(kRedBlock) k_bpupdate(SolveArgs a, BatchArgs b, const double *p_old, double *p_new)
+__global__ void __launch_bounds__(256) k_bpupdate(SolveArgs a, BatchArgs b, const double *p_old, double *p_new)
 {
     PcgScalars *sc = a.sc;
     if (sc->done) return;
@@ -666,19 +677,7 @@ __global__ void __launch_bounds__(kRedBlock) k_bspmv(SolveArgs a, const double *
         const int w = a.a_width[tile];
         const int *ind = a.a_ind + a.a_off[tile] + lane;
         const double *val = a.a_val + a.a_off[tile] + lane;
-        double acc = 0.0;
-        int t = 0;
-        for (; t + 4 <= w; t += 4) {
-            int j[4];
-            double v[4], pj[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) { j[u] = ind[(t + u) * kWave]; v[u] = val[(t + u) * kWave]; }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) pj[u] = p[j[u]];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) acc = fma_t(v[u], pj[u], acc);
-        }
-        for (; t < w; ++t) acc = fma_t(val[t * kWave], p[ind[t * kWave]], acc);
+        const double acc = tile_row(ind, val, w, [&](int j) { return p[j]; });
         if (q < a.n) a.ap[q] = acc;
     }
 }
@@ -694,8 +693,7 @@ __global__ void __launch_bounds__(kRedBlock) k_bresid(SolveArgs a)
         const int w = a.a_width[tile];
         const int *ind = a.a_ind + a.a_off[tile] + lane;
         const double *val = a.a_val + a.a_off[tile] + lane;
-        double acc = 0.0;
-        for (int t = 0; t < w; ++t) acc = fma_t(val[t * kWave], a.x[ind[t * kWave]], acc);
+        const double acc = tile_row(ind, val, w, [&](int j) { return a.x[j]; });
         if (p < a.n) a.ap[p] = acc - a.b[p];
     }
 }
@@ -704,9 +702,9 @@ __global__ void __launch_bounds__(kRedBlock) k_bresid(SolveArgs a)
 // sums (pap: p'Ap; rz: r'z and r'r; bnorm: b'b; res: d'd and b'b with d in ap)
 // and the per-system update made by the system's last block.
 template <typename T, int Op>
-__global__ void __launch_bounds__(kRedBlock) k_bseg(SolveArgs a, BatchArgs b, const double *pv, int init)
+__global__ void __launch_bounds__(kSegBlock) k_bseg(SolveArgs a, BatchArgs b, const double *pv, int init)
 {
-    __shared__ double lds[kRedBlock / kWave];
+    __shared__ double lds[kSegBlock / kWave];
     __shared__ int flag;
     PcgScalars *sc = a.sc;
     if ((Op == kOpPap || Op == kOpRz) && sc->done) return;
@@ -744,10 +742,9 @@ __global__ void __launch_bounds__(kRedBlock) k_bseg(SolveArgs a, BatchArgs b, co
     __syncthreads();
     const int b0 = b.sys_blk0[s], b1 = b.sys_blk0[s + 1];
     if (threadIdx.x == 0) {
-        fence_release();
+        drain_stores();
         const unsigned int old = atomicAdd(b.arrive + s, 1u);
         flag = (old == (unsigned int)(b1 - b0 - 1)) ? 1 : 0;
-        if (flag) fence_acquire();
     }
     __syncthreads();
     if (!flag) return;
@@ -798,10 +795,11 @@ __global__ void __launch_bounds__(kRedBlock) k_bseg(SolveArgs a, BatchArgs b, co
             b.beta[s] = 0.0;
         }
     }
-    fence_release();
+    // the flag is all that the last arrival reads of another system
+    st_relaxed(b.done + s, b.done[s]);
+    drain_stores();
     const unsigned int old = atomicAdd(b.arrive_all, 1u);
     if (old != (unsigned int)(b.nsys - 1)) return;
-    fence_acquire();
     *b.arrive_all = 0u;
     int all = 1;
     for (int q = 0; q < b.nsys; ++q) all &= (ld_relaxed(b.done + q) != 0) ? 1 : 0;
@@ -839,7 +837,7 @@ void launch_pcg_iteration(const SolveArgs &a, int parity, hipStream_t s)
 {
     double *p_old = parity ? a.p1 : a.p0;
     double *p_new = parity ? a.p0 : a.p1;
-    hipLaunchKernelGGL(k_pupdate<T>, dim3(2048), dim3(kRedBlock), 0, s, a, (const double *)p_old, p_new);
+    hipLaunchKernelGGL(k_pupdate<T>, dim3(2048), dim3(256), 0, s, a, (const double *)p_old, p_new);
     hipLaunchKernelGGL(k_spmv<T>, dim3(a.reduce_blocks), dim3(kRedBlock), 0, s, a, (const double *)p_new);
     launch_fwd<T>(a, (const double *)p_new, 1, s);
     launch_bwd<T>(a, s);
@@ -924,11 +922,11 @@ void launch_batch_init(const SolveArgs &a, const BatchArgs &b, hipStream_t s)
     hipLaunchKernelGGL(k_fill_sentinel<T>, dim3(2048), dim3(256), 0, s, (T *)a.y, a.n);
     hipLaunchKernelGGL(k_fill_sentinel<T>, dim3(2048), dim3(256), 0, s, (T *)a.z, a.n);
     hipLaunchKernelGGL(k_pcg_prepare<T>, dim3(2048), dim3(256), 0, s, a);
-    hipLaunchKernelGGL((k_bseg<T, kOpBnorm>), dim3(batch_grid(b)), dim3(kRedBlock), 0, s, a, b,
+    hipLaunchKernelGGL((k_bseg<T, kOpBnorm>), dim3(batch_grid(b)), dim3(kSegBlock), 0, s, a, b,
                        (const double *)nullptr, 1);
     launch_fwd<T>(a, (const double *)a.p0, 0, s);
     launch_bwd<T>(a, s);
-    hipLaunchKernelGGL((k_bseg<T, kOpRz>), dim3(batch_grid(b)), dim3(kRedBlock), 0, s, a, b, (const double *)nullptr,
+    hipLaunchKernelGGL((k_bseg<T, kOpRz>), dim3(batch_grid(b)), dim3(kSegBlock), 0, s, a, b, (const double *)nullptr,
                        1);
 }
 
@@ -937,20 +935,20 @@ void launch_batch_iteration(const SolveArgs &a, const BatchArgs &b, int parity, 
 {
     double *p_old = parity ? a.p1 : a.p0;
     double *p_new = parity ? a.p0 : a.p1;
-    hipLaunchKernelGGL(k_bpupdate<T>, dim3(a.reduce_blocks), dim3(kRedBlock), 0, s, a, b, (const double *)p_old, p_new);
+    hipLaunchKernelGGL(k_bpupdate<T>, dim3(2048), dim3(256), 0, s, a, b, (const double *)p_old, p_new);
     hipLaunchKernelGGL(k_bspmv, dim3(a.reduce_blocks), dim3(kRedBlock), 0, s, a, (const double *)p_new);
-    hipLaunchKernelGGL((k_bseg<T, kOpPap>), dim3(batch_grid(b)), dim3(kRedBlock), 0, s, a, b, (const double *)p_new,
+    hipLaunchKernelGGL((k_bseg<T, kOpPap>), dim3(batch_grid(b)), dim3(kSegBlock), 0, s, a, b, (const double *)p_new,
                        0);
     launch_fwd<T>(a, (const double *)p_new, 1, s);
     launch_bwd<T>(a, s);
-    hipLaunchKernelGGL((k_bseg<T, kOpRz>), dim3(batch_grid(b)), dim3(kRedBlock), 0, s, a, b, (const double *)nullptr,
+    hipLaunchKernelGGL((k_bseg<T, kOpRz>), dim3(batch_grid(b)), dim3(kSegBlock), 0, s, a, b, (const double *)nullptr,
                        0);
 }
 
 void launch_batch_residual(const SolveArgs &a, const BatchArgs &b, hipStream_t s)
 {
     hipLaunchKernelGGL(k_bresid, dim3(a.reduce_blocks), dim3(kRedBlock), 0, s, a);
-    hipLaunchKernelGGL((k_bseg<double, kOpRes>), dim3(batch_grid(b)), dim3(kRedBlock), 0, s, a, b,
+    hipLaunchKernelGGL((k_bseg<double, kOpRes>), dim3(batch_grid(b)), dim3(kSegBlock), 0, s, a, b,
                        (const double *)nullptr, 0);
 }
 

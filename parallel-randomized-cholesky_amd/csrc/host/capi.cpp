@@ -1598,6 +1598,14 @@ static int rc_load_factor_impl(rc_handle_t h, const char *prefix)
 // ------------------------------------------------------------------ solve
 }  // extern "C"
 
+// Workgroups of the SpMV and reduction kernels (1024 rows each at least, a
+// multiple of the eight XCDs).
+static int reduction_blocks(rc_handle_t h)
+{
+    const int need = (h->ns / 1024 + 8) / 8 * 8;
+    return need < h->reduce_blocks ? need : h->reduce_blocks;
+}
+
 SolveArgs solve_args(rc_handle_t h)
 {
     SolveArgs a;
@@ -1635,7 +1643,7 @@ SolveArgs solve_args(rc_handle_t h)
     a.partials = h->partials.as<double>();
     a.ctr_fwd = h->ctrs.as<unsigned int>();
     a.ctr_bwd = h->ctrs.as<unsigned int>() + kClaimQueues * kClaimStride;
-    a.reduce_blocks = h->reduce_blocks;
+    a.reduce_blocks = reduction_blocks(h);
     a.sweep_blocks = h->sweep_blocks;
     a.bulk_chunks = h->bulk_chunks;
     a.tail_level = h->tail_level;

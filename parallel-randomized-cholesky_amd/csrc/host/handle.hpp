@@ -139,7 +139,7 @@ struct rc_handle_s {
     DevVec a_ptr, a_ind, a_val;
     DevVec x, r, ap, p0, p1, y, z, b, bu, scal, partials, ctrs, perm_d, loc_d, loc_pos;
     DevVec calib;                   // copy-kernel calibration buffer (rc_time_kernel)
-    int reduce_blocks = 1024;
+    int reduce_blocks = 256;
     int sweep_blocks = 1024;
     int sweep_blocks_max = 1024;    // occupancy limit of the persistent sweep grid
     bool rhs_set = false;
