@@ -426,9 +426,8 @@ __global__ void __launch_bounds__(kFillWaves * kWave)
     int *rbs = s_rb[wl], *rls = s_rl[wl];
     for (int c = wave; c < nchunks; c += nwaves) {
         const int nc = cnt[c];                  // <= 256 rows (sweep chunks)
-        const int P = sweep_rows_pow2(nc);
-        const int G = sweep_group(nc);
-        const int stride = P * G;
+        const int gb = sweep_group_bits(nc), sb = sweep_rows_bits(nc) + gb;
+        const int stride = 1 << sb;
         const int total = slices[c] * stride;
         const int o = off[c];
         // the previous chunk's reads of the wave's slots are done before they
@@ -455,9 +454,9 @@ __global__ void __launch_bounds__(kFillWaves * kWave)
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int idx = idx0 + u * kWave + lane;
-                const int sl = idx / stride, t = idx - sl * stride;
-                const int i = t / G, g = t - i * G;
-                const int et = sl * G + g;
+                const int sl = idx >> sb, t = idx & (stride - 1);
+                const int i = t >> gb, g = t & ((1 << gb) - 1);
+                const int et = (sl << gb) + g;
                 const bool in = idx < total && i < nc;
                 const int b = in ? rbs[i] : 0;
                 const int len = in ? rls[i] : 0;

@@ -210,16 +210,17 @@ void launch_mul64(const int *in, int *out, int n, hipStream_t s);
 // row (P = next power of two >= cnt).  Entry t of chunk row i lives in slice
 // s = t / G at off[c] + s * P * G + i * G + (t % G).  slices[c] =
 // ceil(width[c] / G); size[c] = slices[c] * P * G.
-constexpr int kSweepThreads = 256;
-__host__ __device__ inline int sweep_rows_pow2(int cnt)
+constexpr int kSweepThreads = 256, kSweepBits = 8;
+// Powers of two by shifts: an integer division costs some forty instructions
+// in the middle of the sweeps' dependency chain.
+__host__ __device__ inline int sweep_rows_bits(int cnt) { return cnt <= 1 ? 0 : 32 - __builtin_clz((unsigned)(cnt - 1)); }
+__host__ __device__ inline int sweep_rows_pow2(int cnt) { return 1 << sweep_rows_bits(cnt); }
+__host__ __device__ inline int sweep_group_bits(int cnt)
 {
-    return cnt <= 1 ? 1 : 1 << (32 - __builtin_clz((unsigned)(cnt - 1)));
+    const int g = kSweepBits - sweep_rows_bits(cnt);
+    return g > 6 ? 6 : g;
 }
-__host__ __device__ inline int sweep_group(int cnt)
-{
-    int g = kSweepThreads / sweep_rows_pow2(cnt);
-    return g > 64 ? 64 : g;
-}
+__host__ __device__ inline int sweep_group(int cnt) { return 1 << sweep_group_bits(cnt); }
 void launch_sweep_layout(int nchunks, const int *cnt, const int *width, int *slices, int *size, hipStream_t s);
 
 // Tail of the level order: the rows at positions [tp0, ns) (the narrow

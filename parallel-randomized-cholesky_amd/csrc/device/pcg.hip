@@ -78,21 +78,46 @@ __device__ __forceinline__ bool last_block(unsigned int *arrive, int *lds_flag)
     return *lds_flag != 0;
 }
 
-template <typename T>
-__device__ __noinline__ T wait_slow(T *p, long long spin_ticks, PcgScalars *sc, int nap_max)
+// Replaces the sentinels among v[u] = vec[j[u]] by their values, awaiting them.
+// All pending values of a lane are polled together: polled one after the other
+// (each with a status load in between) a row paid two device-scope round trips
+// per pending value, also for values long written whose line the L2 holds in
+// an older state.
+template <typename T, int B>
+__device__ __forceinline__ void await_values(T (&v)[B], const int (&j)[B], T *vec, long long spin_ticks, PcgScalars *sc,
+                                             int nap_max)
 {
-    long long t0 = wall_clock64();
-    int nap = 1;
+    bool pend = false;
+#pragma unroll
+    for (int u = 0; u < B; ++u) pend = pend || is_sent(v[u]);
+    if (!pend) return;
+    long long t0 = 0;
+    int tries = 0, nap = 1;
     while (true) {
-        T v = ld_relaxed_val(p);
-        if (!is_sent(v)) return v;
-        if (ld_relaxed(&sc->status) & kPcgTimeout) return (T)0;
-        if (wall_clock64() - t0 > spin_ticks) {
-            atomicOr(&sc->status, kPcgTimeout);
-            return (T)0;
+#pragma unroll
+        for (int u = 0; u < B; ++u)
+            if (is_sent(v[u])) v[u] = ld_relaxed_val(vec + j[u]);
+        pend = false;
+#pragma unroll
+        for (int u = 0; u < B; ++u) pend = pend || is_sent(v[u]);
+        if (!pend) return;
+        if ((++tries & 63) == 0) {               // bounded: see kPcgTimeout
+            const long long now = wall_clock64();
+            if (t0 == 0) t0 = now;
+            bool stop = (ld_relaxed(&sc->status) & kPcgTimeout) != 0;
+            if (now - t0 > spin_ticks) {
+                atomicOr(&sc->status, kPcgTimeout);
+                stop = true;
+            }
+            if (stop) {
+#pragma unroll
+                for (int u = 0; u < B; ++u) v[u] = is_sent(v[u]) ? (T)0 : v[u];
+                return;
+            }
         }
-        // exponential back-off keeps waiting waves from flooding memory
-        for (int q = 0; q < nap; ++q) __builtin_amdgcn_s_sleep(2);
+        // polls follow at once (a first s_sleep 2 cost 2-5 % of the sweeps);
+        // nap_max > 1 lets the back-off grow
+        for (int q = 1; q < nap; ++q) __builtin_amdgcn_s_sleep(2);
         nap = nap < nap_max ? nap * 2 : nap_max;
     }
 }
@@ -116,18 +141,16 @@ __device__ __forceinline__ T grouped_row_solve(const int *ind, const T *val, int
         }
 #pragma unroll
         for (int u = 0; u < B; ++u) v[u] = vec[j[u]];
+        await_values<T, B>(v, j, vec, spin, sc, nap_max);
 #pragma unroll
-        for (int u = 0; u < B; ++u) {
-            if (is_sent(v[u])) v[u] = wait_slow(vec + j[u], spin, sc, nap_max);
-            acc = fma_t(-l[u], v[u], acc);
-        }
+        for (int u = 0; u < B; ++u) acc = fma_t(-l[u], v[u], acc);
     }
     for (; sl < nsl; ++sl) {
-        int j = ind[sl * stride];
+        int j[1] = {ind[sl * stride]};
         T l = val[sl * stride];
-        T v = vec[j];
-        if (is_sent(v)) v = wait_slow(vec + j, spin, sc, nap_max);
-        acc = fma_t(-l, v, acc);
+        T v[1] = {vec[j[0]]};
+        await_values<T, 1>(v, j, vec, spin, sc, nap_max);
+        acc = fma_t(-l, v[0], acc);
     }
     return acc;
 }
@@ -143,13 +166,14 @@ __device__ __forceinline__ T grouped_row_solve_pref(const int *jp, const T *lp, 
                                                     int nap_max)
 {
     T v[kBulkPref];
+    int j[kBulkPref];
 #pragma unroll
     for (int u = 0; u < kBulkPref; ++u) v[u] = vec[jp[u]];
 #pragma unroll
-    for (int u = 0; u < kBulkPref; ++u) {
-        if (is_sent(v[u])) v[u] = wait_slow(vec + jp[u], spin, sc, nap_max);
-        acc = fma_t(-lp[u], v[u], acc);
-    }
+    for (int u = 0; u < kBulkPref; ++u) j[u] = jp[u];
+    await_values<T, kBulkPref>(v, j, vec, spin, sc, nap_max);
+#pragma unroll
+    for (int u = 0; u < kBulkPref; ++u) acc = fma_t(-lp[u], v[u], acc);
     if (nsl > kBulkPref)
         acc = grouped_row_solve<T>(ind + kBulkPref * stride, val + kBulkPref * stride, nsl - kBulkPref, stride, vec,
                                    acc, spin, sc, nap_max);
@@ -295,9 +319,10 @@ __device__ __forceinline__ void fwd_chunk(const SolveArgs &a, int4 m, int t, dou
     T *y = (T *)a.y;
     T *z = (T *)a.z;
     const int cnt = m.y;
-    const int G = sweep_group(cnt);
-    const int stride = sweep_rows_pow2(cnt) * G;
-    const int i = t / G, g = t - i * G;
+    const int lg = sweep_group_bits(cnt);
+    const int G = 1 << lg;
+    const int stride = sweep_rows_pow2(cnt) << lg;
+    const int i = t >> lg, g = t & (G - 1);
     const bool active = t < stride && i < cnt;
     const bool lead = active && g == G - 1;     // the lane that receives the group sum
     const int k = m.x + i;
@@ -340,9 +365,10 @@ __device__ __forceinline__ void bwd_chunk(const SolveArgs &a, int4 m, int t, con
     T *y = (T *)a.y;
     T *z = (T *)a.z;
     const int cnt = m.y;
-    const int G = sweep_group(cnt);
-    const int stride = sweep_rows_pow2(cnt) * G;
-    const int i = t / G, g = t - i * G;
+    const int lg = sweep_group_bits(cnt);
+    const int G = 1 << lg;
+    const int stride = sweep_rows_pow2(cnt) << lg;
+    const int i = t >> lg, g = t & (G - 1);
     const bool active = t < stride && i < cnt;
     const bool lead = active && g == G - 1;     // the lane that receives the group sum
     const int k = m.x + i;
@@ -409,7 +435,7 @@ __global__ void __launch_bounds__(kSweepThreads) k_sweep_bulk(SolveArgs a, const
     // zero entry where it has no slice), and nothing is computed from the
     // values until the chunk is processed
     auto fetch = [&](const int4 &m, int *j, T *l) {
-        const int stride = sweep_rows_pow2(m.y) * sweep_group(m.y);
+        const int stride = sweep_rows_pow2(m.y) << sweep_group_bits(m.y);
 #pragma unroll
         for (int u = 0; u < kBulkPref; ++u) {
             const bool has = t < stride && u < m.w;
