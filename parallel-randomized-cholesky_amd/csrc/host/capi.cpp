@@ -101,8 +101,9 @@ static int rc_create_impl(rc_handle_t *out, const rc_options *opt)
     h->na_err = noalloc_workspace(o.device, &h->na_ws);
     h->num_blocks = o.num_blocks > 0 ? o.num_blocks : factor_occupancy_blocks(o.device);
     factor_kernel_setup();
-    h->sweep_blocks = sweep_occupancy_blocks(o.device);
-    h->sweep_blocks_max = h->sweep_blocks;
+    h->sweep_blocks_max = sweep_occupancy_blocks(o.device);
+    if (hipDeviceGetAttribute(&h->cus, hipDeviceAttributeMultiprocessorCount, o.device) != hipSuccess || h->cus < 1)
+        h->cus = 256;
     {
         const char *lo = std::getenv("RCHOL_LEVEL_ORDER");      // "spatial" (default) | "length" | "bucket"
         if (lo && std::string(lo) == "length") h->level_order = 0;
@@ -853,13 +854,13 @@ static int bit_width(int64_t v)
 // First level of the tail (see dense_tail.hip).  With a width limit, the
 // trailing run of narrower levels; limit < 0: the split with the least
 // estimated sweep time.  A level of the dataflow sweep costs one store ->
-// poll round trip through device-scope memory (2.2 us, measured), a tail block
+// poll round trip through device-scope memory (1.8 us, measured), a tail block
 // two launches and their memory round trips (about 9 us, its share of the
 // inversion included) and the bytes of its triangle (3 TB/s).  Returns the widest tail
 // level + 1 in *width.
 static int tail_start(int limit, const std::vector<int> &hl, int nl, int vbytes, int *width)
 {
-    constexpr double kLevelUs = 2.2, kBulkUs = 6.0, kBlockUs = 9.0, kBytesPerUs = 3.0e6;
+    constexpr double kLevelUs = 1.8, kBulkUs = 6.0, kBlockUs = 9.0, kBytesPerUs = 3.0e6;
     const int ns = nl > 0 ? hl[(size_t)nl] : 0;
     int best = nl, widest = 0;
     double best_us = nl * kLevelUs + (nl > 0 ? kBulkUs : 0.0);
@@ -1606,6 +1607,22 @@ static int reduction_blocks(rc_handle_t h)
     return need < h->reduce_blocks ? need : h->reduce_blocks;
 }
 
+// Persistent sweep workgroups for `values` vector entries (rows x lanes): the
+// autotuner's choice, else one per CU, two from 1.5 M values, for many
+// right-hand sides four from 32 M.  More of them hold chunks far ahead of the front, and their polls
+// slow it down; wide levels want more in flight.  Forward / backward sweep, us,
+// at 256 / 512 / 1024 workgroups: 64^3 SDDM 231/225, 252/243, 285/289; 701x699
+// 130/119, 141/129, 156/154; 128^3 SDDM 611/625, 589/586, 663/679; 192^3
+// learned 993/951, 960/882, 1035/965; 47x48x45 x 5 318/317, 341/341, 356/359;
+// 385x384 x 64 280/305, 203/235, 203/243; 2048x1024 x 64 4365/4412, 2468/2470,
+// 2466/1594.
+static int sweep_grid(rc_handle_t h, double values, bool multi)
+{
+    if (h->sweep_blocks > 0) return h->sweep_blocks;
+    const int per_cu = values < 1.5e6 ? 1 : (multi && values > 3.2e7 ? 4 : 2);
+    return std::min(h->sweep_blocks_max, per_cu * h->cus);
+}
+
 SolveArgs solve_args(rc_handle_t h)
 {
     SolveArgs a;
@@ -1644,7 +1661,7 @@ SolveArgs solve_args(rc_handle_t h)
     a.ctr_fwd = h->ctrs.as<unsigned int>();
     a.ctr_bwd = h->ctrs.as<unsigned int>() + kClaimQueues * kClaimStride;
     a.reduce_blocks = reduction_blocks(h);
-    a.sweep_blocks = h->sweep_blocks;
+    a.sweep_blocks = sweep_grid(h, h->ns, false);
     a.bulk_chunks = h->bulk_chunks;
     a.tail_level = h->tail_level;
     a.tail_pos0 = h->tail_pos0;
@@ -1991,7 +2008,7 @@ static int multi_args(rc_handle_t h, int k, MultiArgs &a)
     a.ctr_fwd = h->ctrs.as<unsigned int>();
     a.ctr_bwd = h->ctrs.as<unsigned int>() + kClaimQueues * kClaimStride;
     a.reduce_blocks = h->reduce_blocks;
-    a.sweep_blocks = h->sweep_blocks;
+    a.sweep_blocks = sweep_grid(h, (double)n * K, true);
     a.spin_ticks = h->spin_ticks;
     return RC_OK;
 }
@@ -2678,7 +2695,7 @@ static int rc_autotune_impl(rc_handle_t h, int reps, rc_tune_stats *st)
         *out = f + b;
         return rc;
     };
-    const int tail0 = h->tail_max_rows, grid0 = h->sweep_blocks;
+    const int tail0 = h->tail_max_rows, grid0 = sweep_grid(h, h->ns, false);
     double base = 0.0;
     int rc = sweep_ms(&base);
     if (rc != RC_OK) return rc;

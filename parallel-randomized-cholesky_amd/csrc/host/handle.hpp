@@ -140,7 +140,8 @@ struct rc_handle_s {
     DevVec x, r, ap, p0, p1, y, z, b, bu, scal, partials, ctrs, perm_d, loc_d, loc_pos;
     DevVec calib;                   // copy-kernel calibration buffer (rc_time_kernel)
     int reduce_blocks = 256;
-    int sweep_blocks = 1024;
+    int cus = 256;                  // compute units of the device
+    int sweep_blocks = 0;           // persistent sweep grid chosen by the autotuner (0: sweep_grid)
     int sweep_blocks_max = 1024;    // occupancy limit of the persistent sweep grid
     bool rhs_set = false;
     std::vector<double> xref;
