@@ -35,30 +35,44 @@ __device__ __forceinline__ float bf16r(float x)
 __device__ __forceinline__ unsigned short bf16bits(float x) { return (unsigned short)(__float_as_uint(bf16r(x)) >> 16); }
 
 // ---------------------------------------------------------------- aggregation
-// M[v, :D] = sum_u a[v,u] H[u, :D]; D = 64: one wave per row, lane = feature.
-__global__ void k_agg64(int n, const int *ptr, const int *ind, const float *a, const float *H, float *M)
+// M[v, :] = sum_u a[v,u] H[u, :] (kAdd = false) or the transposed aggregation of
+// the backward pass, M[u, :] += sum_{v in N(u)} a[v,u] H[v, :] with a[v,u] =
+// w / wdeg_v stored at the (u -> v) entry.  Sixteen lanes per row, four features
+// each; the row's entries eight at a time (indices, then the gathers, all in
+// flight), summed in entry order.  Bound by the gathered rows; one wave per row
+// with one entry in flight took 33 us at 64k rows, this 15 us.
+template <bool kAdd>
+__global__ void __launch_bounds__(256) k_agg64(int n, const int *ptr, const int *ind, const float *a, const float *H,
+                                               float *M)
 {
-    const int lane = lane_id();
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-    const int nwaves = gridDim.x * blockDim.x / kWave;
-    for (int v = wave; v < n; v += nwaves) {
-        float acc = 0.f;
-        for (int e = ptr[v]; e < ptr[v + 1]; ++e) acc = fmaf(a[e], H[(size_t)ind[e] * kH + lane], acc);
-        M[(size_t)v * kH + lane] = acc;
-    }
-}
-
-// Transposed aggregation for the backward pass: out[u] += sum_{v in N(u)} a[v,u] G[v]
-// with a[v,u] = w / wdeg_v stored at the (u -> v) entry as at[e].
-__global__ void k_aggT64(int n, const int *ptr, const int *ind, const float *at, const float *G, float *out)
-{
-    const int lane = lane_id();
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-    const int nwaves = gridDim.x * blockDim.x / kWave;
-    for (int u = wave; u < n; u += nwaves) {
-        float acc = out[(size_t)u * kH + lane];
-        for (int e = ptr[u]; e < ptr[u + 1]; ++e) acc = fmaf(at[e], G[(size_t)ind[e] * kH + lane], acc);
-        out[(size_t)u * kH + lane] = acc;
+    constexpr int B = 8;
+    const int c = (threadIdx.x & 15) * 4;
+    for (int v = blockIdx.x * 16 + threadIdx.x / 16; v < n; v += gridDim.x * 16) {
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (kAdd) acc = *reinterpret_cast<const float4 *>(M + (size_t)v * kH + c);
+        const int e1 = ptr[v + 1];
+        for (int e = ptr[v]; e < e1; e += B) {
+            int j[B];
+            float w[B];
+            float4 h[B];
+#pragma unroll
+            for (int u = 0; u < B; ++u) {
+                const int ee = e + u < e1 ? e + u : e1 - 1;
+                j[u] = ind[ee];
+                w[u] = a[ee];
+            }
+#pragma unroll
+            for (int u = 0; u < B; ++u) h[u] = *reinterpret_cast<const float4 *>(H + (size_t)j[u] * kH + c);
+#pragma unroll
+            for (int u = 0; u < B; ++u)
+                if (e + u < e1) {
+                    acc.x = fmaf(w[u], h[u].x, acc.x);
+                    acc.y = fmaf(w[u], h[u].y, acc.y);
+                    acc.z = fmaf(w[u], h[u].z, acc.z);
+                    acc.w = fmaf(w[u], h[u].w, acc.w);
+                }
+        }
+        *reinterpret_cast<float4 *>(M + (size_t)v * kH + c) = acc;
     }
 }
 
@@ -76,7 +90,7 @@ __global__ void k_agg2(int n, const int *ptr, const int *ind, const float *a, co
 }
 
 // ---------------------------------------------------------------- layer 1 (2 -> 64)
-__global__ void k_dense1(int n, const float *H0, const float *M1, const float *w, float *Z, float *H)
+__global__ void k_dense1(int n, const float *H0, const float *M1, const float *w, float *H)
 {
     const float *Ws = w + kGnnWs1, *Wn = w + kGnnWn1, *b = w + kGnnB1;
     const int lane = lane_id();
@@ -93,7 +107,6 @@ __global__ void k_dense1(int n, const float *H0, const float *M1, const float *w
         z = fmaf(ws1, h1, z);
         z = fmaf(wn0, m0, z);
         z = fmaf(wn1, m1, z);
-        Z[(size_t)v * kH + lane] = z;
         H[(size_t)v * kH + lane] = z > 0.f ? z : 0.f;
     }
 }
@@ -104,54 +117,63 @@ __global__ void k_dense1(int n, const float *H0, const float *M1, const float *w
 // v_mfma_f32_16x16x16_bf16 operand layout (per lane l): A holds row l % 16,
 // k = 4 (l / 16) .. +3; B holds column l % 16, same k; D holds rows
 // 4 (l / 16) .. +3 of column l % 16.
+// All of W stays in the wave's registers (64 x 128 bf16 are 64 per lane); a lane
+// loads its row 16 bytes at a time.  (Through LDS, 16 lanes met in one bank and
+// every workgroup converted W for 64 rows: 50 us at 64k rows, now 16.)
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-__global__ void __launch_bounds__(256) k_dense_mfma(int n, const float *Hin, const float *Min, const float *Ws,
-                                                    const float *Wn, const float *b, float *Z, float *Hout)
+__device__ __forceinline__ bf16x4 to_bf16x4(float4 v)
 {
-    __shared__ unsigned short sw[kH * 2 * kH];   // W[o][k], k < 128, bf16 bits
-    for (int i = threadIdx.x; i < kH * 2 * kH; i += blockDim.x) {
-        int o = i / (2 * kH), k = i % (2 * kH);
-        float v = k < kH ? Ws[o * kH + k] : Wn[o * kH + (k - kH)];
-        sw[i] = bf16bits(v);
-    }
-    __syncthreads();
+    bf16x4 r;
+    r[0] = (short)bf16bits(v.x);
+    r[1] = (short)bf16bits(v.y);
+    r[2] = (short)bf16bits(v.z);
+    r[3] = (short)bf16bits(v.w);
+    return r;
+}
+
+__global__ void __launch_bounds__(256) k_dense_mfma(int n, const float *Hin, const float *Min, const float *Ws,
+                                                    const float *Wn, const float *b, float *Hout)
+{
     const int lane = lane_id();
-    const int wid = threadIdx.x / kWave;
     const int r16 = lane % 16, kq = lane / 16;
-    const int ntiles = (n + 15) / 16;
-    for (int tile = blockIdx.x * 4 + wid; tile < ntiles; tile += gridDim.x * 4) {
-        const int row = tile * 16 + r16;
-        f32x4 acc[4];
-        for (int c = 0; c < 4; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bf16x4 wv[8][4];
+    float bias[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const int col = c * 16 + r16;
+        bias[c] = b[col];
+#pragma unroll
         for (int ks = 0; ks < 8; ++ks) {
-            const int k0 = ks * 16 + kq * 4;
-            bf16x4 av;
-            for (int t = 0; t < 4; ++t) {
-                int k = k0 + t;
-                float x = 0.f;
-                if (row < n) x = k < kH ? Hin[(size_t)row * kH + k] : Min[(size_t)row * kH + (k - kH)];
-                av[t] = (short)bf16bits(x);
-            }
-            for (int c = 0; c < 4; ++c) {
-                const int col = c * 16 + r16;
-                bf16x4 bv;
-                for (int t = 0; t < 4; ++t) bv[t] = (short)sw[col * 2 * kH + k0 + t];
-                acc[c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, bv, acc[c], 0, 0, 0);
-            }
+            const float *W = ks < 4 ? Ws : Wn;
+            wv[ks][c] = to_bf16x4(*reinterpret_cast<const float4 *>(W + col * kH + (ks & 3) * 16 + kq * 4));
         }
-        for (int c = 0; c < 4; ++c) {
-            const int col = c * 16 + r16;
+    }
+    const int ntiles = (n + 15) / 16;
+    for (int tile = blockIdx.x * 4 + threadIdx.x / kWave; tile < ntiles; tile += gridDim.x * 4) {
+        const int row = min(tile * 16 + r16, n - 1);          // rows past the end are not written
+        float4 x[8];
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks)
+            x[ks] = *reinterpret_cast<const float4 *>((ks < 4 ? Hin : Min) + (size_t)row * kH + (ks & 3) * 16 + kq * 4);
+        f32x4 acc[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) {
+            const bf16x4 av = to_bf16x4(x[ks]);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) acc[c] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(av, wv[ks][c], acc[c], 0, 0, 0);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
             for (int t = 0; t < 4; ++t) {
                 const int rr = tile * 16 + kq * 4 + t;
-                if (rr < n) {
-                    float z = acc[c][t] + b[col];
-                    Z[(size_t)rr * kH + col] = z;
-                    Hout[(size_t)rr * kH + col] = z > 0.f ? z : 0.f;
-                }
+                const float z = acc[c][t] + bias[c];
+                if (rr < n) Hout[(size_t)rr * kH + c * 16 + r16] = z > 0.f ? z : 0.f;
             }
-        }
     }
 }
 
@@ -172,119 +194,249 @@ __global__ void k_score(int n, const float *H3, const float *w, float *s)
 }
 
 // ---------------------------------------------------------------- backward
-// dH3[v][o] = ds[v] wo[o]; partial dwo / dbo per block.
-__global__ void k_score_back(int n, const float *H3, const float *w, const float *ds, float *dH, float *part)
+// dZ = dH where H > 0 (H = relu(Z)); at the output layer dH[v][o] = ds[v] wo[o]
+// is formed on the fly.  Four consecutive features c..c+3 of row v.
+template <bool kLast>
+__device__ __forceinline__ void load_dz(int v, int c, const float *dH, const float *H, const float *ds,
+                                        const float *wl, float *dz, float *h)
 {
-    const float *wo = w + kGnnWo;
-    const int lane = lane_id();
-    const float wl = bf16r(wo[lane]);
-    float gwo = 0.f, gbo = 0.f;
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-    const int nwaves = gridDim.x * blockDim.x / kWave;
-    for (int v = wave; v < n; v += nwaves) {
-        float d = ds[v];
-        dH[(size_t)v * kH + lane] = d * wl;
-        gwo = fmaf(d, bf16r(H3[(size_t)v * kH + lane]), gwo);
-        gbo += d;
+    const float4 hv = *reinterpret_cast<const float4 *>(H + (size_t)v * kH + c);
+    h[0] = hv.x; h[1] = hv.y; h[2] = hv.z; h[3] = hv.w;
+    if (kLast) {
+        const float d = ds[v];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) dz[t] = d * wl[t];
+    } else {
+        const float4 g = *reinterpret_cast<const float4 *>(dH + (size_t)v * kH + c);
+        dz[0] = g.x; dz[1] = g.y; dz[2] = g.z; dz[3] = g.w;
     }
-    // fixed-order per-block reduction over the block's waves through LDS
-    __shared__ float red[256];
-    red[threadIdx.x] = gwo;
-    __syncthreads();
-    if (threadIdx.x < kWave) {
-        float t = 0.f;
-        for (int w2 = 0; w2 < (int)blockDim.x / kWave; ++w2) t += red[w2 * kWave + threadIdx.x];
-        part[(size_t)blockIdx.x * (kH + 1) + threadIdx.x] = t;
-    }
-    __syncthreads();
-    red[threadIdx.x] = lane == 0 ? gbo : 0.f;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float t = 0.f;
-        for (int w2 = 0; w2 < (int)blockDim.x / kWave; ++w2) t += red[w2 * kWave];
-        part[(size_t)blockIdx.x * (kH + 1) + kH] = t;
-    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) dz[t] = h[t] > 0.f ? dz[t] : 0.f;
 }
 
-// dZ = dH * (Z > 0) in place in dH.
-__global__ void k_relu_back(size_t total, const float *Z, float *dH)
+// Weight-gradient partials of a 64-wide layer over this workgroup's rows:
+// gWs[o][i] = sum_v dZ[v][o] bf16(X[v][i]), gWn likewise with M, gb[o] = sum_v
+// dZ[v][o]; at the output layer also gwo[o] = sum_v ds[v] bf16(H[v][o]) and gbo =
+// sum_v ds[v].  Products on v_mfma_f32_16x16x4_f32 (FP32 in and accumulated),
+// four rows a step: lane l holds features 4 (l % 16) .. +3 of row l / 16, so
+// tile t of an operand is made of the features 4 j + t.  A wave keeps all 64 x
+// 128 sums; the workgroup's waves are added through LDS in order.  (One thread
+// per output row and 250 rows one after the other took 567 us at 64k rows, this
+// 25 us.)
+// Layout of a partial: [Ws | Wn | b | wo | bo], as in the weights.
+constexpr int kWgLen = 2 * kH * kH + kH + kH + 1;
+template <bool kLast>
+__global__ void __launch_bounds__(256) k_wgrad64(int n, int rows_per_wave, const float *dH, const float *H,
+                                                 const float *ds, const float *wo, const float *X, const float *M,
+                                                 float *part)
 {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x)
-        if (!(Z[i] > 0.f)) dH[i] = 0.f;
-}
-
-// Weight-gradient partials of one layer: for the rows of this block,
-// gWs[o][i] = sum_v dZ[v][o] bf16(X[v][i]), gWn likewise with M, gb[o] = sum dZ.
-// Thread (o, i-slice): 256 threads = 64 outputs x 4 slices of the D inputs.
-template <int D>
-__global__ void __launch_bounds__(256) k_wgrad(int n, int rows_per_block, const float *dZ, const float *X,
-                                               const float *M, float *part)
-{
-    const int o = threadIdx.x % kH;
-    const int slice = threadIdx.x / kH;      // 0..3
-    constexpr int per = (D + 3) / 4;
-    float gs[per], gn[per];
-    for (int t = 0; t < per; ++t) { gs[t] = 0.f; gn[t] = 0.f; }
-    float gb = 0.f;
-    const int r0 = blockIdx.x * rows_per_block;
-    const int r1 = min(n, r0 + rows_per_block);
-    for (int v = r0; v < r1; ++v) {
-        const float d = dZ[(size_t)v * kH + o];
-        if (d == 0.f) continue;
-        for (int t = 0; t < per; ++t) {
-            const int i = slice * per + t;
-            if (i < D) {
-                gs[t] = fmaf(d, bf16r(X[(size_t)v * D + i]), gs[t]);
-                gn[t] = fmaf(d, bf16r(M[(size_t)v * D + i]), gn[t]);
+    __shared__ float red[2 * kH * kH];
+    __shared__ float redb[4][2 * kH + 1];
+    const int lane = lane_id(), w = threadIdx.x / kWave;
+    const int c = (lane & 15) * 4, vq = lane >> 4;
+    float wl[4] = {0.f, 0.f, 0.f, 0.f};
+    if (kLast)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) wl[t] = bf16r(wo[c + t]);
+    f32x4 ax[4][4], am[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) ax[i][j] = am[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float gb[4] = {0.f, 0.f, 0.f, 0.f}, gwo[4] = {0.f, 0.f, 0.f, 0.f}, gbo = 0.f;
+    const int v0 = min((blockIdx.x * 4 + w) * rows_per_wave, n);
+    const int v1 = min(v0 + rows_per_wave, n);
+    constexpr int U = 2;
+    for (int vb = v0; vb < v1; vb += 4 * U) {
+        float dz[U][4], h[U][4];
+        float4 x[U], m[U];
+        float d[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int v = min(vb + 4 * u + vq, v1 - 1);
+            load_dz<kLast>(v, c, dH, H, ds, wl, dz[u], h[u]);
+            x[u] = *reinterpret_cast<const float4 *>(X + (size_t)v * kH + c);
+            m[u] = *reinterpret_cast<const float4 *>(M + (size_t)v * kH + c);
+            d[u] = kLast ? ds[v] : 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool in = vb + 4 * u + vq < v1;
+            const float xv[4] = {bf16r(x[u].x), bf16r(x[u].y), bf16r(x[u].z), bf16r(x[u].w)};
+            const float mv[4] = {bf16r(m[u].x), bf16r(m[u].y), bf16r(m[u].z), bf16r(m[u].w)};
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                dz[u][t] = in ? dz[u][t] : 0.f;
+                gb[t] += dz[u][t];
+                if (kLast && in) gwo[t] = fmaf(d[u], bf16r(h[u][t]), gwo[t]);
             }
-        }
-        gb += d;
-    }
-    // layout of a block's partial: [Ws (64 x D) | Wn (64 x D) | b (64)]
-    float *p = part + (size_t)blockIdx.x * (2 * kH * D + kH);
-    for (int t = 0; t < per; ++t) {
-        const int i = slice * per + t;
-        if (i < D) {
-            p[o * D + i] = gs[t];
-            p[kH * D + o * D + i] = gn[t];
+            if (kLast && in) gbo += d[u];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    ax[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(dz[u][i], xv[j], ax[i][j], 0, 0, 0);
+                    am[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(dz[u][i], mv[j], am[i][j], 0, 0, 0);
+                }
         }
     }
-    if (slice == 0) p[2 * kH * D + o] = gb;
+    // the four rows of a step sit in the lane groups of 16
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int off = 16; off < kWave; off <<= 1) {
+            gb[t] += __shfl_xor(gb[t], off, kWave);
+            gwo[t] += __shfl_xor(gwo[t], off, kWave);
+        }
+    gbo += __shfl_xor(gbo, 16, kWave);
+    gbo += __shfl_xor(gbo, 32, kWave);
+    if (lane < 16)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            redb[w][c + t] = gb[t];
+            redb[w][kH + c + t] = gwo[t];
+        }
+    if (lane == 0) redb[w][2 * kH] = gbo;
+    for (int s = 0; s < 4; ++s) {
+        if (w == s)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const int o = 4 * (4 * vq + q) + i, col = c + j;     // row 4 (l / 16) + q of tile i
+                        float &rx = red[o * kH + col], &rm = red[kH * kH + o * kH + col];
+                        rx = s == 0 ? ax[i][j][q] : rx + ax[i][j][q];
+                        rm = s == 0 ? am[i][j][q] : rm + am[i][j][q];
+                    }
+        __syncthreads();
+    }
+    float *p = part + (size_t)blockIdx.x * kWgLen;
+    for (int i = threadIdx.x; i < 2 * kH * kH; i += 256) p[i] = red[i];
+    if (threadIdx.x < 2 * kH + 1)
+        p[2 * kH * kH + threadIdx.x] = ((redb[0][threadIdx.x] + redb[1][threadIdx.x]) + redb[2][threadIdx.x]) +
+                                       redb[3][threadIdx.x];
 }
 
-// Sum block partials (fixed order) into out[0..len).
-__global__ void k_sum_partials(const float *part, int nblocks, int len, float *out)
+// The same for the first layer (two inputs): lane = output, four rows in
+// flight per wave.
+constexpr int kWgLen2 = 2 * kH * 2 + kH;
+__global__ void __launch_bounds__(256) k_wgrad2(int n, int rows_per_wave, const float *dH, const float *H,
+                                                const float *X, const float *M, float *part)
 {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < len; i += gridDim.x * blockDim.x) {
-        float s = 0.f;
-        for (int b = 0; b < nblocks; ++b) s += part[(size_t)b * len + i];
-        out[i] = s;
+    __shared__ float red[4][5][kWave];
+    const int lane = lane_id(), w = threadIdx.x / kWave;
+    float g[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+    const int v0 = min((blockIdx.x * 4 + w) * rows_per_wave, n);
+    const int v1 = min(v0 + rows_per_wave, n);
+    constexpr int U = 8;
+    for (int vb = v0; vb < v1; vb += U) {
+        float d[U];
+        float2 x[U], m[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int v = min(vb + u, v1 - 1);
+            d[u] = H[(size_t)v * kH + lane] > 0.f ? dH[(size_t)v * kH + lane] : 0.f;
+            x[u] = *reinterpret_cast<const float2 *>(X + (size_t)v * 2);
+            m[u] = *reinterpret_cast<const float2 *>(M + (size_t)v * 2);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const float dv = vb + u < v1 ? d[u] : 0.f;
+            g[0] = fmaf(dv, bf16r(x[u].x), g[0]);
+            g[1] = fmaf(dv, bf16r(x[u].y), g[1]);
+            g[2] = fmaf(dv, bf16r(m[u].x), g[2]);
+            g[3] = fmaf(dv, bf16r(m[u].y), g[3]);
+            g[4] += dv;
+        }
     }
-}
-
-// dX[v][i] = sum_o dZ[v][o] bf16(Ws[o][i]);  G[v][i] = sum_o dZ[v][o] bf16(Wn[o][i])
-// (D = 64: one wave per row, lane = i).
-__global__ void k_back_dense(int n, const float *dZ, const float *Ws, const float *Wn, float *dX, float *G)
-{
-    __shared__ float ws[kH * kH], wn[kH * kH];
-    for (int t = threadIdx.x; t < kH * kH; t += blockDim.x) {
-        ws[t] = bf16r(Ws[t]);
-        wn[t] = bf16r(Wn[t]);
-    }
+#pragma unroll
+    for (int i = 0; i < 5; ++i) red[w][i][lane] = g[i];
     __syncthreads();
-    const int lane = lane_id();
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-    const int nwaves = gridDim.x * blockDim.x / kWave;
-    for (int v = wave; v < n; v += nwaves) {
-        const float dz = dZ[(size_t)v * kH + lane];
-        float a = 0.f, g = 0.f;
-        for (int o = 0; o < kH; ++o) {
-            const float d = __shfl(dz, o, kWave);
-            a = fmaf(d, ws[o * kH + lane], a);
-            g = fmaf(d, wn[o * kH + lane], g);
+    if (w != 0) return;
+    float *p = part + (size_t)blockIdx.x * kWgLen2;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) g[i] = ((red[0][i][lane] + red[1][i][lane]) + red[2][i][lane]) + red[3][i][lane];
+    p[lane * 2] = g[0];
+    p[lane * 2 + 1] = g[1];
+    p[2 * kH + lane * 2] = g[2];
+    p[2 * kH + lane * 2 + 1] = g[3];
+    p[4 * kH + lane] = g[4];
+}
+
+// Sum of nblocks partials into out[0..len), eight threads per output, each over
+// its share of the partials in order, then the eight in order.
+__global__ void __launch_bounds__(256) k_sum_partials(const float *part, int nblocks, int stride, int len,
+                                                      float *out)
+{
+    __shared__ float red[8][32];
+    const int o = threadIdx.x & 31, s = threadIdx.x >> 5;
+    const int i = blockIdx.x * 32 + o;
+    const int per = (nblocks + 7) / 8;
+    const int b0 = s * per, b1 = min(nblocks, b0 + per);
+    float t = 0.f;
+    if (i < len)
+        for (int b = b0; b < b1; b += 8) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = b + u < b1 ? part[(size_t)(b + u) * stride + i] : 0.f;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) t += v[u];
         }
-        dX[(size_t)v * kH + lane] = a;
-        G[(size_t)v * kH + lane] = g;
+    red[s][o] = t;
+    __syncthreads();
+    if (s == 0 && i < len) {
+        for (int q = 1; q < 8; ++q) t += red[q][o];
+        out[i] = t;
+    }
+}
+
+// dX[v][i] = sum_o dZ[v][o] bf16(Ws[o][i]);  G[v][i] = sum_o dZ[v][o] bf16(Wn[o][i]):
+// 16 rows x 128 outputs per wave on v_mfma_f32_16x16x4_f32 with both weight
+// matrices in registers (128 per lane): 20 us at 64k rows (one row per wave with
+// 64 broadcasts, 98).
+template <bool kLast>
+__global__ void __launch_bounds__(256) k_back_dense(int n, const float *dH, const float *H, const float *ds,
+                                                    const float *wo, const float *Ws, const float *Wn, float *dX,
+                                                    float *G)
+{
+    const int lane = lane_id();
+    const int r16 = lane % 16, kq = lane / 16;
+    float wv[4][4][8];           // [k block][k in block][column tile]: W[16 b + 4 kq + j][16 c + r16]
+    float wl[4][4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int o = 16 * b + 4 * kq + j;
+            wl[b][j] = kLast ? bf16r(wo[o]) : 0.f;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) wv[b][j][c] = bf16r((c < 4 ? Ws : Wn)[o * kH + (c & 3) * 16 + r16]);
+        }
+    const int ntiles = (n + 15) / 16;
+    for (int tile = blockIdx.x * 4 + threadIdx.x / kWave; tile < ntiles; tile += gridDim.x * 4) {
+        const int row = min(tile * 16 + r16, n - 1);
+        float dz[4][4], h[4][4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) load_dz<kLast>(row, 16 * b + 4 * kq, dH, H, ds, wl[b], dz[b], h[b]);
+        f32x4 acc[8];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int c = 0; c < 8; ++c)
+                    acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(dz[b][j], wv[b][j][c], acc[c], 0, 0, 0);
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const int rr = tile * 16 + kq * 4 + t;
+                if (rr < n) (c < 4 ? dX : G)[(size_t)rr * kH + (c & 3) * 16 + r16] = acc[c][t];
+            }
     }
 }
 
@@ -297,64 +449,73 @@ int grid_for_waves(int n)
 
 }  // namespace
 
+// Workgroups of four waves over 16-row tiles, at most two per CU (the weights
+// are loaded once per wave).
+static int tile_grid(int n)
+{
+    const int t = (n + 63) / 64;
+    return t < 512 ? t : 512;
+}
+
 void gnn_forward(const GnnArgs &g, const float *w, bool keep, float *scores, hipStream_t s)
 {
     const int n = g.n;
-    const int gw = grid_for_waves(n);
+    const int gw = grid_for_waves(n), ga = (n + 15) / 16 < 16384 ? (n + 15) / 16 : 16384;
     // layer 1
     hipLaunchKernelGGL(k_agg2, dim3(1024), dim3(256), 0, s, n, g.ptr, g.ind, g.a, g.H0, g.M1);
-    hipLaunchKernelGGL(k_dense1, dim3(gw), dim3(256), 0, s, n, (const float *)g.H0, (const float *)g.M1, w, g.Z[0],
-                       g.H[0]);
+    hipLaunchKernelGGL(k_dense1, dim3(gw), dim3(256), 0, s, n, (const float *)g.H0, (const float *)g.M1, w, g.H[0]);
     // layers 2, 3
-    const int gm = (((n + 15) / 16) + 3) / 4 < 4096 ? ((((n + 15) / 16) + 3) / 4 > 0 ? (((n + 15) / 16) + 3) / 4 : 1) : 4096;
     for (int l = 1; l < 3; ++l) {
         const float *Hin = g.H[keep ? l - 1 : (l - 1) & 1];
         float *Mout = g.M[keep ? l : 0];
-        float *Zout = g.Z[keep ? l : 0];
         float *Hout = g.H[keep ? l : (l & 1)];
-        hipLaunchKernelGGL(k_agg64, dim3(gw), dim3(256), 0, s, n, g.ptr, g.ind, g.a, Hin, Mout);
+        hipLaunchKernelGGL(k_agg64<false>, dim3(ga), dim3(256), 0, s, n, g.ptr, g.ind, g.a, Hin, Mout);
         const float *Ws = w + (l == 1 ? kGnnWs2 : kGnnWs3);
         const float *Wn = w + (l == 1 ? kGnnWn2 : kGnnWn3);
         const float *b = w + (l == 1 ? kGnnB2 : kGnnB3);
-        hipLaunchKernelGGL(k_dense_mfma, dim3(gm), dim3(256), 0, s, n, Hin, (const float *)Mout, Ws, Wn, b, Zout, Hout);
+        hipLaunchKernelGGL(k_dense_mfma, dim3(tile_grid(n)), dim3(256), 0, s, n, Hin, (const float *)Mout, Ws, Wn, b,
+                           Hout);
     }
     const float *H3 = g.H[keep ? 2 : 0];
     hipLaunchKernelGGL(k_score, dim3(gw), dim3(256), 0, s, n, H3, w, scores);
 }
 
+size_t gnn_partial_floats() { return (size_t)kGnnPartials * kWgLen; }
+
 void gnn_backward(const GnnArgs &g, const float *w, const float *ds, float *dw, hipStream_t s)
 {
     const int n = g.n;
-    const int gw = grid_for_waves(n);
-    const size_t total = (size_t)n * kH;
-    float *dH = g.dA;
-    float *dX = g.dB;
-    float *G = g.dC;
-    const int nb = g.nblocks;
-    const int rows = (n + nb - 1) / nb;
-    // output layer
-    hipLaunchKernelGGL(k_score_back, dim3(nb), dim3(256), 0, s, n, (const float *)g.H[2], w, ds, dH, g.part);
-    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(128), 0, s, (const float *)g.part, nb, kH + 1, dw + kGnnWo);
-    for (int l = 2; l >= 0; --l) {
-        hipLaunchKernelGGL(k_relu_back, dim3(2048), dim3(256), 0, s, total, (const float *)g.Z[l], dH);
-        if (l > 0) {
-            hipLaunchKernelGGL(k_wgrad<kH>, dim3(nb), dim3(256), 0, s, n, rows, (const float *)dH,
-                               (const float *)g.H[l - 1], (const float *)g.M[l], g.part);
-            const int len = 2 * kH * kH + kH;
-            const int off = l == 1 ? kGnnWs2 : kGnnWs3;   // Ws, Wn, b are contiguous per layer
-            hipLaunchKernelGGL(k_sum_partials, dim3(64), dim3(256), 0, s, (const float *)g.part, nb, len, dw + off);
-            const float *Ws = w + (l == 1 ? kGnnWs2 : kGnnWs3);
-            const float *Wn = w + (l == 1 ? kGnnWn2 : kGnnWn3);
-            hipLaunchKernelGGL(k_back_dense, dim3(gw), dim3(256), 0, s, n, (const float *)dH, Ws, Wn, dX, G);
-            hipLaunchKernelGGL(k_aggT64, dim3(gw), dim3(256), 0, s, n, g.ptr, g.ind, g.at, (const float *)G, dX);
-            float *t = dH; dH = dX; dX = t;    // dH_{l-1}
-        } else {
-            hipLaunchKernelGGL(k_wgrad<2>, dim3(nb), dim3(256), 0, s, n, rows, (const float *)dH, (const float *)g.H0,
-                               (const float *)g.M1, g.part);
-            const int len = 2 * kH * 2 + kH;
-            hipLaunchKernelGGL(k_sum_partials, dim3(4), dim3(256), 0, s, (const float *)g.part, nb, len, dw + kGnnWs1);
-        }
-    }
+    const int ga = (n + 15) / 16 < 16384 ? (n + 15) / 16 : 16384;
+    // rows per wave of the weight gradients: four waves a workgroup, at most
+    // kGnnPartials workgroups, at least one 8-row step a wave
+    int rows = (n + 4 * kGnnPartials - 1) / (4 * kGnnPartials);
+    rows = (rows + 7) / 8 * 8;
+    const int nb = (n + 4 * rows - 1) / (4 * rows);
+    auto sum = [&](int stride, int len, float *out) {
+        hipLaunchKernelGGL(k_sum_partials, dim3((len + 31) / 32), dim3(256), 0, s, (const float *)g.part, nb, stride, len,
+                           out);
+    };
+    float *dH = g.dA, *dX = g.dB, *G = g.dC;
+    // layer 3 with the output layer (its gradients follow the layer's in dw)
+    hipLaunchKernelGGL(k_wgrad64<true>, dim3(nb), dim3(256), 0, s, n, rows, (const float *)nullptr,
+                       (const float *)g.H[2], ds, w + kGnnWo, (const float *)g.H[1], (const float *)g.M[2], g.part);
+    sum(kWgLen, kWgLen, dw + kGnnWs3);
+    hipLaunchKernelGGL(k_back_dense<true>, dim3(tile_grid(n)), dim3(256), 0, s, n, (const float *)nullptr,
+                       (const float *)g.H[2], ds, w + kGnnWo, w + kGnnWs3, w + kGnnWn3, dH, G);
+    hipLaunchKernelGGL(k_agg64<true>, dim3(ga), dim3(256), 0, s, n, g.ptr, g.ind, g.at, (const float *)G, dH);
+    // layer 2
+    hipLaunchKernelGGL(k_wgrad64<false>, dim3(nb), dim3(256), 0, s, n, rows, (const float *)dH, (const float *)g.H[1],
+                       (const float *)nullptr, (const float *)nullptr, (const float *)g.H[0], (const float *)g.M[1],
+                       g.part);
+    sum(kWgLen, 2 * kH * kH + kH, dw + kGnnWs2);
+    hipLaunchKernelGGL(k_back_dense<false>, dim3(tile_grid(n)), dim3(256), 0, s, n, (const float *)dH,
+                       (const float *)g.H[1], (const float *)nullptr, (const float *)nullptr, w + kGnnWs2, w + kGnnWn2,
+                       dX, G);
+    hipLaunchKernelGGL(k_agg64<true>, dim3(ga), dim3(256), 0, s, n, g.ptr, g.ind, g.at, (const float *)G, dX);
+    // layer 1
+    hipLaunchKernelGGL(k_wgrad2, dim3(nb), dim3(256), 0, s, n, rows, (const float *)dX, (const float *)g.H[0],
+                       (const float *)g.H0, (const float *)g.M1, g.part);
+    sum(kWgLen2, kWgLen2, dw + kGnnWs1);
 }
 
 }  // namespace rc

@@ -366,13 +366,14 @@ struct GnnArgs {
     const float *a;               // w / wdeg(row)        (forward aggregation)
     const float *at;              // w / wdeg(neighbour)  (transposed aggregation)
     float *H0, *M1;               // n x 2
-    float *H[3], *M[3], *Z[3];    // n x 64 (index 0..2 = layers 1..3; M[0] unused)
+    float *H[3], *M[3];           // n x 64 (index 0..2 = layers 1..3; M[0] unused)
     float *dA, *dB, *dC;          // n x 64 backward scratch
-    float *part;                  // nblocks x (2*64*64 + 64)
-    int nblocks;
+    float *part;                  // gnn_partial_floats()
 };
+constexpr int kGnnPartials = 256;   // most workgroups of a weight gradient
+size_t gnn_partial_floats();
 // keep = true stores every layer (for the backward pass); otherwise layers
-// ping-pong through H[0..1], M[0], Z[0].
+// ping-pong through H[0..1] and M[0].
 void gnn_forward(const GnnArgs &g, const float *w, bool keep, float *scores, hipStream_t s);
 // dw = d(sum_v ds[v] s[v]) / dw, using the stored forward pass.
 void gnn_backward(const GnnArgs &g, const float *w, const float *ds, float *dw, hipStream_t s);

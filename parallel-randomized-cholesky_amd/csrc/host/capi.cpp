@@ -439,13 +439,12 @@ static int gnn_setup(rc_handle_t h, bool keep)
     for (int l = 0; l < nl; ++l) RC_HIP(h->g_H[l].ensure(n * kGnnHidden * sizeof(float) + 16));
     for (int l = 0; l < (keep ? 3 : 1); ++l) {
         RC_HIP(h->g_M[l].ensure(n * kGnnHidden * sizeof(float) + 16));
-        RC_HIP(h->g_Z[l].ensure(n * kGnnHidden * sizeof(float) + 16));
     }
     if (keep) {
         RC_HIP(h->g_dA.ensure(n * kGnnHidden * sizeof(float) + 16));
         RC_HIP(h->g_dB.ensure(n * kGnnHidden * sizeof(float) + 16));
         RC_HIP(h->g_dC.ensure(n * kGnnHidden * sizeof(float) + 16));
-        RC_HIP(h->g_part.ensure((size_t)256 * (2 * kGnnHidden * kGnnHidden + kGnnHidden) * sizeof(float)));
+        RC_HIP(h->g_part.ensure(gnn_partial_floats() * sizeof(float)));
         RC_HIP(h->g_dw.ensure((size_t)kGnnParams * sizeof(float)));
         RC_HIP(h->g_ds.ensure(n * sizeof(float) + 16));
     }
@@ -478,13 +477,11 @@ static GnnArgs gnn_args(rc_handle_t h)
     for (int l = 0; l < 3; ++l) {
         g.H[l] = h->g_H[l].as<float>();
         g.M[l] = h->g_M[l].as<float>();
-        g.Z[l] = h->g_Z[l].as<float>();
     }
     g.dA = h->g_dA.as<float>();
     g.dB = h->g_dB.as<float>();
     g.dC = h->g_dC.as<float>();
     g.part = h->g_part.as<float>();
-    g.nblocks = 256;
     return g;
 }
 
@@ -521,7 +518,6 @@ static int rc_gnn_gradient_impl(rc_handle_t h, const float *w, const float *dsco
     RC_HIP(hipMemcpyAsync(h->g_ds.p, dscores, (size_t)h->gnn_n * sizeof(float), hipMemcpyHostToDevice, s));
     GnnArgs g = gnn_args(h);
     gnn_forward(g, h->g_w.as<float>(), true, h->g_s.as<float>(), s);
-    RC_HIP(hipMemsetAsync(h->g_dw.p, 0, (size_t)kGnnParams * sizeof(float), s));
     gnn_backward(g, h->g_w.as<float>(), h->g_ds.as<float>(), h->g_dw.as<float>(), s);
     RC_HIP(hipGetLastError());
     RC_HIP(hipMemcpyAsync(dw, h->g_dw.p, (size_t)kGnnParams * sizeof(float), hipMemcpyDeviceToHost, s));

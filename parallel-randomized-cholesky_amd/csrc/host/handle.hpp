@@ -156,7 +156,7 @@ struct rc_handle_s {
     // ordering network: graph + activations of the loaded system
     bool gnn_ready = false, gnn_keep = false;
     int gnn_n = 0;
-    DevVec g_ptr, g_ind, g_a, g_at, g_H0, g_M1, g_H[3], g_M[3], g_Z[3], g_dA, g_dB, g_dC, g_part, g_w, g_dw, g_s, g_ds;
+    DevVec g_ptr, g_ind, g_a, g_at, g_H0, g_M1, g_H[3], g_M[3], g_dA, g_dB, g_dC, g_part, g_w, g_dw, g_s, g_ds;
 
     // fixed workspace of rc_solve_noalloc on this handle's device (resolved at rc_create)
     void *na_ws = nullptr;
