@@ -130,16 +130,19 @@ __global__ void k_lt_fill(AssembleArgs a, const int *lt_ptr, int *lt_ind, T *lt_
     }
 }
 
-__global__ void k_level_max(int ns, const int *level, unsigned long long *out)
+__global__ void __launch_bounds__(1024) k_level_max(int ns, const int *level, unsigned long long *out)
 {
+    __shared__ int red[1024 / kWave];
     int m = 0;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < ns; i += gridDim.x * blockDim.x)
         m = level[i] > m ? level[i] : m;
-    for (int off = 32; off > 0; off >>= 1) {
-        int o = __shfl_xor(m, off, kWave);
-        m = o > m ? o : m;
+    m = (int)wave_max(m);
+    if (lane_id() == 0) red[threadIdx.x / kWave] = m;
+    __syncthreads();
+    if (threadIdx.x < kWave) {
+        m = (int)wave_max(threadIdx.x < 1024 / kWave ? red[threadIdx.x] : 0);
+        if (threadIdx.x == 0) atomicMax(out, (unsigned long long)m);    // one a workgroup
     }
-    if (lane_id() == 0) atomicMax(out, (unsigned long long)m);
 }
 
 __global__ void k_iota(int *v, int n)
@@ -514,9 +517,10 @@ void launch_lt_fill(const AssembleArgs &a, const int *lt_ptr, int *lt_ind, T *lt
     hipLaunchKernelGGL(k_lt_fill<T>, dim3(2048), dim3(256), 0, s, a, lt_ptr, lt_ind, lt_val, diag_out);
 }
 
+static int reduce_grid(int n) { return n < 128 * 1024 ? (n + 1023) / 1024 : 128; }
 void launch_level_max(int ns, const int *level, unsigned long long *out, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_level_max, dim3(1024), dim3(256), 0, s, ns, level, out);
+    hipLaunchKernelGGL(k_level_max, dim3(reduce_grid(ns)), dim3(1024), 0, s, ns, level, out);
 }
 void launch_iota(int *v, int n, hipStream_t s) { hipLaunchKernelGGL(k_iota, dim3(2048), dim3(256), 0, s, v, n); }
 void launch_copy_keys(const int *src, uint32_t *dst, int n, hipStream_t s)

@@ -74,6 +74,11 @@ __device__ __forceinline__ int wave_sum_int(int v)
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
     return v;
 }
+__device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
+{
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+    return v;
+}
 __device__ __forceinline__ int64_t wave_max(int64_t v)
 {
     for (int off = 32; off > 0; off >>= 1) {

@@ -1114,55 +1114,52 @@ int factor_occupancy_blocks(int device)
 }
 
 // Statistics after the factor: nnz_off, fills, max degree, zero pivots
-// (over the first n-1 columns; the last column is a zero pivot by definition).
-__global__ void k_factor_stats(int n, const int *out_cnt, unsigned long long *ctr)
+// (over the first n-1 columns; the last column is a zero pivot by definition),
+// and the level of the last column (never eliminated): 1 + max level of the
+// columns whose factor column holds it (rows are sorted, so it is their last
+// entry).  One atomic per workgroup and word: with one per wave (4,096 of
+// them on each word) the two passes took 150 us whatever the size.
+constexpr int kStatBlock = 1024;
+__global__ void __launch_bounds__(kStatBlock) k_factor_stats(int n, const long long *out_start, const int *out_cnt,
+                                                             const int *out_row, int *level, unsigned long long *ctr)
 {
-    unsigned long long nnz = 0, fills = 0, zp = 0, mx = 0;
+    __shared__ unsigned long long red[5][kStatBlock / kWave];
+    unsigned long long v[5] = {0, 0, 0, 0, 0};       // nnz, fills, zero pivots, max degree, level + 1
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        unsigned long long d = (unsigned long long)out_cnt[i];
-        nnz += d;
-        fills += d > 0 ? d - 1 : 0;
-        zp += d == 0 ? 1 : 0;
-        mx = d > mx ? d : mx;
+        const unsigned long long d = (unsigned long long)out_cnt[i];
+        v[0] += d;
+        v[1] += d > 0 ? d - 1 : 0;
+        v[2] += d == 0 ? 1 : 0;
+        v[3] = d > v[3] ? d : v[3];
+        if (d > 0 && i < n - 1 && out_row[out_start[i] + (long long)d - 1] == n - 1) {
+            const unsigned long long l = (unsigned long long)level[i] + 1;
+            v[4] = l > v[4] ? l : v[4];
+        }
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        nnz += __shfl_xor(nnz, off, kWave);
-        fills += __shfl_xor(fills, off, kWave);
-        zp += __shfl_xor(zp, off, kWave);
-        unsigned long long o = __shfl_xor(mx, off, kWave);
-        mx = o > mx ? o : mx;
+    for (int q = 0; q < 5; ++q) {
+        v[q] = q < 3 ? (unsigned long long)wave_sum_u64(v[q]) : (unsigned long long)wave_max((int64_t)v[q]);
+        if (lane_id() == 0) red[q][threadIdx.x / kWave] = v[q];
     }
-    if (lane_id() == 0) {
-        atomicAdd(&ctr[kCtrNnzOff], nnz);
-        atomicAdd(&ctr[kCtrFills], fills);
-        atomicAdd(&ctr[kCtrZeroPivots], zp);
-        atomicMax(&ctr[kCtrMaxDeg], mx);
+    __syncthreads();
+    if (threadIdx.x >= kWave) return;
+    for (int q = 0; q < 5; ++q) {
+        const unsigned long long t = threadIdx.x < kStatBlock / kWave ? red[q][threadIdx.x] : 0;
+        v[q] = q < 3 ? wave_sum_u64(t) : (unsigned long long)wave_max((int64_t)t);
     }
-}
-
-// Level of the last column (never eliminated): 1 + max level of the columns
-// whose factor column holds it (rows are sorted, so it is their last entry).
-__global__ void k_last_level(int n, const long long *out_start, const int *out_cnt, const int *out_row,
-                             int *level)
-{
-    int m = -1;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n - 1; k += gridDim.x * blockDim.x) {
-        int c = out_cnt[k];
-        if (c > 0 && out_row[out_start[k] + c - 1] == n - 1) m = level[k] > m ? level[k] : m;
+    if (threadIdx.x == 0) {
+        atomicAdd(&ctr[kCtrNnzOff], v[0]);
+        atomicAdd(&ctr[kCtrFills], v[1]);
+        atomicAdd(&ctr[kCtrZeroPivots], v[2]);
+        atomicMax(&ctr[kCtrMaxDeg], v[3]);
+        if (v[4] > 0) atomicMax(&level[n - 1], (int)v[4]);
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        int o = __shfl_xor(m, off, kWave);
-        m = o > m ? o : m;
-    }
-    if (lane_id() == 0 && m >= 0) atomicMax(&level[n - 1], m + 1);
 }
 
 void launch_factor_finish(const FactorArgs &a, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_factor_stats, dim3(1024), dim3(256), 0, s, a.n, (const int *)a.out_cnt, a.ctr);
-    if (a.n > 1)
-        hipLaunchKernelGGL(k_last_level, dim3(1024), dim3(256), 0, s, a.n, (const long long *)a.out_start,
-                           (const int *)a.out_cnt, (const int *)a.out_row, a.level);
+    const int g = a.n < 128 * kStatBlock ? (a.n + kStatBlock - 1) / kStatBlock : 128;
+    hipLaunchKernelGGL(k_factor_stats, dim3(g), dim3(kStatBlock), 0, s, a.n, (const long long *)a.out_start,
+                       (const int *)a.out_cnt, (const int *)a.out_row, a.level, a.ctr);
 }
 
 }  // namespace rc

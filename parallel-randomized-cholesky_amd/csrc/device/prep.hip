@@ -127,23 +127,26 @@ __global__ void k_trim_fill(int n, const int *ptr, const int *ind, const double 
 // lower slice and dependency counts, one wave per column: rows are sorted,
 // so the strict-lower entries of column j are a suffix; dep[j] counts the
 // rows above j (the pattern is symmetric: the lower entries in row j)
+__device__ __forceinline__ int first_at_least(const int *ind, int b, int e, int r)
+{
+    while (b < e) {
+        const int mid = b + ((e - b) >> 1);
+        if (ind[mid] < r) b = mid + 1; else e = mid;
+    }
+    return b;
+}
+
+// Rows below and above the diagonal of every (sorted) column by bisection, one
+// thread per column: a wave per column read an appended ground column of 2.1 M
+// entries alone, 10.8 ms of the 128^3 SDDM preparation.
 __global__ void k_lower_count(int n, const int *ptr, const int *ind, int *cnt, int *dep)
 {
-    const int lane = threadIdx.x & 63;
-    const int nw = (gridDim.x * blockDim.x) >> 6;
-    for (int j = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; j < n; j += nw) {
-        int lo = 0, up = 0;
-        for (int p = ptr[j] + lane; p < ptr[j + 1]; p += 64) {
-            const int r = ind[p];
-            lo += r > j;
-            up += r < j;
-        }
-        lo = wave_sum_int(lo);
-        up = wave_sum_int(up);
-        if (lane == 0) {
-            cnt[j] = lo;
-            dep[j] = up;
-        }
+    for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
+        const int b = ptr[j], e = ptr[j + 1];
+        const int d = first_at_least(ind, b, e, j);
+        const int l = d < e && ind[d] == j ? d + 1 : d;
+        cnt[j] = e - l;
+        dep[j] = d - b;
     }
 }
 
