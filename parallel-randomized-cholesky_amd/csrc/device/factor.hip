@@ -15,7 +15,9 @@
 //     launch (one wave64 per column, grid-stride over the round's list), so
 //     the kernel boundary orders all communication -- no fences, no waits;
 //   * gather, duplicate merge, sorts and the prefix sum run in LDS (global
-//     per-wave scratch for columns above the LDS capacity);
+//     per-workgroup scratch for columns above the LDS capacity); columns of more
+//     than 128 entries, and of more than 64 where few are ready, are eliminated
+//     by eight waves;
 //   * the sampling draw is Philox4x32-10 keyed by (seed, i, column): with the
 //     canonical (row, weight) merge order and (weight, row) sampling order the
 //     factor is a pure function of (matrix, seed), independent of schedule;
@@ -38,8 +40,12 @@ namespace rc {
 namespace {
 
 constexpr int kLdsCap = 128;                                   // entries per wave in LDS (round kernel)
-static_assert(kLdsCap <= 2 * 64, "the round kernel sorts its columns in registers (two slots per lane)");
+static_assert(kLdsCap <= 2 * 64, "the round kernel sorts two entries per lane");
 constexpr int kBytesPerEntry = 16 + 8 + 8 + 4 + 4 + 4 + 4;  // s mw C mrow mmult minc jt
+// global scratch of a column above kBigCap entries: the column buffer, the
+// sorts' second entry array, and eight bytes per 64 entries (one an entry is
+// more than that) for the scan's block sums
+constexpr int kScratchBytesPerEntry = kBytesPerEntry + 16 + 1;
 constexpr long long kFillChunk = 2048;
 constexpr long long kOutChunk = 2048;
 
@@ -51,6 +57,24 @@ struct __attribute__((aligned(16))) SEnt {
     int pay;
     double w;
 };
+
+// A pointer of the argument block, known to be device memory: the block itself
+// is read from memory, and without this its pointers would be dereferenced with
+// flat accesses, which occupy the LDS queue as well.
+template <typename T>
+using Global = __attribute__((address_space(1))) T;
+template <typename T>
+__device__ __forceinline__ Global<T> *gp(T *p)
+{
+    return (Global<T> *)p;
+}
+// ... and as an operand of an atomic (global still, as the compiler sees where
+// it comes from)
+template <typename T>
+__device__ __forceinline__ T *at(Global<T> *p)
+{
+    return (T *)p;
+}
 
 struct ColBuf {
     SEnt *s;
@@ -78,412 +102,77 @@ __device__ __forceinline__ int next_pow2(int v)
     return p;
 }
 
-// Ascending sorting network (bitonic with a mirrored first comparator in
-// every merge stage); every comparator puts the minimum at the lower index, so
-// positions >= len behave as +infinity and need no padding.
-// kByRow: key (row, w); otherwise key (w, row); the payload travels along.
-// The comparators of a stage touch disjoint pairs, so each lane reads all of
-// its pairs of the stage (kNB = P / 128 of them, at most 8 at a time) before
-// it compares and writes any: one LDS round trip per stage instead of one per
-// 64 comparators.  kNB is a template argument so no slot is computed idly.
-template <bool kByRow>
-__device__ __forceinline__ bool key_less(int ra, double wa, int rb, double wb)
+// Orders the accesses of one wave's lanes among each other (they are executed in
+// order; this keeps the compiler from moving them).
+__device__ __forceinline__ void wave_fence()
 {
-    return kByRow ? (ra < rb || (ra == rb && wa < wb)) : (wa < wb || (wa == wb && ra < rb));
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+template <int kWaves>
+__device__ __forceinline__ void sync_waves()
+{
+    if constexpr (kWaves == 1) wave_fence();
+    else __syncthreads();
 }
 
-template <bool kByRow, int kNB>
-__device__ __forceinline__ void wave_sort_nb(SEnt *e, int len, int P)
+// The sorts place an entry by counting those before it, in the order (row, w) or
+// (w, row): entries are compared against one broadcast entry at a time, with
+// independent reads, where a network is a chain of shuffles (64 entries: 5.0 us
+// for the network's 21 stages).  Equal entries (unit weights) go by their
+// index.  A weight that is not a number counts as infinity, so that every place
+// is taken once whatever the weights.
+__device__ __forceinline__ double sort_key(double w) { return w != w ? __builtin_inf() : w; }
+template <bool kByRow>
+__device__ __forceinline__ bool ent_before(int xr, double xw, int vr, double vw, bool tie)
 {
-    const int lane = lane_id();
-    const int half = P >> 1;
-    for (int k = 2; k <= P; k <<= 1) {
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int t0 = 0; t0 < half; t0 += kNB * kWave) {
-                int ia[kNB], la[kNB];
-                SEnt ei[kNB], el[kNB];
-                bool act[kNB];
+    const bool lr = xr < vr, er = xr == vr, lw = xw < vw, ew = xw == vw;    // no branches
+    return kByRow ? lr | (er & (lw | (ew & tie))) : lw | (ew & (lr | (er & tie)));
+}
+
+constexpr int kCountBatch = 8;
+// For entry index i (key vr, vw): entries among e[j0..j1) that come before it.
+// Weights in e are sort keys.
+template <bool kByRow, int R>
+__device__ __forceinline__ void count_before(const SEnt *e, int j0, int j1, const int (&i)[R], const int (&vr)[R],
+                                             const double (&vw)[R], int (&c)[R])
+{
+    for (; j0 < j1; j0 += kCountBatch) {
+        SEnt x[kCountBatch];
 #pragma unroll
-                for (int b = 0; b < kNB; ++b) {
-                    const int t = t0 + b * kWave + lane;
-                    const int i = ((t & ~(j - 1)) << 1) | (t & (j - 1));
-                    const int l = (j == (k >> 1)) ? (i ^ (k - 1)) : (i + j);
-                    act[b] = l < len;                      // t < half always; l > i, so i < len as well
-                    ia[b] = i;
-                    la[b] = l;
-                    // read unconditionally (i, l < P <= the buffer's capacity),
-                    // so no branch sits between the reads of the slots
-                    ei[b] = e[i];
-                    el[b] = e[l];
-                }
+        for (int u = 0; u < kCountBatch; ++u) x[u] = e[min(j0 + u, j1 - 1)];
 #pragma unroll
-                for (int b = 0; b < kNB; ++b) {
-                    if (act[b] && key_less<kByRow>(el[b].row, el[b].w, ei[b].row, ei[b].w)) {
-                        e[ia[b]] = el[b];
-                        e[la[b]] = ei[b];
-                    }
-                }
-            }
-            __syncthreads();
-        }
+        for (int u = 0; u < kCountBatch; ++u)
+#pragma unroll
+            for (int s = 0; s < R; ++s)
+                c[s] += (j0 + u < j1) & ent_before<kByRow>(x[u].row, x[u].w, vr[s], vw[s], j0 + u < i[s]);
     }
 }
-// Networks of P >= 256 positions (shorter columns use the register sorts).
-template <bool kByRow>
+
+// Sorts e[0..len) by one wave, len <= 64 R, the payload travelling along.
+template <bool kByRow, int R>
 __device__ __forceinline__ void wave_sort(SEnt *e, int len)
 {
-    const int P = next_pow2(len);
-    if (P <= 256) wave_sort_nb<kByRow, 2>(e, len, 256);
-    else if (P <= 512) wave_sort_nb<kByRow, 4>(e, len, 512);
-    else wave_sort_nb<kByRow, 8>(e, len, P);
-}
-
-// The same ordering for len <= 64 R entries held in registers, entry i in
-// slot i / 64 of lane i % 64: a bitonic network whose comparator pairs are
-// lane pairs (shuffles) for distances below 64 and slot pairs inside a lane
-// above, with no LDS round trips between stages.  Positions >= len hold
-// +infinity keys.  Ties keep their values (the sorted output is unique: equal
-// keys carry equal payloads in both uses).
-template <bool kByRow, int R>
-__device__ __forceinline__ void lane_sort(SEnt *e, int len)
-{
     const int lane = lane_id();
-    const int P = next_pow2(len);
-    int r[R], y[R];
-    double x[R];
+    SEnt v[R];
+    int i[R], row[R], c[R];
+    double key[R];
 #pragma unroll
     for (int s = 0; s < R; ++s) {
-        const int i = s * kWave + lane;
-        SEnt v;
-        v.row = 0x7fffffff;
-        v.pay = 0;
-        v.w = __builtin_inf();
-        if (i < len) v = e[i];
-        r[s] = v.row;
-        x[s] = v.w;
-        y[s] = v.pay;
+        i[s] = s * kWave + lane;
+        v[s] = e[min(i[s], len - 1)];
+        row[s] = v[s].row;
+        key[s] = sort_key(v[s].w);
+        c[s] = 0;
+        if (v[s].w != v[s].w && i[s] < len) e[i[s]].w = key[s];
     }
-    for (int k = 2; k <= P; k <<= 1) {
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            if (j >= kWave) {
-                const int js = j / kWave;
+    wave_fence();
+    count_before<kByRow, R>(e, 0, len, i, row, key, c);
+    wave_fence();
 #pragma unroll
-                for (int s = 0; s < R; ++s) {
-                    const int t = s ^ js;
-                    if (t > s && t < R) {
-                        const bool asc = ((s * kWave + lane) & k) == 0;
-                        const bool swap = asc ? key_less<kByRow>(r[t], x[t], r[s], x[s])
-                                              : key_less<kByRow>(r[s], x[s], r[t], x[t]);
-                        if (swap) {
-                            const int tr = r[s]; r[s] = r[t]; r[t] = tr;
-                            const double tx = x[s]; x[s] = x[t]; x[t] = tx;
-                            const int ty = y[s]; y[s] = y[t]; y[t] = ty;
-                        }
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int s = 0; s < R; ++s) {
-                    const int ro = __shfl_xor(r[s], j, kWave);
-                    const double xo = __shfl_xor(x[s], j, kWave);
-                    const int yo = __shfl_xor(y[s], j, kWave);
-                    const bool asc = ((s * kWave + lane) & k) == 0;
-                    const bool keep_min = asc == ((lane & j) == 0);
-                    const bool take = keep_min ? key_less<kByRow>(ro, xo, r[s], x[s])
-                                               : key_less<kByRow>(r[s], x[s], ro, xo);
-                    if (take) { r[s] = ro; x[s] = xo; y[s] = yo; }
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int s = 0; s < R; ++s) {
-        const int i = s * kWave + lane;
-        if (i < len) {
-            SEnt v;
-            v.row = r[s];
-            v.pay = y[s];
-            v.w = x[s];
-            e[i] = v;
-        }
-    }
-    __syncthreads();
-}
-
-// kMaxR bounds the register slots (and so the kernel's register budget).  Both
-// kernels use 2: above 128 entries the LDS network measured faster than
-// 4 or 8 slots per lane.
-// kShort (the round kernel): the caller guarantees len <= kMaxR * 64 (longer
-// columns are deferred), so only the register networks are compiled in (the
-// LDS network's registers would lower the round kernel's occupancy).
-// Otherwise (the large-LDS kernels) only the LDS network is.
-template <bool kByRow, int kMaxR, bool kShort = false>
-__device__ __forceinline__ void column_sort(SEnt *e, int len)
-{
-    if constexpr (kShort) {
-        if (len <= kWave) lane_sort<kByRow, 1>(e, len);
-        else lane_sort<kByRow, kMaxR>(e, len);
-        return;
-    }
-    // the large-LDS kernels order columns of up to kRankMax entries by
-    // counting and come here for them only when a row run is longer than the
-    // in-register merge takes, so they need no register network (its code
-    // would only enlarge the kernels' instruction footprint)
-    wave_sort<kByRow>(e, len);
-}
-
-// ---- counting sorts for the kernels that run one wave per CU
-// A column of at most kRankMax entries is put in order by counting, for every
-// entry, the keys below its own: each lane compares its kRankSlots-or-fewer
-// keys with every key of the column (broadcast LDS reads, kRankBatch keys in
-// flight at a time) and then stores each entry at its count: one LDS round
-// trip per kRankBatch keys, where the network needs one per stage (21-36
-// stages).  The large-LDS kernels run one wave per CU, so the VALU is
-// theirs; the round kernel keeps its register networks (its six waves per
-// SIMD share the VALU).  Above two keys per lane the comparisons cost more
-// than the network's round trips (measured: 129-256 entries 11.3 -> 13.5 us
-// for the row order, 9.7 -> 12.9 us for the value order).
-constexpr int kRankMax = 128;
-constexpr int kRankSlots = kRankMax / kWave;
-static_assert(kRankSlots == 2, "the dispatchers take one or two keys per lane");
-constexpr int kRun = 8;    // duplicates of one row merged in registers; a longer run uses the network
-
-// ascending 8-input sorting network (19 comparators in 6 layers)
-__device__ __forceinline__ void sort8(double *v)
-{
-    auto cx = [&](int x, int y) {
-        const double lo = fmin(v[x], v[y]);
-        const double hi = fmax(v[x], v[y]);
-        v[x] = lo;
-        v[y] = hi;
-    };
-    cx(0, 2); cx(1, 3); cx(4, 6); cx(5, 7);
-    cx(0, 4); cx(1, 5); cx(2, 6); cx(3, 7);
-    cx(0, 1); cx(2, 3); cx(4, 5); cx(6, 7);
-    cx(2, 4); cx(3, 5);
-    cx(1, 4); cx(3, 6);
-    cx(1, 2); cx(3, 4); cx(5, 6);
-}
-
-// Entries [0, m) of b.s reordered by (row, gathered index): the
-// key (row << 32 | index) is unique, so the counts are the positions.  The
-// keys are staged in b.C (unused until the scan), padded with +infinity to a
-// multiple of kRankBatch; every batch of keys is read before any is compared,
-// so a batch costs one LDS round trip.
-constexpr int kRankBatch = 16;
-__device__ __forceinline__ int rank_pad(int m) { return (m + kRankBatch - 1) & ~(kRankBatch - 1); }
-
-template <int R>
-__device__ __forceinline__ void rank_by_row(const ColBuf &b, int m)
-{
-    const int lane = lane_id();
-    unsigned long long *key = reinterpret_cast<unsigned long long *>(b.C);
-    int r[R], mu[R], rk[R];
-    double w[R];
-    unsigned long long k[R];
-#pragma unroll
-    for (int s = 0; s < R; ++s) {
-        const int i = s * kWave + lane;
-        const bool in = i < m;
-        SEnt v;
-        v.row = 0;
-        v.pay = 0;
-        v.w = 0.0;
-        if (in) v = b.s[i];
-        r[s] = v.row;
-        w[s] = v.w;
-        mu[s] = v.pay;
-        k[s] = in ? (((unsigned long long)(unsigned int)r[s] << 32) | (unsigned int)i) : ~0ull;
-        if (in) key[i] = k[s];
-        rk[s] = 0;
-    }
-    const int mp = rank_pad(m);
-    if (m + lane < mp) key[m + lane] = ~0ull;
-    __syncthreads();
-    const ulonglong2 *kp = reinterpret_cast<const ulonglong2 *>(key);
-    for (int o = 0; o < mp; o += kRankBatch) {
-        ulonglong2 kk[kRankBatch / 2];
-#pragma unroll
-        for (int q = 0; q < kRankBatch / 2; ++q) kk[q] = kp[o / 2 + q];
-#pragma unroll
-        for (int q = 0; q < kRankBatch / 2; ++q) {
-#pragma unroll
-            for (int s = 0; s < R; ++s) rk[s] += (kk[q].x < k[s] ? 1 : 0) + (kk[q].y < k[s] ? 1 : 0);
-        }
-    }
-    __syncthreads();   // every entry is in registers: the arrays are rewritten in place
-#pragma unroll
-    for (int s = 0; s < R; ++s) {
-        if (s * kWave + lane < m) {
-            SEnt v;
-            v.row = r[s];
-            v.pay = mu[s];
-            v.w = w[s];
-            b.s[rk[s]] = v;
-        }
-    }
-    __syncthreads();
-}
-
-// Step 2 by counting: entries ordered by (row, index), then every run of one
-// row (at most kRun entries) is put in ascending weight in registers and
-// summed left to right -- the sums of the (row, weight) sort and merge, bit
-// for bit (equal weights are interchangeable).  Returns the merged count, or
-// -1 if some run is longer than kRun (the caller then sorts by network).
-__device__ __forceinline__ int rank_merge(const ColBuf &b, int m_in)
-{
-    const int lane = lane_id();
-    const int m = __builtin_amdgcn_readfirstlane(m_in);
-    const int R = (m + kWave - 1) / kWave;
-    if (R <= 1) rank_by_row<1>(b, m);
-    else rank_by_row<kRankSlots>(b, m);
-    int d = 0;
-    bool over = false;
-    for (int base_i = 0; base_i < m; base_i += kWave) {
-        const int i = base_i + lane;
-        bool head = false;
-        int rr = 0, ms = 0;
-        double ws = 0.0;
-        if (i < m) {
-            rr = b.s[i].row;
-            head = (i == 0) || (b.s[i - 1].row != rr);
-        }
-        if (head) {
-            // the run is [i, i + g): rows are in order; reads past m stay
-            // inside the buffer (m + kRun <= its capacity) and are masked
-            double v[kRun];
-            int g = 0;
-#pragma unroll
-            for (int t = 0; t < kRun; ++t) {
-                const int e = i + t;
-                const SEnt x = b.s[e];
-                const bool in = e < m && x.row == rr;
-                v[t] = in ? x.w : __builtin_inf();
-                ms += in ? x.pay : 0;
-                g += in ? 1 : 0;
-            }
-            over = over || (i + kRun < m && b.s[i + kRun].row == rr);
-            sort8(v);
-            ws = v[0];
-#pragma unroll
-            for (int t = 1; t < kRun; ++t)
-                if (t < g) ws += v[t];
-        }
-        const uint64_t mask = ballot(head);
-        if (head) {
-            const int pos = d + lanes_below(mask);
-            b.mrow[pos] = rr;
-            b.mw[pos] = ws;
-            b.mmult[pos] = ms;
-            b.minc[pos] = 0;
-        }
-        d += __popcll(mask);
-    }
-    const bool any_over = ballot(over) != 0ull;
-    __syncthreads();
-    return any_over ? -1 : d;
-}
-
-// Step 3's order by counting: merged entries [0, d) by (w, row) (rows are
-// distinct, so the order is strict), written to b.s (payload = merged
-// index).  mw / mrow must be padded with +infinity / INT_MAX up to
-// rank_pad(d).
-template <int R>
-__device__ __forceinline__ void rank_by_value(const ColBuf &b, int d)
-{
-    const int lane = lane_id();
-    int r[R], rk[R];
-    double w[R];
-#pragma unroll
-    for (int s = 0; s < R; ++s) {
-        const int i = s * kWave + lane;
-        r[s] = i < d ? b.mrow[i] : 0x7fffffff;
-        w[s] = i < d ? b.mw[i] : __builtin_inf();
-        rk[s] = 0;
-    }
-    const int dp = rank_pad(d);
-    const double2 *wp = reinterpret_cast<const double2 *>(b.mw);
-    const int2 *rp = reinterpret_cast<const int2 *>(b.mrow);
-    for (int o = 0; o < dp; o += kRankBatch) {
-        double2 wo[kRankBatch / 2];
-        int2 ro[kRankBatch / 2];
-#pragma unroll
-        for (int q = 0; q < kRankBatch / 2; ++q) {
-            wo[q] = wp[o / 2 + q];
-            ro[q] = rp[o / 2 + q];
-        }
-#pragma unroll
-        for (int q = 0; q < kRankBatch / 2; ++q) {
-#pragma unroll
-            for (int s = 0; s < R; ++s) {
-                rk[s] += (wo[q].x < w[s] || (wo[q].x == w[s] && ro[q].x < r[s])) ? 1 : 0;
-                rk[s] += (wo[q].y < w[s] || (wo[q].y == w[s] && ro[q].y < r[s])) ? 1 : 0;
-            }
-        }
-    }
-#pragma unroll
-    for (int s = 0; s < R; ++s) {
-        const int i = s * kWave + lane;
-        if (i < d) {
-            SEnt v;
-            v.row = r[s];
-            v.pay = i;
-            v.w = w[s];
-            b.s[rk[s]] = v;
-        }
-    }
-    __syncthreads();
-}
-
-// Step 2 by the sorting networks: (row, w) order, then each run of one row
-// summed left to right (ascending weight).  Returns the merged count.
-template <int kMaxR, bool kShort>
-__device__ __forceinline__ int sort_merge(const ColBuf &b, int m)
-{
-    const int lane = lane_id();
-    column_sort<true, kMaxR, kShort>(b.s, m);
-    int d = 0;
-    for (int base_i = 0; base_i < m; base_i += kWave) {
-        int i = base_i + lane;
-        bool head = false;
-        int r = 0, ms = 0;
-        double ws = 0.0;
-        if (i < m) {
-            r = b.s[i].row;
-            head = (i == 0) || (b.s[i - 1].row != r);
-            if (head) {
-                // the run [i, i + g) summed left to right, kRun records per
-                // LDS round trip (records past m are masked)
-                ws = b.s[i].w;
-                ms = b.s[i].pay;
-                bool more = true;
-                for (int t0 = i + 1; more; t0 += kRun) {
-                    SEnt x[kRun];
-#pragma unroll
-                    for (int u = 0; u < kRun; ++u) x[u] = b.s[t0 + u < m ? t0 + u : m - 1];
-#pragma unroll
-                    for (int u = 0; u < kRun; ++u) {
-                        more = more && t0 + u < m && x[u].row == r;
-                        if (more) {
-                            ws += x[u].w;
-                            ms += x[u].pay;
-                        }
-                    }
-                }
-            }
-        }
-        uint64_t mask = ballot(head);
-        if (head) {
-            int pos = d + lanes_below(mask);
-            b.mrow[pos] = r;
-            b.mw[pos] = ws;
-            b.mmult[pos] = ms;
-            b.minc[pos] = 0;
-        }
-        d += __popcll(mask);
-    }
-    __syncthreads();
-    return d;
+    for (int s = 0; s < R; ++s)
+        if (i[s] < len) e[c[s]] = v[s];
+    wave_fence();
 }
 
 __device__ __forceinline__ void raise_status(unsigned long long *ctr, unsigned long long bits)
@@ -553,7 +242,7 @@ __device__ __forceinline__ void list_append(const FactorArgs &a, unsigned int *s
     const unsigned int cap = (unsigned int)a.seg_cap;
     const int seg = (int)(blockIdx.x % kListSegs);
     unsigned int base = 0;
-    if (lane_id() == 0) base = atomicAdd(&set[seg], cnt);
+    if (lane_id() == 0) base = atomicAdd(at(gp(set) + seg), cnt);
     base = bcast(base, 0);
     const unsigned int pos = base + (unsigned int)lanes_below(mask);
     if (base + cnt > cap) {
@@ -561,29 +250,51 @@ __device__ __forceinline__ void list_append(const FactorArgs &a, unsigned int *s
         unsigned int ob = 0;
         if (lane_id() == 0) ob = atomicAdd(&set[kListSegs], base + cnt - lo);
         ob = bcast(ob, 0);
-        if (ready && pos >= cap) list[(size_t)kListSegs * cap + ob + (pos - lo)] = value;
+        if (ready && pos >= cap) gp(list)[(size_t)kListSegs * cap + ob + (pos - lo)] = value;
     }
-    if (ready && pos < cap) list[(size_t)seg * cap + pos] = value;
+    if (ready && pos < cap) gp(list)[(size_t)seg * cap + pos] = value;
 }
 
-// Gathers column k's strict-lower entries and its pending fills (kFillLists
-// linked lists, walked in lockstep, one lane per list; f = this lane's list
-// head) into b, writing the first `cap` entries; returns the total count, or
-// with kStopOverCap any count above `cap` as soon as one is reached (the
-// column is then handed on without walking the rest of its lists).
-// The order of the gathered entries does not matter: the (row, weight) sort
-// makes it canonical.
-template <bool kStopOverCap>
-__device__ __forceinline__ int gather_column(const FactorArgs &a, int lo0, int norig, int f, const ColBuf &b, int cap)
+// A fill record through agent-scope accesses (two words of 8 bytes).
+__device__ __forceinline__ FillRec load_record(const FillRec *p)
 {
-    const int lane = lane_id();
-    for (int t = lane; t < norig && t < cap; t += kWave) {
+    const unsigned long long *q = reinterpret_cast<const unsigned long long *>(p);
+    const unsigned long long rn = ld_relaxed(q), w = ld_relaxed(q + 1);
+    FillRec r;
+    r.row = (int)(unsigned int)rn;
+    r.next = (int)(unsigned int)(rn >> 32);
+    r.w = __longlong_as_double((long long)w);
+    return r;
+}
+__device__ __forceinline__ void store_record(FillRec *p, const FillRec &r)
+{
+    unsigned long long *q = reinterpret_cast<unsigned long long *>(p);
+    st_relaxed(q, ((unsigned long long)(unsigned int)r.next << 32) | (unsigned int)r.row);
+    st_relaxed(q + 1, (unsigned long long)__double_as_longlong(r.w));
+}
+
+// Gathers column k: its strict-lower entries ...
+__device__ __forceinline__ void gather_original(const FactorArgs &a, int lo0, int norig, const ColBuf &b, int cap, int t,
+                                                int nt)
+{
+    for (; t < norig && t < cap; t += nt) {
         SEnt v;
-        v.row = a.lo_row[lo0 + t];
+        v.row = gp(a.lo_row)[lo0 + t];
         v.pay = 1;
-        v.w = a.lo_w[lo0 + t];
+        v.w = gp(a.lo_w)[lo0 + t];
         b.s[t] = v;
     }
+}
+// ... and its pending fills (kFillLists linked lists, walked in lockstep by one
+// wave, one lane per list; f = this lane's list head), writing the first `cap`
+// entries; returns the total count, or with kStopOverCap any count above `cap`
+// as soon as one is reached (the column is then handed on without walking the
+// rest of its lists).  kCoherent (queue-driven kernel): records written by
+// running waves of the same launch are read with agent-scope loads.  The order
+// of the gathered entries does not matter: the (row, weight) sort makes it canonical.
+template <bool kStopOverCap, bool kCoherent>
+__device__ __forceinline__ int gather_fills(const FactorArgs &a, int norig, int f, const ColBuf &b, int cap)
+{
     int t = norig;
     while (true) {
         if (kStopOverCap && t > cap) break;
@@ -591,7 +302,7 @@ __device__ __forceinline__ int gather_column(const FactorArgs &a, int lo0, int n
         const uint64_t mask = ballot(act);
         if (!mask) break;
         if (act) {
-            const FillRec rec = a.pool[f];
+            const FillRec rec = kCoherent ? load_record(at(gp(a.pool) + f)) : *at(gp(a.pool) + f);
             const int pos = t + lanes_below(mask);
             if (pos < cap) {
                 SEnt v;
@@ -604,166 +315,412 @@ __device__ __forceinline__ int gather_column(const FactorArgs &a, int lo0, int n
         }
         t += __popcll(mask);
     }
-    __syncthreads();
     return t;
 }
 
-// Steps 2-5 of a column whose m >= 1 entries are gathered in b.  Inlined at
-// every call so that b's accesses compile to LDS or global instructions (a
-// generic pointer would make each LDS access wait for all memory traffic).
-template <int kMaxR, bool kAsync, bool kShort = false>
-__device__ __forceinline__ bool process_column(const FactorArgs &a, int k, int round, const ColBuf &b, int m,
-                                               Cursor &fcur, Cursor &ocur, int *next, unsigned int *next_set)
+// A run of one row in the (row, weight) order starting at entry i: summed left
+// to right (ascending weight), kRun records per LDS round trip.
+constexpr int kRun = 8;
+struct RowRun {
+    bool head;
+    int row, mult;
+    double w;
+};
+__device__ __forceinline__ RowRun row_run(const SEnt *s, int i, int m)
+{
+    RowRun r;
+    const SEnt first = s[i];
+    r.row = first.row;
+    r.head = i == 0 || s[i - 1].row != first.row;
+    r.mult = first.pay;
+    r.w = first.w;
+    if (r.head) {
+        bool more = true;
+        for (int t0 = i + 1; more; t0 += kRun) {
+            SEnt x[kRun];
+#pragma unroll
+            for (int u = 0; u < kRun; ++u) x[u] = s[t0 + u < m ? t0 + u : m - 1];
+#pragma unroll
+            for (int u = 0; u < kRun; ++u) {
+                more = more && t0 + u < m && x[u].row == r.row;
+                if (more) {
+                    r.w += x[u].w;
+                    r.mult += x[u].pay;
+                }
+            }
+        }
+    }
+    return r;
+}
+__device__ __forceinline__ void put_merged(const ColBuf &b, int pos, const RowRun &r)
+{
+    b.mrow[pos] = r.row;
+    b.mw[pos] = r.w;
+    b.mmult[pos] = r.mult;
+    b.minc[pos] = 0;
+}
+__device__ __forceinline__ SEnt merged_entry(const ColBuf &b, int i)
+{
+    SEnt v;
+    v.row = b.mrow[i];
+    v.pay = i;
+    v.w = b.mw[i];
+    return v;
+}
+
+// Doubling scan of 64 values, one per lane (each step from the previous step's
+// values).
+__device__ __forceinline__ double block_scan64(double x)
 {
     const int lane = lane_id();
+    for (int off = 1; off < kWave; off <<= 1) {
+        const double o = __shfl_up(x, off, kWave);
+        if (lane >= off) x = x + o;
+    }
+    return x;
+}
+
+// Partner j of fill i and the new dependency of the larger row (:598-631; gpu
+// auxilliary.hpp:543-592).
+__device__ __forceinline__ void sample_partner(const FactorArgs &a, int k, const ColBuf &b, int i, int d, double S)
+{
+    const double u = sample_uniform(a.seed, (uint32_t)i, (uint32_t)k);
+    const double Ci = b.C[i];
+    const double rest = S - Ci;
+    const double tgt = u * rest;
+    int lo = i + 1, hi = d - 1;
+    while (lo < hi) {
+        const int mid = lo + ((hi - lo) >> 1);
+        if (b.C[mid] - Ci < tgt) lo = mid + 1; else hi = mid;
+    }
+    b.jt[i] = lo;
+    const SEnt ei = b.s[i], el = b.s[lo];
+    atomicAdd(&b.minc[ei.row > el.row ? ei.pay : el.pay], 1);   // the larger row gains a dependency
+}
+
+// Pushes fill e as record rec onto its column's lists; returns the old head.
+__device__ __forceinline__ int push_head(const FactorArgs &a, const ColBuf &b, int e, int rec)
+{
+    const int ri = b.s[e].row, rj = b.s[b.jt[e]].row;
+    const int c = ri > rj ? rj : ri;
+    return atomicExch(at(&gp(a.head)[(size_t)c * kFillLists + (rec & (kFillLists - 1))]), rec);
+}
+__device__ __forceinline__ FillRec fill_record(const ColBuf &b, int e, double S, int next)
+{
+    const SEnt se = b.s[e];
+    const int ri = se.row, rj = b.s[b.jt[e]].row;
+    FillRec fr;
+    fr.row = ri > rj ? ri : rj;
+    fr.next = next;
+    fr.w = (se.w * (S - b.C[e])) / S;
+    return fr;
+}
+
+// ---- columns by a whole workgroup -------------------------------------------
+// The large-LDS kernels (deferred columns, narrow rounds, the queue-driven
+// rest) run one workgroup per CU, and their time is the latency of one column
+// after the other.  The first wave takes the columns and eliminates those of at
+// most kWave entries by itself, without a barrier; for a larger one all kWgWaves
+// waves work together.  One wave with sorting networks took 14 us for up to 64
+// entries, 30 us for 129-256 and 45 us for 257-512, two thirds of it sorting;
+// the queue-driven rest of a 192^3 grid (learned order) took 26 ms that way and
+// takes 15.7 ms, its whole factorization 58.5 and 47.4 ms (101 x 83 x 89: 18.9
+// and 14.2 ms; 64^2: 0.76 and 0.70 ms).
+constexpr int kWgWaves = 8;
+constexpr int kWgThreads = kWgWaves * kWave;
+
+struct WgShared {
+    int k;                             // the large column (< 0: the end)
+    int m;                             // its gathered entries
+    int round;                         // its level
+    int ok;                            // pools not exhausted
+    int cnt[kWgWaves];                 // merged rows per wave
+    long long fbase, obase;            // its pool entries
+    double tot[kBigCap / kWave];       // block sums of the scan
+};
+
+// Sorts e[0..m) by the workgroup with tmp[0..m) as the second array; returns
+// the array that holds the result.  Up to kCountMax entries, every wave counts
+// over its share of them and the shares are added.  Above, a wave sorts
+// 64-entry runs; within groups of kGroup runs an entry's place is then its place
+// in its run plus the number of smaller entries in every other run (bisections,
+// kPar at a time: one pass where pairwise merges take three), and groups are
+// merged in pairs.  The second weight sort has distinct rows and the runs are
+// compared in index order, so equal entries keep their order throughout.
+constexpr int kCountMax = 2 * kWave;
+template <bool kByRow>
+__device__ __forceinline__ SEnt *wg_sort(SEnt *e, SEnt *tmp, int m)
+{
+    constexpr int kPar = 4, kGroup = 8;
+    const int lane = lane_id(), w = threadIdx.x / kWave;
+    if (m <= kCountMax) {
+        const int parts = m <= kWave ? kWgWaves : kWgWaves / 2;
+        const int share = (m + parts - 1) / parts;
+        const int part = w % parts;
+        const int i[1] = {w / parts * kWave + lane};
+        const SEnt v = e[min(i[0], m - 1)];
+        const int row[1] = {v.row};
+        const double key[1] = {sort_key(v.w)};
+        int c[1] = {0};
+        int *cnt = reinterpret_cast<int *>(tmp);          // per wave and lane
+        __syncthreads();
+        if (v.w != v.w && part == 0 && i[0] < m) e[i[0]].w = key[0];
+        __syncthreads();
+        count_before<kByRow, 1>(e, part * share, min(part * share + share, m), i, row, key, c);
+        cnt[w * kWave + lane] = c[0];
+        __syncthreads();
+        if (part == 0 && i[0] < m) {
+            int rank = 0;
+            for (int p = 0; p < parts; ++p) rank += cnt[(w + p) * kWave + lane];
+            e[rank] = v;
+        }
+        __syncthreads();
+        return e;
+    }
+    const int nr = (m + kWave - 1) / kWave;
+    for (int r = w; r < nr; r += kWgWaves) wave_sort<kByRow, 1>(e + r * kWave, min(m - r * kWave, kWave));
+    __syncthreads();
+    for (int r = w; r < nr; r += kWgWaves) {
+        const int i = r * kWave + lane;
+        if (i < m) {
+            const SEnt v = e[i];
+            const double key = sort_key(v.w);
+            const int g0 = r / kGroup * kGroup, g1 = min(g0 + kGroup, nr);
+            int rank = g0 * kWave + lane;
+            for (int q0 = g0; q0 < g1; q0 += kPar) {
+                int lo[kPar], hi[kPar];
+#pragma unroll
+                for (int u = 0; u < kPar; ++u) {
+                    const int q = q0 + u;
+                    lo[u] = 0;
+                    hi[u] = q < g1 && q != r ? min(m - q * kWave, kWave) : 0;
+                }
+                for (int step = 0; step < 7; ++step) {    // 65 possible counts
+                    SEnt x[kPar];
+                    int mid[kPar];
+#pragma unroll
+                    for (int u = 0; u < kPar; ++u) {
+                        mid[u] = (lo[u] + hi[u]) >> 1;
+                        const int at = (q0 + u) * kWave + mid[u];
+                        x[u] = e[at < m ? at : 0];
+                    }
+#pragma unroll
+                    for (int u = 0; u < kPar; ++u)
+                        if (lo[u] < hi[u]) {
+                            const bool before = ent_before<kByRow>(x[u].row, sort_key(x[u].w), v.row, key, q0 + u < r);
+                            lo[u] = before ? mid[u] + 1 : lo[u];
+                            hi[u] = before ? hi[u] : mid[u];
+                        }
+                }
+#pragma unroll
+                for (int u = 0; u < kPar; ++u) rank += lo[u];
+            }
+            tmp[rank] = v;
+        }
+    }
+    __syncthreads();
+    SEnt *src = tmp, *dst = e;
+    for (int len = kGroup * kWave; len < m; len *= 2) {
+        for (int base = 0; base < m; base += kWgThreads) {
+            const int i = base + (int)threadIdx.x;
+            if (i >= m) continue;
+            const SEnt v = src[i];
+            const double key = sort_key(v.w);
+            const int block = i / len * len;
+            const bool second = (i / len) & 1;
+            const int p0 = second ? block - len : block + len;   // the partner's first entry
+            int lo = 0, hi = max(0, min(m - p0, len));
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                const SEnt x = src[p0 + mid];
+                if (ent_before<kByRow>(x.row, sort_key(x.w), v.row, key, second)) lo = mid + 1;
+                else hi = mid;
+            }
+            dst[i - block + (second ? p0 : block) + lo] = v;
+        }
+        __syncthreads();
+        SEnt *s = src;
+        src = dst;
+        dst = s;
+    }
+    return src;
+}
+
+// Steps 2-5 of a column whose m >= 1 entries are gathered in b, by kWaves waves;
+// one wave: m <= 64 R.  tmp (m entries) and tot (a double per 64 entries): only
+// for more than one wave.  The cursors are the first wave's.  Returns false if
+// the pools are exhausted (status set).
+template <bool kAsync, int kWaves, int R>
+__device__ __forceinline__ bool process_column(const FactorArgs &a, WgShared *sh, int k, int round, const ColBuf &b,
+                                               SEnt *tmp, double *tot, int m, Cursor &fcur, Cursor &ocur, int *next,
+                                               unsigned int *next_set)
+{
+    constexpr int kT = kWaves * kWave;
+    const int lane = lane_id(), w = kWaves == 1 ? 0 : threadIdx.x / kWave;
+    const int t = w * kWave + lane;
     const int last = a.n - 1;
     // ---- 2. sort by (row, w); merge duplicates left to right (:520-560)
-    int d = -1;
-    if constexpr (!kShort) {
-        if (m <= kRankMax) d = rank_merge(b, m);
+    const SEnt *rs = b.s;
+    if constexpr (kWaves > 1) {
+        rs = wg_sort<true>(b.s, tmp, m);
+    } else {
+        if (R == 1 || m <= kWave) wave_sort<true, 1>(b.s, m);
+        else wave_sort<true, R>(b.s, m);
     }
-    if (d < 0) d = sort_merge<kMaxR, kShort>(b, m);
+    int d = 0;
+    for (int base = 0; base < m; base += kT) {
+        const int i = base + t;
+        RowRun run;
+        run.head = false;
+        if (i < m) run = row_run(rs, i, m);
+        const uint64_t mask = ballot(run.head);
+        int off = d, all = __popcll(mask);
+        if constexpr (kWaves > 1) {
+            if (lane == 0) sh->cnt[w] = all;
+            __syncthreads();
+            all = 0;
+            for (int q = 0; q < kWaves; ++q) {
+                const int c = sh->cnt[q];
+                off += q < w ? c : 0;
+                all += c;
+            }
+        }
+        if (run.head) put_merged(b, off + lanes_below(mask), run);
+        d += all;
+        sync_waves<kWaves>();
+    }
 
     // ---- 3. sort merged entries by (w, row), carrying the merged index;
     //         forward cumulative sums (:573-593)
-    bool ranked = false;
-    if constexpr (!kShort) {
-        if (d <= kRankMax) {
-            d = __builtin_amdgcn_readfirstlane(d);
-            if (d + lane < rank_pad(d)) {
-                b.mw[d + lane] = __builtin_inf();
-                b.mrow[d + lane] = 0x7fffffff;
-            }
+    for (int i = t; i < d; i += kT) b.s[i] = merged_entry(b, i);
+    sync_waves<kWaves>();
+    if constexpr (kWaves > 1) {
+        const SEnt *vs = wg_sort<false>(b.s, tmp, d);
+        if (vs != b.s) {
+            for (int i = t; i < d; i += kT) b.s[i] = vs[i];
             __syncthreads();
-            const int R = (d + kWave - 1) / kWave;
-            if (R <= 1) rank_by_value<1>(b, d);
-            else rank_by_value<kRankSlots>(b, d);
-            ranked = true;
         }
-    }
-    if (!ranked) {
-        for (int t = lane; t < d; t += kWave) {
-            SEnt v;
-            v.row = b.mrow[t];
-            v.pay = t;
-            v.w = b.mw[t];
-            b.s[t] = v;
-        }
-        __syncthreads();
-        column_sort<false, kMaxR, kShort>(b.s, d);
+    } else {
+        if (R == 1 || d <= kWave) wave_sort<false, 1>(b.s, d);
+        else wave_sort<false, R>(b.s, d);
     }
     // canonical blocked scan (shared with the oracle): per 64-entry block the
     // doubling scan x_i += x_{i-off}, off = 1..32, then the previous block's
     // last sum is added
-    {
-        double carry = 0.0;
-        for (int base_i = 0; base_i < d; base_i += kWave) {
-            const int i = base_i + lane;
-            double x = i < d ? b.s[i].w : 0.0;
-            for (int off = 1; off < kWave; off <<= 1) {
-                const double o = __shfl_up(x, off, kWave);
-                if (lane >= off) x = x + o;
+    if constexpr (kWaves > 1) {
+        // the blocks by all waves, the sums before each by one thread
+        for (int q = w; q * kWave < d; q += kWaves) {
+            const int i = q * kWave + lane;
+            const double x = block_scan64(i < d ? b.s[i].w : 0.0);
+            if (i < d) b.C[i] = x;
+            if (lane == kWave - 1) tot[q] = x;
+        }
+        __syncthreads();
+        if (d > kWave) {
+            if (t == 0) {
+                double carry = tot[0];
+                for (int q = 1; q * kWave < d; ++q) {
+                    const double x = tot[q];
+                    tot[q] = carry;
+                    carry = carry + x;
+                }
             }
-            const double c = base_i == 0 ? x : carry + x;
+            __syncthreads();
+            for (int i = kWave + t; i < d; i += kT) b.C[i] = tot[i / kWave] + b.C[i];
+            __syncthreads();
+        }
+    } else {
+        double carry = 0.0;
+        for (int base = 0; base < d; base += kWave) {
+            const int i = base + lane;
+            const double x = block_scan64(i < d ? b.s[i].w : 0.0);
+            const double c = base == 0 ? x : carry + x;
             if (i < d) b.C[i] = c;
             carry = __shfl(c, kWave - 1, kWave);
         }
+        wave_fence();
     }
-    __syncthreads();
     const double S = b.C[d - 1];
 
-    // ---- 4. sampled partners (:598-631; gpu auxilliary.hpp:543-592):
-    //         partner j of every fill i and the new dependencies per neighbour
+    // ---- 4. sampled partners
     const int nfill_out = d - 1;
-    for (int i = lane; i < nfill_out; i += kWave) {
-        double u = sample_uniform(a.seed, (uint32_t)i, (uint32_t)k);
-        double Ci = b.C[i];
-        double rest = S - Ci;
-        double tgt = u * rest;
-        int lo = i + 1, hi = d - 1;
-        while (lo < hi) {
-            int mid = lo + ((hi - lo) >> 1);
-            if (b.C[mid] - Ci < tgt) lo = mid + 1; else hi = mid;
-        }
-        b.jt[i] = lo;
-        const SEnt ei = b.s[i], el = b.s[lo];
-        atomicAdd(&b.minc[ei.row > el.row ? ei.pay : el.pay], 1);   // the larger row gains a dependency
-    }
+    for (int i = t; i < nfill_out; i += kT) sample_partner(a, k, b, i, d, S);
     long long fbase = 0, obase = 0;
-    if (nfill_out > 0 && !carve_pool(fcur, nfill_out, kFillChunk, &a.ctr[kCtrFillTop], a.pool_cap, fbase)) {
-        if (lane == 0) raise_status(a.ctr, kStatusFillPool);
-        return false;
+    bool ok = true;
+    if (w == 0) {
+        if (nfill_out > 0 && !carve_pool(fcur, nfill_out, kFillChunk, &a.ctr[kCtrFillTop], a.pool_cap, fbase)) {
+            if (lane == 0) raise_status(a.ctr, kStatusFillPool);
+            ok = false;
+        }
+        if (ok && !carve_pool(ocur, d, kOutChunk, &a.ctr[kCtrOutTop], a.out_cap, obase)) {
+            if (lane == 0) raise_status(a.ctr, kStatusOutPool);
+            ok = false;
+        }
+        if (ok && lane == 0) {
+            // a column is eliminated in the round after its last dependency, so
+            // its level in the triangular-solve DAG is its round (:638-645); the
+            // queue-driven levels come from atomicMax
+            if (!kAsync) gp(a.level)[k] = round;
+            gp(a.out_start)[k] = obase;
+            gp(a.out_cnt)[k] = d;
+            gp(a.diag)[k] = S;
+        }
+        if (kWaves > 1 && lane == 0) {
+            sh->fbase = fbase;
+            sh->obase = obase;
+            sh->ok = ok;
+        }
     }
-    if (!carve_pool(ocur, d, kOutChunk, &a.ctr[kCtrOutTop], a.out_cap, obase)) {
-        if (lane == 0) raise_status(a.ctr, kStatusOutPool);
-        return false;
+    sync_waves<kWaves>();   // minc and jt complete
+    if constexpr (kWaves > 1) {
+        fbase = sh->fbase;
+        obase = sh->obase;
+        ok = sh->ok != 0;
     }
-    // a column is eliminated in the round after its last dependency, so its
-    // level in the triangular-solve DAG is its round (:638-645)
-    if (lane == 0) {
-        if (!kAsync) a.level[k] = round;     // the queue-driven tail's levels come from atomicMax
-        a.out_start[k] = obase;
-        a.out_cnt[k] = d;
-        a.diag[k] = S;
-    }
-    __syncthreads();   // minc and jt complete
+    if (!ok) return false;
 
-    // ---- 5. per block of 64 entries: the neighbour's net dependency update
-    //         (:653-687), the fill edge (max, min, w_i (S - C_i) / S) pushed
-    //         onto column min's lists, and the factor entry -w/S in row order.
-    //         Up to kB blocks are handled together: their returning atomics
-    //         (list-head exchanges, dependency adds) are all in flight at once,
-    //         so a long column pays one memory round trip per kB blocks, not
-    //         one per block.  The queue-driven tail makes every push, entry and
-    //         raised level visible (release fence) before any dependency add,
-    //         since a neighbour may be taken by another wave as soon as its
-    //         count reaches zero.
-    constexpr int kB = kShort ? 2 : 8;
-    for (int sb = 0; sb < d; sb += kB * kWave) {
-        // the returning atomics of the batch: list-head exchanges and (rounds
-        // only: nothing orders them there but the kernel boundary) the
-        // dependency adds, all in flight together
+    // ---- 5. per entry: the neighbour's net dependency update (:653-687), the
+    //         fill edge (max, min, w_i (S - C_i) / S) pushed onto column min's
+    //         lists, and the factor entry -w/S in row order.  In a round the
+    //         column's returning atomics (list-head exchanges, dependency adds)
+    //         are all in flight at once: nothing orders them but the kernel
+    //         boundary.  Queue-driven: every push and raised level is complete
+    //         before any dependency add (a neighbour may be taken by another
+    //         workgroup as soon as its count reaches zero); they are agent-scope
+    //         accesses, so the wait alone makes them visible, and factor
+    //         entries are read by later launches only.
+    constexpr int kB = kWaves == 1 ? R : 4;
+    for (int sb = 0; sb < d; sb += kB * kT) {
         int old[kB], r[kB], nd[kB];
         bool upd[kB];
 #pragma unroll
         for (int u = 0; u < kB; ++u) {
-            const int e = sb + u * kWave + lane;
+            const int e = sb + u * kT + t;
             old[u] = -1;
             r[u] = -1;
             upd[u] = false;
             nd[u] = 1;
-            if (e < nfill_out) {
-                const int j = b.jt[e];
-                const int ri = b.s[e].row, rj = b.s[j].row;
-                const int cc = ri > rj ? rj : ri;
-                const int rec = (int)(fbase + e);
-                old[u] = atomicExch(&a.head[(size_t)cc * kFillLists + (rec & (kFillLists - 1))], rec);
-            }
+            if (e < nfill_out) old[u] = push_head(a, b, e, (int)(fbase + e));
             if (!kAsync && e < d) {
                 r[u] = b.mrow[e];
                 const int delta = b.minc[e] - b.mmult[e];
                 upd[u] = r[u] != last && delta != 0;
-                if (upd[u]) nd[u] = atomicAdd(&a.dep[r[u]], delta) + delta;
+                if (upd[u]) nd[u] = atomicAdd(at(&gp(a.dep)[r[u]]), delta) + delta;
             }
         }
 #pragma unroll
         for (int u = 0; u < kB; ++u) {
-            const int e = sb + u * kWave + lane;
+            const int e = sb + u * kT + t;
             if (e < d) {
                 const int rr = b.mrow[e];
-                a.out_row[obase + e] = rr;
-                a.out_val[obase + e] = -(b.mw[e] / S);
-                if (kAsync && rr != last) atomicMax(&a.level[rr], round + 1);
+                gp(a.out_row)[obase + e] = rr;
+                gp(a.out_val)[obase + e] = -(b.mw[e] / S);
+                if (kAsync && rr != last) atomicMax(at(&gp(a.level)[rr]), round + 1);
             }
             if (e < nfill_out) {
-                const int j = b.jt[e];
-                const SEnt se = b.s[e];
-                const int ri = se.row, rj = b.s[j].row;
-                FillRec fr;
-                fr.row = ri > rj ? ri : rj;
-                fr.next = old[u];
-                fr.w = (se.w * (S - b.C[e])) / S;
-                a.pool[(int)(fbase + e)] = fr;
+                const FillRec fr = fill_record(b, e, S, old[u]);
+                if (kAsync) store_record(at(gp(a.pool) + (int)(fbase + e)), fr);
+                else *at(gp(a.pool) + (int)(fbase + e)) = fr;
             }
         }
         if constexpr (!kAsync) {
@@ -772,13 +729,14 @@ __device__ __forceinline__ bool process_column(const FactorArgs &a, int k, int r
         }
     }
     if constexpr (kAsync) {
-        fence_release();
-        for (int sb = 0; sb < d; sb += kB * kWave) {
+        drain_stores();
+        sync_waves<kWaves>();
+        for (int sb = 0; sb < d; sb += kB * kT) {
             int r[kB], nd[kB];
             bool upd[kB];
 #pragma unroll
             for (int u = 0; u < kB; ++u) {
-                const int e = sb + u * kWave + lane;
+                const int e = sb + u * kT + t;
                 r[u] = -1;
                 upd[u] = false;
                 nd[u] = 1;
@@ -786,11 +744,10 @@ __device__ __forceinline__ bool process_column(const FactorArgs &a, int k, int r
                     r[u] = b.mrow[e];
                     const int delta = b.minc[e] - b.mmult[e];
                     upd[u] = r[u] != last && delta != 0;
-                    if (upd[u]) nd[u] = atomicAdd(&a.dep[r[u]], delta) + delta;
+                    if (upd[u]) nd[u] = atomicAdd(at(&gp(a.dep)[r[u]]), delta) + delta;
                 }
             }
-            fence_acq_rel();
-            // the ready neighbours of these blocks, one queue atomic for all
+            // the ready neighbours of this wave, one queue atomic for all
             unsigned int cnt = 0;
             uint64_t mk[kB];
 #pragma unroll
@@ -800,7 +757,7 @@ __device__ __forceinline__ bool process_column(const FactorArgs &a, int k, int r
             }
             if (cnt) {
                 unsigned int qb = 0;
-                if (lane == 0) qb = atomicAdd(a.aq_ctr + kAqTail, cnt);
+                if (lane == 0) qb = atomicAdd(at(gp(a.aq_ctr) + kAqTail), cnt);
                 qb = bcast(qb, 0);
 #pragma unroll
                 for (int u = 0; u < kB; ++u) {
@@ -808,71 +765,172 @@ __device__ __forceinline__ bool process_column(const FactorArgs &a, int k, int r
                     // queue's end means inconsistent dependency counts
                     const bool ready = (mk[u] >> lane) & 1ull;
                     const unsigned int slot = qb + (unsigned int)lanes_below(mk[u]);
-                    if (ready && slot < a.aq_total) st_relaxed(&next[slot], r[u]);
+                    if (ready && slot < a.aq_total) st_relaxed(at(gp(next) + slot), r[u]);
                     if (ready && slot >= a.aq_total) raise_status(a.ctr, kStatusInconsistent);
                     qb += (unsigned int)__popcll(mk[u]);
                 }
             }
         }
     }
-    __syncthreads();
+    sync_waves<kWaves>();
     return true;
 }
 
-// Eliminates column k; newly ready neighbours are appended to `next`.
-// Returns false if the pools or the scratch are exhausted (status set).
-// kDefer (round kernel): a column larger than the LDS buffer is appended to
-// the round's deferred list; otherwise (large-LDS kernel) it is gathered
-// again into this workgroup's global scratch.
-template <int kMaxR, bool kDefer, bool kAsync = false>
-__device__ bool eliminate_column(const FactorArgs &a, int k, int round, char *lds, int lds_cap, Cursor &fcur,
-                                 Cursor &ocur, int *next, unsigned int *next_set, unsigned int *defer_count)
+// A column without entries: zero pivot (driver_local.cpp:491-498).  One lane.
+template <bool kAsync>
+__device__ __forceinline__ void empty_column(const FactorArgs &a, int k, int round)
+{
+    if (!kAsync) gp(a.level)[k] = round;
+    gp(a.out_start)[k] = 0;
+    gp(a.out_cnt)[k] = 0;
+    gp(a.diag)[k] = 0.0;
+}
+
+// Eliminates column k in the round kernel; newly ready neighbours are appended
+// to `next`.  A column larger than the LDS buffer is appended to the round's
+// deferred list.  Returns false if the pools are exhausted (status set).
+__device__ __forceinline__ bool eliminate_column(const FactorArgs &a, int k, int round, char *lds, Cursor &fcur,
+                                                 Cursor &ocur, int *next, unsigned int *next_set,
+                                                 unsigned int *defer_count)
 {
     const int lane = lane_id();
     // the list heads do not depend on the column's slice: one memory trip for both
-    const int f0 = lane < kFillLists ? a.head[(size_t)k * kFillLists + lane] : -1;
-    const int lo0 = a.lo_ptr[k];
-    const int norig = a.lo_ptr[k + 1] - lo0;
-
-    // ---- 1. gather (driver_local.cpp:459-487; cpu auxilliary.hpp:89-173)
-    // into this kernel's LDS; the entries are counted as they come (no fill
-    // counter is kept), and a column that turns out larger than the buffer is
-    // deferred (round kernel) or gathered again into the global scratch
-    const ColBuf b = carve(lds, lds_cap);
-    int m = gather_column<kDefer>(a, lo0, norig, f0, b, lds_cap);
-    if (m == 0) {                      // empty column: zero pivot (driver_local.cpp:491-498)
-        if (lane == 0) {
-            if (!kAsync) a.level[k] = round;
-            a.out_start[k] = 0;
-            a.out_cnt[k] = 0;
-            a.diag[k] = 0.0;
-        }
+    const int f0 = gp(a.head)[(size_t)k * kFillLists + lane];
+    const int lo0 = gp(a.lo_ptr)[k];
+    const int norig = gp(a.lo_ptr)[k + 1] - lo0;
+    // ---- 1. gather (driver_local.cpp:459-487; cpu auxilliary.hpp:89-173);
+    // the entries are counted as they come (no fill counter is kept)
+    const ColBuf b = carve(lds, kLdsCap);
+    gather_original(a, lo0, norig, b, kLdsCap, lane, kWave);
+    const int m = gather_fills<true, false>(a, norig, f0, b, kLdsCap);
+    wave_fence();
+    if (m == 0) {
+        if (lane == 0) empty_column<false>(a, k, round);
         return true;
     }
-    const int P = next_pow2(m);
-    if (P > lds_cap) {
-        if constexpr (kDefer) {
-            // too big for this kernel's LDS: the round's large-LDS kernel takes it
-            if (lane == 0) a.big_list[atomicAdd(defer_count, 1u)] = k;
-            return true;
-        } else {
-            if (P > a.scratch_cap) {
-                if (lane == 0) {
-                    atomicMax(&a.ctr[kCtrScratchNeed], (unsigned long long)P);
-                    raise_status(a.ctr, kStatusScratch);
-                }
-                return false;
-            }
-            const ColBuf g = carve(a.scratch + (size_t)blockIdx.x * (size_t)a.scratch_cap * kBytesPerEntry, a.scratch_cap);
-            if (gather_column<false>(a, lo0, norig, f0, g, a.scratch_cap) != m) {
-                if (lane == 0) raise_status(a.ctr, kStatusInconsistent);
-                return false;
-            }
-            return process_column<kMaxR, kAsync>(a, k, round, g, m, fcur, ocur, next, next_set);
-        }
+    if (m > kLdsCap) {                 // the round's large-LDS kernel takes it
+        if (lane == 0) gp(a.big_list)[atomicAdd(defer_count, 1u)] = k;
+        return true;
     }
-    // the round kernel (kDefer) reaches here only with P <= lds_cap = kLdsCap entries
-    return process_column<kMaxR, kAsync, kDefer>(a, k, round, b, m, fcur, ocur, next, next_set);
+    return process_column<false, 1, kLdsCap / kWave>(a, nullptr, k, round, b, nullptr, nullptr, m, fcur,
+                                                     ocur, next, next_set);
+}
+
+// LDS of the large-LDS kernels: the column buffer, the sorts' second entry
+// array and the workgroup's words.
+constexpr size_t kWgColBytes = (size_t)kBigCap * kBytesPerEntry;
+constexpr size_t kWgTmpBytes = (size_t)kBigCap * sizeof(SEnt);
+constexpr size_t kWgLds = kWgColBytes + kWgTmpBytes + sizeof(WgShared);
+static_assert(kWgLds <= 160 * 1024, "one workgroup's LDS");
+
+// A column of more than kBigCap entries, in this workgroup's global scratch
+// (column buffer, entry array, block sums).  Not inlined: it is rare, and the
+// kernels' code stays half as long without it.
+template <bool kAsync>
+__device__ __attribute__((noinline)) bool eliminate_in_scratch(const FactorArgs *pa, WgShared *psh, int k, int round,
+                                                               int m, Cursor *fcur, Cursor *ocur, int *next,
+                                                               unsigned int *next_set)
+{
+    const FactorArgs &a = *pa;
+    WgShared &sh = *psh;
+    const int t = threadIdx.x;
+    const int P = next_pow2(m);
+    if (P > a.scratch_cap) {
+        if (t == 0) {
+            atomicMax(&a.ctr[kCtrScratchNeed], (unsigned long long)P);
+            raise_status(a.ctr, kStatusScratch);
+        }
+        return false;
+    }
+    const int lo0 = gp(a.lo_ptr)[k];
+    const int norig = gp(a.lo_ptr)[k + 1] - lo0;
+    char *mine = at(gp(a.scratch) + (size_t)blockIdx.x * (size_t)a.scratch_cap * kScratchBytesPerEntry);
+    const ColBuf g = carve(mine, a.scratch_cap);
+    SEnt *tmp = reinterpret_cast<SEnt *>(mine + (size_t)a.scratch_cap * kBytesPerEntry);
+    double *tot = reinterpret_cast<double *>(tmp + a.scratch_cap);
+    gather_original(a, lo0, norig, g, a.scratch_cap, t, kWgThreads);
+    if (t < kWave) {
+        const int *hd = at(gp(a.head) + (size_t)k * kFillLists + t);
+        const int c = gather_fills<false, kAsync>(a, norig, kAsync ? ld_relaxed(hd) : *hd, g, a.scratch_cap);
+        if (t == 0) sh.ok = c == m;
+    }
+    __syncthreads();
+    if (!sh.ok) {
+        if (t == 0) raise_status(a.ctr, kStatusInconsistent);
+        return false;
+    }
+    return process_column<kAsync, kWgWaves, 0>(a, &sh, k, round, g, tmp, tot, m, *fcur, *ocur, next, next_set);
+}
+
+// The columns that pop() hands to this workgroup's first wave (column < 0: no
+// more; round: its level), until there are none or the pools are exhausted.
+template <bool kAsync, typename Pop>
+__device__ __forceinline__ void wg_columns(const FactorArgs &a, char *lds, Pop pop, int *next, unsigned int *next_set)
+{
+    static_assert(kFillLists == kWave, "one list per lane");
+    WgShared &sh = *reinterpret_cast<WgShared *>(lds + kWgColBytes + kWgTmpBytes);
+    SEnt *tmp = reinterpret_cast<SEnt *>(lds + kWgColBytes);
+    const ColBuf b = carve(lds, kBigCap);
+    const int t = threadIdx.x, lane = lane_id();
+    long long *ws = a.wave_state + 4 * ((size_t)a.big_ws + blockIdx.x);
+    Cursor fcur, ocur;
+    fcur.cur = ws[0]; fcur.end = ws[1];
+    ocur.cur = ws[2]; ocur.end = ws[3];
+    while (true) {
+        if (t < kWave) {
+            int k, m = 0, round = 0;
+            while (true) {
+                k = pop(round);
+                if (k < 0) break;
+                // ---- 1. gather (as the round kernel, up to kBigCap entries)
+                const int *hd = at(gp(a.head) + (size_t)k * kFillLists + lane);
+                const int f0 = kAsync ? ld_relaxed(hd) : *hd;
+                const int lo0 = gp(a.lo_ptr)[k];
+                const int norig = gp(a.lo_ptr)[k + 1] - lo0;
+                gather_original(a, lo0, norig, b, kWave, lane, kWave);
+                m = gather_fills<false, kAsync>(a, norig, f0, b, kBigCap);
+                wave_fence();
+                if (m > kWave) break;
+                if (m == 0) {
+                    if (lane == 0) empty_column<kAsync>(a, k, round);
+                    continue;
+                }
+                if (!process_column<kAsync, 1, 1>(a, &sh, k, round, b, nullptr, nullptr, m, fcur, ocur, next, next_set)) {
+                    k = -1;
+                    break;
+                }
+            }
+            if (lane == 0) {
+                sh.k = k;
+                sh.m = m;
+                sh.round = round;
+            }
+        }
+        __syncthreads();
+        const int k = sh.k, m = sh.m, round = sh.round;
+        if (k < 0) break;
+        bool ok;
+        if (m <= kBigCap) {
+            // original entries past the first kWave (few columns have them)
+            const int lo0 = gp(a.lo_ptr)[k];
+            const int norig = gp(a.lo_ptr)[k + 1] - lo0;
+            if (norig > kWave) {
+                gather_original(a, lo0, norig, b, kBigCap, kWave + t, kWgThreads);
+                __syncthreads();
+            }
+            ok = process_column<kAsync, kWgWaves, 0>(a, &sh, k, round, b, tmp, sh.tot, m, fcur, ocur, next, next_set);
+        } else {
+            Cursor fc = fcur, oc = ocur;       // copies: the call takes addresses
+            ok = eliminate_in_scratch<kAsync>(&a, &sh, k, round, m, &fc, &oc, next, next_set);
+            fcur = fc;
+            ocur = oc;
+        }
+        if (!ok) break;
+    }
+    if (t == 0) {
+        ws[0] = fcur.cur; ws[1] = fcur.end;
+        ws[2] = ocur.cur; ws[3] = ocur.end;
+    }
 }
 
 }  // namespace
@@ -892,7 +950,7 @@ __global__ void __launch_bounds__(kWave) k_factor_round(const FactorArgs *__rest
     const unsigned int ncur = __shfl(incl, kWave - 1, kWave);
     if (blockIdx.x == 0) {
         list_set(a, round + 2)[lane_id()] = 0u;
-        if (lane_id() == 0) a.round_count[round] = ncur;
+        if (lane_id() == 0) gp(a.round_count)[round] = ncur;
     }
     if (ncur <= (unsigned int)kBigGrid) return;     // a narrow round: the large-LDS kernel takes all of it
     if (status != 0ull) return;
@@ -901,13 +959,10 @@ __global__ void __launch_bounds__(kWave) k_factor_round(const FactorArgs *__rest
     fcur.cur = ws[0]; fcur.end = ws[1];
     ocur.cur = ws[2]; ocur.end = ws[3];
     unsigned int *next_set = list_set(a, round + 1);
-    bool ok = true;
     for (unsigned int i = blockIdx.x; i < ncur; i += gridDim.x) {
         const int col = cur[list_index(a, c, incl, i)];
-        if (!eliminate_column<2, true>(a, col, round, lds, kLdsCap, fcur, ocur, next, next_set,
-                                       &a.big_count[round])) { ok = false; break; }
+        if (!eliminate_column(a, col, round, lds, fcur, ocur, next, next_set, &a.big_count[round])) break;
     }
-    (void)ok;
     if (lane_id() == 0) {
         ws[0] = fcur.cur; ws[1] = fcur.end;
         ws[2] = ocur.cur; ws[3] = ocur.end;
@@ -915,10 +970,10 @@ __global__ void __launch_bounds__(kWave) k_factor_round(const FactorArgs *__rest
 }
 
 // The round's columns deferred by k_factor_round (more than kLdsCap entries):
-// one wave per column with kBigCap entries of LDS (columns above that use the
+// one workgroup per column with kBigCap entries of LDS (columns above that use the
 // per-workgroup global scratch).  Runs after k_factor_round of the same round.
-__global__ void __launch_bounds__(kWave) k_factor_round_big(const FactorArgs *__restrict__ pa, int round, const int *cur,
-                                                            int *next)
+__global__ void __launch_bounds__(kWgThreads) k_factor_round_big(const FactorArgs *__restrict__ pa, int round,
+                                                                 const int *cur, int *next)
 {
     const FactorArgs &a = *pa;
     extern __shared__ __attribute__((aligned(16))) char lds_big[];
@@ -926,63 +981,50 @@ __global__ void __launch_bounds__(kWave) k_factor_round_big(const FactorArgs *__
     // column per workgroup); otherwise the columns k_factor_round deferred
     unsigned int c, incl;
     list_counts(a, list_set(a, round), c, incl);
-    const unsigned int ndef = a.big_count[round];
+    const unsigned int ndef = gp(a.big_count)[round];
     const unsigned long long status = a.ctr[kCtrStatus];
     const unsigned int ncur = __shfl(incl, kWave - 1, kWave);
     const bool narrow = ncur <= (unsigned int)kBigGrid;
     const unsigned int nbig = narrow ? ncur : ndef;
     if (nbig == 0) return;
-    if (status != 0ull) return;
-    Cursor fcur, ocur;
-    long long *ws = a.wave_state + 4 * ((size_t)a.big_ws + blockIdx.x);
-    fcur.cur = ws[0]; fcur.end = ws[1];
-    ocur.cur = ws[2]; ocur.end = ws[3];
-    for (unsigned int i = blockIdx.x; i < nbig; i += gridDim.x) {
-        const int col = narrow ? cur[list_index(a, c, incl, i)] : a.big_list[i];
-        if (!eliminate_column<2, false>(a, col, round, lds_big, kBigCap, fcur, ocur, next, list_set(a, round + 1), nullptr))
-            break;
-    }
-    if (lane_id() == 0) {
-        ws[0] = fcur.cur; ws[1] = fcur.end;
-        ws[2] = ocur.cur; ws[3] = ocur.end;
-    }
+    unsigned int i = blockIdx.x;
+    wg_columns<false>(a, lds_big, [&](int &level) {
+        if (i >= nbig || status != 0ull) return -1;
+        const int k = narrow ? cur[list_index(a, c, incl, i)] : gp(a.big_list)[i];
+        level = round;
+        i += gridDim.x;
+        return k;
+    }, next, list_set(a, round + 1));
 }
 
 // ---- queue-driven tail -----------------------------------------------------
 // Once a round holds at most kBigGrid columns, the rest of the elimination runs
-// in this one persistent launch: every wave takes the next queue index, waits
-// until that slot holds a column (slots start at -1), eliminates it in the
-// large LDS buffer and appends the neighbours it made ready.  A column's level
+// in this one persistent launch: every workgroup takes the next queue index,
+// waits until that slot holds a column (slots start at -1), eliminates it and
+// appends the neighbours it made ready.  A column's level
 // is 1 + the largest level of its lower neighbours (atomicMax by each of them
 // before its dependency update), the same value the rounds assign.  Slot h is
-// written by the wave that made its column ready, which is running, so every
+// written by the workgroup that made its column ready, which is running, so every
 // wait ends; the waits are bounded all the same (status bit on expiry).
 __device__ __forceinline__ bool factor_should_stop(const FactorArgs &a)
 {
     return ld_relaxed(&a.ctr[kCtrStatus]) != 0ull;
 }
 
-__global__ void __launch_bounds__(kWave) k_factor_async(const FactorArgs *__restrict__ pa, unsigned int total)
+__global__ void __launch_bounds__(kWgThreads) k_factor_async(const FactorArgs *__restrict__ pa, unsigned int total)
 {
     const FactorArgs &a = *pa;
     extern __shared__ __attribute__((aligned(16))) char lds_big[];
-    const int lane = lane_id();
-    Cursor fcur, ocur;
-    long long *ws = a.wave_state + 4 * ((size_t)a.big_ws + blockIdx.x);
-    fcur.cur = ws[0]; fcur.end = ws[1];
-    ocur.cur = ws[2]; ocur.end = ws[3];
-    while (true) {
+    wg_columns<true>(a, lds_big, [&](int &level) {
         unsigned int h = 0;
-        if (lane == 0) h = atomicAdd(a.aq_ctr + kAqHead, 1u);
-        h = bcast(h, 0);
-        if (h >= total) break;
         int k = -1;
-        if (lane == 0) {
-            k = ld_relaxed(&a.aq[h]);
-            if (k < 0) {
+        if (lane_id() == 0) {
+            h = atomicAdd(at(gp(a.aq_ctr) + kAqHead), 1u);
+            if (h < total) k = ld_relaxed(at(&gp(a.aq)[h]));
+            if (h < total && k < 0) {
                 const long long t0 = wall_clock64();
                 int nap = 1;
-                while ((k = ld_relaxed(&a.aq[h])) < 0) {
+                while ((k = ld_relaxed(at(&gp(a.aq)[h]))) < 0) {
                     if (factor_should_stop(a)) break;
                     if (wall_clock64() - t0 > a.spin_ticks) {
                         raise_status(a.ctr, kStatusTimeout);
@@ -994,17 +1036,10 @@ __global__ void __launch_bounds__(kWave) k_factor_async(const FactorArgs *__rest
             }
         }
         k = bcast(k, 0);
-        if (k < 0) break;                          // stopped (status raised)
-        fence_acquire();
-        const int lvl = a.level[k];
-        if (!eliminate_column<2, false, true>(a, k, lvl, lds_big, kBigCap, fcur, ocur, a.aq, nullptr, nullptr))
-            break;
-        if (factor_should_stop(a)) break;
-    }
-    if (lane == 0) {
-        ws[0] = fcur.cur; ws[1] = fcur.end;
-        ws[2] = ocur.cur; ws[3] = ocur.end;
-    }
+        asm volatile("" ::: "memory");             // the column's loads follow the slot's
+        if (k >= 0) level = ld_relaxed(at(&gp(a.level)[k]));
+        return k;                                  // < 0: all columns taken, or stopped (status raised)
+    }, a.aq, nullptr);
 }
 
 // The queue starts with round `round`'s list (its columns' level is the round).
@@ -1019,7 +1054,7 @@ __global__ void k_factor_async_init(FactorArgs a, int round, const int *cur, uns
         s_c[threadIdx.x] = c;
         s_incl[threadIdx.x] = incl;
     }
-    for (unsigned int i = threadIdx.x; i < total; i += blockDim.x) a.aq[i] = -1;
+    for (unsigned int i = threadIdx.x; i < total; i += blockDim.x) gp(a.aq)[i] = -1;
     __syncthreads();
     const unsigned int ncur = min(s_incl[kWave - 1], total);
     for (unsigned int i = threadIdx.x; i < ncur; i += blockDim.x) {
@@ -1027,12 +1062,12 @@ __global__ void k_factor_async_init(FactorArgs a, int round, const int *cur, uns
         while (s < kWave - 1 && s_incl[s] <= i) ++s;
         const size_t idx = (size_t)s * (size_t)a.seg_cap + (i - (s_incl[s] - s_c[s]));
         const int col = cur[idx];
-        a.aq[i] = col;
-        a.level[col] = round;
+        gp(a.aq)[i] = col;
+        gp(a.level)[col] = round;
     }
     if (threadIdx.x == 0) {
-        a.aq_ctr[kAqHead] = 0u;
-        a.aq_ctr[kAqTail] = ncur;
+        gp(a.aq_ctr)[kAqHead] = 0u;
+        gp(a.aq_ctr)[kAqTail] = ncur;
     }
 }
 
@@ -1076,7 +1111,7 @@ void launch_factor_rounds(const FactorArgs &a, const FactorArgs *da, int num_blo
         const int *cur = (r & 1) ? a.list1 : a.list0;
         int *next = (r & 1) ? a.list0 : a.list1;
         hipLaunchKernelGGL(k_factor_round, dim3(num_blocks), dim3(kWave), 0, s, da, r, cur, next);
-        hipLaunchKernelGGL(k_factor_round_big, dim3(kBigGrid), dim3(kWave), (size_t)kBigCap * kBytesPerEntry, s, da, r,
+        hipLaunchKernelGGL(k_factor_round_big, dim3(kBigGrid), dim3(kWgThreads), kWgLds, s, da, r,
                            cur, next);
     }
 }
@@ -1084,9 +1119,9 @@ void launch_factor_rounds(const FactorArgs &a, const FactorArgs *da, int num_blo
 void factor_kernel_setup()
 {
     (void)hipFuncSetAttribute((const void *)k_factor_round_big, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)((size_t)kBigCap * kBytesPerEntry));
+                              (int)kWgLds);
     (void)hipFuncSetAttribute((const void *)k_factor_async, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              (int)((size_t)kBigCap * kBytesPerEntry));
+                              (int)kWgLds);
 }
 
 void launch_factor_async(const FactorArgs &a0, const FactorArgs *da, int round, unsigned int total, hipStream_t s)
@@ -1096,11 +1131,11 @@ void launch_factor_async(const FactorArgs &a0, const FactorArgs *da, int round, 
     const int *cur = (round & 1) ? a.list1 : a.list0;
     // one block: the init kernel's slot clearing must finish before it seeds the queue
     hipLaunchKernelGGL(k_factor_async_init, dim3(1), dim3(1024), 0, s, a, round, cur, total);
-    hipLaunchKernelGGL(k_factor_async, dim3(kBigGrid), dim3(kWave), (size_t)kBigCap * kBytesPerEntry, s, da, total);
+    hipLaunchKernelGGL(k_factor_async, dim3(kBigGrid), dim3(kWgThreads), kWgLds, s, da, total);
 }
 
 int factor_lds_capacity() { return kLdsCap; }
-int factor_scratch_bytes_per_entry() { return kBytesPerEntry; }
+int factor_scratch_bytes_per_entry() { return kScratchBytesPerEntry; }
 long long factor_pool_slack(int num_blocks) { return (long long)(num_blocks + kBigGrid) * (kFillChunk + kOutChunk); }
 
 int factor_occupancy_blocks(int device)
