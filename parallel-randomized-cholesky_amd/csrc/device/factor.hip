@@ -12,8 +12,9 @@
 //
 // MI355X design:
 //   * rounds: one launch eliminates every column made ready by the previous
-//     launch (one wave64 per column, grid-stride over the round's list), so
-//     the kernel boundary orders all communication -- no fences, no waits;
+//     launch (a wave64 per column, or per four where many are ready,
+//     grid-stride over the round's list), so the kernel boundary orders all
+//     communication -- no fences, no waits;
 //   * gather, duplicate merge, sorts and the prefix sum run in LDS (global
 //     per-workgroup scratch for columns above the LDS capacity); columns of more
 //     than 128 entries, and of more than 64 where few are ready, are eliminated
@@ -816,6 +817,176 @@ __device__ __forceinline__ bool eliminate_column(const FactorArgs &a, int k, int
                                                      ocur, next, next_set);
 }
 
+// ---- several small columns per wave -------------------------------------------
+// The first rounds of a large matrix hold hundreds of thousands of columns of a
+// few entries each; one wave per column leaves most lanes idle and is bound by
+// the column's chain of memory trips times the waves in flight.  Here a wave
+// eliminates kPack columns at a time, kPackLanes lanes (and entries) each:
+// the first round of a 192^3 grid (learned order) 2.9 -> 1.4 ms, its first
+// twenty 18.6 -> 10.3 ms.  Four waves per SIMD (125 registers) issue most of the
+// time: reading the next columns' lists ahead gained nothing, a fifth wave by
+// spilling lost 3 %.
+constexpr int kPackLanes = 16;
+constexpr int kPack = kWave / kPackLanes;
+
+// Sorts a group's b.s[0..len) (wave_sort, by kPackLanes lanes).
+template <bool kByRow>
+__device__ __forceinline__ void pack_sort(const ColBuf &b, int gl, int len)
+{
+    SEnt v;
+    v.row = 0;
+    v.pay = 0;
+    v.w = 0.0;
+    if (gl < len) v = b.s[gl];
+    const double key = sort_key(v.w);
+    if (v.w != v.w && gl < len) b.s[gl].w = key;
+    wave_fence();
+    int c = 0;
+#pragma unroll
+    for (int j0 = 0; j0 < kPackLanes; j0 += kCountBatch) {
+        if (ballot(j0 < len) == 0ull) break;
+        SEnt x[kCountBatch];
+#pragma unroll
+        for (int u = 0; u < kCountBatch; ++u) x[u] = b.s[j0 + u];
+#pragma unroll
+        for (int u = 0; u < kCountBatch; ++u)
+            c += (j0 + u < len) & ent_before<kByRow>(x[u].row, x[u].w, v.row, key, j0 + u < gl);
+    }
+    wave_fence();
+    if (gl < len) b.s[c] = v;
+    wave_fence();
+}
+
+// Eliminates the groups' columns (k: this lane's group's, < 0: none) with
+// entries in b.  over: a lane of every group whose column has more than
+// kPackLanes entries (left as it was).  Returns false if the pools are exhausted.
+__device__ __forceinline__ bool eliminate_packed(const FactorArgs &a, int k, int round, char *lds, Cursor &fcur,
+                                                 Cursor &ocur, int *next, unsigned int *next_set, uint64_t &over)
+{
+    constexpr int G = kPackLanes, kHeads = kFillLists / G;
+    static_assert(kWave * kBytesPerEntry <= kLdsCap * kBytesPerEntry, "the groups share one column buffer");
+    const int lane = lane_id(), gl = lane % G, gb = lane - gl;
+    const int last = a.n - 1;
+    const uint64_t below = (1ull << lane) - 1ull, group = ((1ull << G) - 1ull) << gb;
+    ColBuf b = carve(lds, kLdsCap);
+    b.s += gb; b.mw += gb; b.C += gb; b.mrow += gb; b.mmult += gb; b.minc += gb; b.jt += gb;
+
+    // ---- 1. gather: originals one per lane, kHeads lists per lane
+    const bool act = k >= 0;
+    int m = 0, f[kHeads];
+#pragma unroll
+    for (int u = 0; u < kHeads; ++u) f[u] = -1;
+    if (act) {
+#pragma unroll
+        for (int u = 0; u < kHeads; ++u) f[u] = gp(a.head)[(size_t)k * kFillLists + gl * kHeads + u];
+        const int lo0 = gp(a.lo_ptr)[k];
+        m = gp(a.lo_ptr)[k + 1] - lo0;
+        if (gl < m && m <= G) {
+            SEnt v;
+            v.row = gp(a.lo_row)[lo0 + gl];
+            v.pay = 1;
+            v.w = gp(a.lo_w)[lo0 + gl];
+            b.s[gl] = v;
+        }
+    }
+    while (true) {
+        uint64_t mask[kHeads], any = 0;
+        FillRec rec[kHeads];
+#pragma unroll
+        for (int u = 0; u < kHeads; ++u) {
+            const bool more = f[u] >= 0 && m <= G;
+            mask[u] = ballot(more);
+            any |= mask[u];
+            if (more) rec[u] = *at(gp(a.pool) + f[u]);
+        }
+        if (!any) break;
+#pragma unroll
+        for (int u = 0; u < kHeads; ++u) {
+            if ((mask[u] >> lane) & 1ull) {
+                const int pos = m + __popcll(mask[u] & group & below);
+                if (pos < G) {
+                    SEnt v;
+                    v.row = rec[u].row;
+                    v.pay = 1;
+                    v.w = rec[u].w;
+                    b.s[pos] = v;
+                }
+                f[u] = rec[u].next;
+            }
+            m += __popcll(mask[u] & group);
+        }
+    }
+    over = ballot(m > G && gl == 0);
+    const bool live = m > 0 && m <= G;
+    if (act && m == 0 && gl == 0) empty_column<false>(a, k, round);
+    if (!live) m = 0;
+    if (ballot(live) == 0ull) return true;
+    wave_fence();
+
+    // ---- 2. sort by (row, w), merge (as process_column, a group's lanes)
+    pack_sort<true>(b, gl, m);
+    RowRun run;
+    run.head = false;
+    if (gl < m) run = row_run(b.s, gl, m);
+    const uint64_t heads = ballot(run.head) & group;
+    if (run.head) put_merged(b, __popcll(heads & below), run);
+    const int d = __popcll(heads);
+    wave_fence();
+
+    // ---- 3. sort by (w, row); sums (one block of the canonical scan)
+    if (gl < d) b.s[gl] = merged_entry(b, gl);
+    wave_fence();
+    pack_sort<false>(b, gl, d);
+    double x = gl < d ? b.s[gl].w : 0.0;
+    for (int off = 1; off < G; off <<= 1) {
+        const double o = __shfl_up(x, off, G);
+        if (gl >= off) x = x + o;
+    }
+    if (gl < d) b.C[gl] = x;
+    wave_fence();
+    const double S = d > 0 ? b.C[d - 1] : 0.0;
+
+    // ---- 4. sampled partners; the groups' pool entries in one piece
+    const bool fill = gl < d - 1, ent = gl < d;
+    if (fill) sample_partner(a, k, b, gl, d, S);
+    const uint64_t fmask = ballot(fill), emask = ballot(ent);
+    long long fbase = 0, obase = 0;
+    if (fmask && !carve_pool(fcur, __popcll(fmask), kFillChunk, &a.ctr[kCtrFillTop], a.pool_cap, fbase)) {
+        if (lane == 0) raise_status(a.ctr, kStatusFillPool);
+        return false;
+    }
+    if (!carve_pool(ocur, __popcll(emask), kOutChunk, &a.ctr[kCtrOutTop], a.out_cap, obase)) {
+        if (lane == 0) raise_status(a.ctr, kStatusOutPool);
+        return false;
+    }
+    const int rec = (int)(fbase + __popcll(fmask & below));
+    const long long oe = obase + __popcll(emask & below);
+    if (live && gl == 0) {
+        gp(a.level)[k] = round;
+        gp(a.out_start)[k] = oe;
+        gp(a.out_cnt)[k] = d;
+        gp(a.diag)[k] = S;
+    }
+    wave_fence();   // minc and jt complete
+
+    // ---- 5. fills, dependency updates, factor entries
+    int old = -1, r = -1, nd = 1;
+    bool upd = false;
+    if (fill) old = push_head(a, b, gl, rec);
+    if (ent) {
+        r = b.mrow[gl];
+        const int delta = b.minc[gl] - b.mmult[gl];
+        upd = r != last && delta != 0;
+        if (upd) nd = atomicAdd(at(&gp(a.dep)[r]), delta) + delta;
+        gp(a.out_row)[oe] = r;
+        gp(a.out_val)[oe] = -(b.mw[gl] / S);
+    }
+    if (fill) *at(gp(a.pool) + rec) = fill_record(b, gl, S, old);
+    list_append(a, next_set, next, upd && nd == 0, r);
+    wave_fence();
+    return true;
+}
+
 // LDS of the large-LDS kernels: the column buffer, the sorts' second entry
 // array and the workgroup's words.
 constexpr size_t kWgColBytes = (size_t)kBigCap * kBytesPerEntry;
@@ -959,9 +1130,24 @@ __global__ void __launch_bounds__(kWave) k_factor_round(const FactorArgs *__rest
     fcur.cur = ws[0]; fcur.end = ws[1];
     ocur.cur = ws[2]; ocur.end = ws[3];
     unsigned int *next_set = list_set(a, round + 1);
-    for (unsigned int i = blockIdx.x; i < ncur; i += gridDim.x) {
-        const int col = cur[list_index(a, c, incl, i)];
-        if (!eliminate_column(a, col, round, lds, fcur, ocur, next, next_set, &a.big_count[round])) break;
+    // several columns per wave where every group has one to do: below, the
+    // second pass over columns too large for a group costs more than it saves
+    // (12000 columns: 53 us, one per wave 45 us; 20000: 104 and 143 us)
+    const bool packed = ncur > (unsigned int)kPack * gridDim.x;
+    const unsigned int per = packed ? kPack : 1;
+    bool ok = true;
+    for (unsigned int i = blockIdx.x * per; ok && i < ncur; i += gridDim.x * per) {
+        int col = -1;
+        for (unsigned int q = 0; q < per; ++q) {
+            const unsigned int j = min(i + q, ncur - 1);
+            const int kq = cur[list_index(a, c, incl, j)];
+            if (!packed || (unsigned int)(lane_id() / kPackLanes) == q) col = i + q < ncur ? kq : -1;
+        }
+        uint64_t left = 1ull;
+        if (packed) ok = eliminate_packed(a, col, round, lds, fcur, ocur, next, next_set, left);
+        for (; ok && left; left &= left - 1ull)
+            ok = eliminate_column(a, bcast(col, __ffsll((unsigned long long)left) - 1), round, lds, fcur, ocur, next, next_set,
+                                  &a.big_count[round]);
     }
     if (lane_id() == 0) {
         ws[0] = fcur.cur; ws[1] = fcur.end;
