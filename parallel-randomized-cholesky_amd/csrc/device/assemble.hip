@@ -24,6 +24,7 @@ constexpr int kScanBlock = 256;
 constexpr int kScanItems = 4;
 constexpr int kScanTile = kScanBlock * kScanItems;
 
+template <int kThreads>
 __device__ int block_exclusive_scan(int v, int *lds_wave, int &total)
 {
     // inclusive wave scan
@@ -37,7 +38,7 @@ __device__ int block_exclusive_scan(int v, int *lds_wave, int &total)
     if (lane == kWave - 1) lds_wave[wid] = x;
     __syncthreads();
     int carry = 0, tot = 0;
-    for (int w = 0; w < kScanBlock / kWave; ++w) {
+    for (int w = 0; w < kThreads / kWave; ++w) {
         if (w < wid) carry += lds_wave[w];
         tot += lds_wave[w];
     }
@@ -58,7 +59,7 @@ __global__ void __launch_bounds__(kScanBlock) k_scan_tiles(const int *in, int *o
         s += v[t];
     }
     int total;
-    int ex = block_exclusive_scan(s, lds_wave, total);
+    int ex = block_exclusive_scan<kScanBlock>(s, lds_wave, total);
     for (int t = 0; t < kScanItems; ++t) {
         int i = base + t;
         if (i < n) out[i] = ex;
@@ -76,7 +77,7 @@ __global__ void __launch_bounds__(kScanBlock) k_scan_single(int *sums, int m, in
         int i = base + threadIdx.x;
         int v = (i < m) ? sums[i] : 0;
         int total;
-        int ex = block_exclusive_scan(v, lds_wave, total);
+        int ex = block_exclusive_scan<kScanBlock>(v, lds_wave, total);
         if (i < m) sums[i] = carry + ex;
         carry += total;
     }
@@ -88,14 +89,46 @@ __global__ void k_scan_add(int *out, int n, const int *tile_off)
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
         out[i] += tile_off[i / kScanTile];
 }
+
+// A short scan in one launch: one large workgroup, kSmallTile values at a time.
+// Up to two rounds it costs what one of the three launches does (4096 unknowns
+// have sixteen scans in an assembly that is bound by its launches).
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallTile = kSmallThreads * kScanItems;
+constexpr int kSmallScan = 2 * kSmallTile;
+__global__ void __launch_bounds__(kSmallThreads) k_scan_small(const int *in, int *out, int n)
+{
+    __shared__ int lds_wave[kSmallThreads / kWave];
+    int carry = 0;
+    for (int base = 0; base < n; base += kSmallTile) {
+        const int i0 = base + (int)threadIdx.x * kScanItems;
+        int v[kScanItems];
+        int s = 0;
+        for (int t = 0; t < kScanItems; ++t) {
+            v[t] = i0 + t < n ? in[i0 + t] : 0;
+            s += v[t];
+        }
+        int total;
+        int ex = carry + block_exclusive_scan<kSmallThreads>(s, lds_wave, total);
+        for (int t = 0; t < kScanItems; ++t) {
+            if (i0 + t < n) out[i0 + t] = ex;
+            ex += v[t];
+        }
+        carry += total;
+    }
+    if (threadIdx.x == 0) out[n] = carry;
+}
 }  // namespace
 
 size_t scan_tmp_elems(int n) { return (size_t)(n + kScanTile - 1) / kScanTile + 1; }
 
 void scan_exclusive(const int *in, int *out, int n, int *tmp, hipStream_t s)
 {
-    int tiles = (n + kScanTile - 1) / kScanTile;
-    if (tiles < 1) tiles = 1;
+    if (n <= kSmallScan) {
+        hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(kSmallThreads), 0, s, in, out, n);
+        return;
+    }
+    const int tiles = (n + kScanTile - 1) / kScanTile;
     hipLaunchKernelGGL(k_scan_tiles, dim3(tiles), dim3(kScanBlock), 0, s, in, out, n, tmp);
     hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(kScanBlock), 0, s, tmp, tiles, out + n);
     hipLaunchKernelGGL(k_scan_add, dim3(1024), dim3(256), 0, s, out, n, (const int *)tmp);
@@ -396,6 +429,14 @@ __global__ void k_chunk_fill(int nchunks, int nlevels, const int *lvl_ptr, const
     }
 }
 
+template <typename T>
+__global__ void k_zero_slots(int ns, int *ind_l, T *val_l, int *ind_u, T *val_u)
+{
+    *ind_l = ns;
+    *ind_u = ns;
+    *val_l = (T)0;
+    *val_u = (T)0;
+}
 __global__ void k_pack_meta(int nchunks, const int *start, const int *cnt, const int *off, const int *slices,
                             int4 *meta)
 {
@@ -636,6 +677,14 @@ void launch_pack_meta(int nchunks, const int *start, const int *cnt, const int *
 {
     hipLaunchKernelGGL(k_pack_meta, dim3(1024), dim3(256), 0, s, nchunks, start, cnt, off, slices, meta);
 }
+
+template <typename T>
+void launch_zero_slots(int ns, int *ind_l, T *val_l, int *ind_u, T *val_u, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_zero_slots<T>, dim3(1), dim3(1), 0, s, ns, ind_l, val_l, ind_u, val_u);
+}
+template void launch_zero_slots<float>(int, int *, float *, int *, float *, hipStream_t);
+template void launch_zero_slots<double>(int, int *, double *, int *, double *, hipStream_t);
 
 template void launch_lt_fill<float>(const AssembleArgs &, const int *, int *, float *, float *, hipStream_t);
 template void launch_lt_fill<double>(const AssembleArgs &, const int *, int *, double *, double *, hipStream_t);

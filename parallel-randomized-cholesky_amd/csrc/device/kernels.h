@@ -176,6 +176,9 @@ void launch_chunk_count(int nlevels, const int *lvl_ptr, const int *lw, int gmin
 void launch_chunk_fill(int nchunks, int nlevels, const int *lvl_ptr, const int *chunk_ptr, const int *lw, int gmin,
                        int *chunk_start, int *chunk_cnt, hipStream_t s);
 // meta[c] = {start[c], cnt[c], off[c], slices[c]}
+// the zero entry (index ns, value 0) after each sweep layout
+template <typename T>
+void launch_zero_slots(int ns, int *ind_l, T *val_l, int *ind_u, T *val_u, hipStream_t s);
 void launch_pack_meta(int nchunks, const int *start, const int *cnt, const int *off, const int *slices, int4 *meta,
                       hipStream_t s);
 template <typename T> void launch_gather_t(const T *src, const int *idx, T *dst, int n, hipStream_t s);

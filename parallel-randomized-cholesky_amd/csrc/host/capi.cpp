@@ -742,57 +742,60 @@ static int run_elimination(rc_handle_t h, double *ms_out, int *regrowths)
         unsigned long long st = 0;
         unsigned long long async_total = 0;      // columns eliminated by the queue-driven tail
         int async_round = -1;
-        unsigned int *probe = nullptr;     // the next round's list counters, then the status word
-        RC_HIP(hipHostMalloc((void **)&probe, (kListSlots + 2) * sizeof(unsigned int), hipHostMallocDefault));
+        // pinned: the next round's list counters and the status word
+        constexpr size_t kProbeBytes = (kListSlots + 2) * sizeof(unsigned int);
+        RC_HIP(h->pin.ensure(kProbeBytes));
+        unsigned int *probe = h->pin.as<unsigned int>(0);
         while (true) {
             int nr = std::min(batch, h->nf + 1 - round);
             if (nr <= 0) break;
             launch_factor_rounds(a, da, h->num_blocks, round, nr, s);
             round += nr;
-            hipError_t e = hipMemcpyAsync(probe, h->seg_count.as<unsigned int>() + (size_t)(round % 3) * kListSlots,
-                                          kListSlots * sizeof(unsigned int), hipMemcpyDeviceToHost, s);
-            if (e == hipSuccess) e = hipMemcpyAsync(probe + kListSlots, h->ctr.as<unsigned long long>() + kCtrStatus,
-                                                    sizeof(unsigned long long), hipMemcpyDeviceToHost, s);
-            if (e == hipSuccess) e = hipStreamSynchronize(s);
-            if (e != hipSuccess) { (void)hipHostFree(probe); return fail(h, RC_ERR_HIP, hipGetErrorString(e)); }
+            RC_HIP(hipMemcpyAsync(probe, h->seg_count.as<unsigned int>() + (size_t)(round % 3) * kListSlots,
+                                  kListSlots * sizeof(unsigned int), hipMemcpyDeviceToHost, s));
+            RC_HIP(hipMemcpyAsync(probe + kListSlots, h->ctr.as<unsigned long long>() + kCtrStatus,
+                                  sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+            RC_HIP(hipStreamSynchronize(s));
             std::memcpy(&st, probe + kListSlots, sizeof(st));
             unsigned long long pending = probe[kListSegs];
             for (int q = 0; q < kListSegs; ++q) pending += std::min<unsigned long long>(probe[q], (unsigned long long)a.seg_cap);
             if (st != 0 || pending == 0) break;
             if (h->async_tail && pending <= (unsigned long long)h->async_width) {
                 // narrow from here: the rest runs in one queue-driven launch
-                std::vector<unsigned int> cnt((size_t)round);
-                e = hipMemcpyAsync(cnt.data(), h->round_count.p, cnt.size() * sizeof(unsigned int),
-                                   hipMemcpyDeviceToHost, s);
-                if (e == hipSuccess) e = hipStreamSynchronize(s);
-                if (e != hipSuccess) { (void)hipHostFree(probe); return fail(h, RC_ERR_HIP, hipGetErrorString(e)); }
+                RC_HIP(h->pin.ensure((size_t)round * sizeof(unsigned int)));
+                const unsigned int *cnt = h->pin.as<unsigned int>(0);
+                RC_HIP(hipMemcpyAsync(h->pin.p, h->round_count.p, (size_t)round * sizeof(unsigned int),
+                                      hipMemcpyDeviceToHost, s));
+                RC_HIP(hipStreamSynchronize(s));
                 unsigned long long before = 0;
-                for (unsigned int v : cnt) before += v;
+                for (int i = 0; i < round; ++i) before += cnt[i];
                 async_total = (unsigned long long)(h->nf - 1) - before;
                 async_round = round;
                 const unsigned int aqt = (unsigned int)async_total;
-                e = hipMemcpyAsync((char *)h->fargs.p + offsetof(FactorArgs, aq_total), &aqt, sizeof(aqt),
-                                   hipMemcpyHostToDevice, s);
-                if (e != hipSuccess) { (void)hipHostFree(probe); return fail(h, RC_ERR_HIP, hipGetErrorString(e)); }
+                RC_HIP(hipMemcpyAsync((char *)h->fargs.p + offsetof(FactorArgs, aq_total), &aqt, sizeof(aqt),
+                                      hipMemcpyHostToDevice, s));
                 launch_factor_async(a, da, round, aqt, s);
                 break;
             }
             batch = std::min(batch * 2, 64);     // bounds the empty rounds launched past the end
         }
-        (void)hipHostFree(probe);
         launch_factor_finish(a, s);
         RC_HIP(hipGetLastError());
         RC_HIP(hipEventRecord(e1, s));
-        unsigned long long c[kCtrCount];
-        RC_HIP(hipMemcpyAsync(c, h->ctr.p, sizeof(c), hipMemcpyDeviceToHost, s));
-        std::vector<unsigned int> counts((size_t)round + 1);
-        RC_HIP(hipMemcpyAsync(counts.data(), h->round_count.p, counts.size() * sizeof(unsigned int),
+        // pinned: the counters, the queue's tail, the rounds' lengths
+        const size_t ncounts = (size_t)round + 1;
+        constexpr size_t kTailAt = kCtrCount * sizeof(unsigned long long), kCountsAt = kTailAt + 8;
+        RC_HIP(h->pin.ensure(kCountsAt + ncounts * sizeof(unsigned int)));
+        const unsigned long long *c = h->pin.as<unsigned long long>(0);
+        const unsigned int *counts = h->pin.as<unsigned int>(kCountsAt);
+        RC_HIP(hipMemcpyAsync(h->pin.p, h->ctr.p, kTailAt, hipMemcpyDeviceToHost, s));
+        RC_HIP(hipMemcpyAsync(h->pin.as<unsigned int>(kCountsAt), h->round_count.p, ncounts * sizeof(unsigned int),
                               hipMemcpyDeviceToHost, s));
-        unsigned int aq_tail = 0;
         if (async_round >= 0)
-            RC_HIP(hipMemcpyAsync(&aq_tail, h->aq_ctr.as<unsigned int>() + kAqTail, sizeof(aq_tail),
-                                  hipMemcpyDeviceToHost, s));
+            RC_HIP(hipMemcpyAsync(h->pin.as<unsigned int>(kTailAt), h->aq_ctr.as<unsigned int>() + kAqTail,
+                                  sizeof(unsigned int), hipMemcpyDeviceToHost, s));
         RC_HIP(hipStreamSynchronize(s));
+        const unsigned int aq_tail = async_round >= 0 ? *h->pin.as<unsigned int>(kTailAt) : 0u;
         float ms = 0.f;
         (void)hipEventElapsedTime(&ms, e0, e1);
         (void)hipEventDestroy(e0);
@@ -802,7 +805,7 @@ static int run_elimination(rc_handle_t h, double *ms_out, int *regrowths)
         if (st == 0) {
             unsigned long long done = async_total;
             int used = 0;
-            const size_t nc = async_round >= 0 ? (size_t)async_round : counts.size();
+            const size_t nc = async_round >= 0 ? (size_t)async_round : ncounts;
             for (size_t i = 0; i < nc; ++i) {
                 done += counts[i];
                 if (counts[i]) used = (int)i + 1;
@@ -915,9 +918,15 @@ static int assemble(rc_handle_t h, double *ms_out, bool tail = true)
     RC_HIP(h->lt_ptr.ensure(nsz * sizeof(int)));
     launch_lt_counts(a, h->tmp_a.as<int>(), s);
     scan_exclusive(h->tmp_a.as<int>(), h->lt_ptr.as<int>(), ns, h->tmp_scan.as<int>(), s);
-    int nnz = 0;
-    RC_HIP(hipMemcpyAsync(&nnz, h->lt_ptr.as<int>() + ns, sizeof(int), hipMemcpyDeviceToHost, s));
+    unsigned long long *d_max = h->ctr.as<unsigned long long>() + kCtrCount - 1;
+    RC_HIP(hipMemsetAsync(d_max, 0, sizeof(unsigned long long), s));
+    launch_level_max(ns, h->level.as<int>(), d_max, s);
+    RC_HIP(h->pin.ensure(16));
+    RC_HIP(hipMemcpyAsync(h->pin.p, d_max, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
+    RC_HIP(hipMemcpyAsync(h->pin.as<int>(8), h->lt_ptr.as<int>() + ns, sizeof(int), hipMemcpyDeviceToHost, s));
     RC_HIP(hipStreamSynchronize(s));
+    const unsigned long long maxlev = *h->pin.as<unsigned long long>(0);
+    const int nnz = *h->pin.as<int>(8);
     h->nnz_lt = nnz;
     RC_HIP(h->lt_ind.ensure((size_t)std::max(nnz, 1) * sizeof(int)));
     RC_HIP(h->lt_val.ensure((size_t)std::max(nnz, 1) * sizeof(T)));
@@ -941,12 +950,6 @@ static int assemble(rc_handle_t h, double *ms_out, bool tail = true)
     launch_segment_bounds(nnz, k0, 0, ns, h->l_ptr.as<int>(), s);
 
     // 3. level order: rows sorted by (level, descending length of their L row)
-    unsigned long long *d_max = h->ctr.as<unsigned long long>() + kCtrCount - 1;
-    RC_HIP(hipMemsetAsync(d_max, 0, sizeof(unsigned long long), s));
-    launch_level_max(ns, h->level.as<int>(), d_max, s);
-    unsigned long long maxlev = 0;
-    RC_HIP(hipMemcpyAsync(&maxlev, d_max, sizeof(maxlev), hipMemcpyDeviceToHost, s));
-    RC_HIP(hipStreamSynchronize(s));
     const int nl = ns > 0 ? (int)maxlev + 1 : 0;
     h->nlevels = nl;
     const int lvl_bits = bit_width(nl);
@@ -1044,9 +1047,12 @@ static int assemble(rc_handle_t h, double *ms_out, bool tail = true)
     RC_HIP(h->tmp_scan.ensure(scan_tmp_elems(nseg + 2) * sizeof(int) + 64));
     launch_chunk_count(nseg, lptr, h->lvl_w.as<int>(), h->sweep_gmin, lcnt, s);
     scan_exclusive(lcnt, cptr, nseg, h->tmp_scan.as<int>(), s);
-    int nchunks = 0;
-    RC_HIP(hipMemcpyAsync(&nchunks, cptr + nseg, sizeof(int), hipMemcpyDeviceToHost, s));
+    // level and chunk boundaries (lptr, lcnt, cptr lie one after the other)
+    RC_HIP(h->pin.ensure(3 * nssz * sizeof(int)));
+    RC_HIP(hipMemcpyAsync(h->pin.p, lptr, 3 * nssz * sizeof(int), hipMemcpyDeviceToHost, s));
     RC_HIP(hipStreamSynchronize(s));
+    const int *hs = h->pin.as<int>(0), *hcs = hs + 2 * nssz;
+    const int nchunks = hcs[nseg];
     h->nchunks = nchunks;
     RC_HIP(h->chunk_start.ensure((size_t)std::max(nchunks, 1) * sizeof(int)));
     RC_HIP(h->chunk_cnt.ensure((size_t)std::max(nchunks, 1) * sizeof(int)));
@@ -1055,10 +1061,6 @@ static int assemble(rc_handle_t h, double *ms_out, bool tail = true)
     // level split: the trailing levels [tail_level, nl) form the tail
     std::vector<int> hl(nlsz), hc(nlsz);
     {
-        std::vector<int> hs(nssz), hcs(nssz);
-        RC_HIP(hipMemcpyAsync(hs.data(), lptr, nssz * sizeof(int), hipMemcpyDeviceToHost, s));
-        RC_HIP(hipMemcpyAsync(hcs.data(), cptr, nssz * sizeof(int), hipMemcpyDeviceToHost, s));
-        RC_HIP(hipStreamSynchronize(s));
         for (size_t L = 0; L < nlsz; ++L) {       // level L starts at its first segment
             hl[L] = hs[L * (size_t)per_level];
             hc[L] = hcs[L * (size_t)per_level];
@@ -1078,42 +1080,32 @@ static int assemble(rc_handle_t h, double *ms_out, bool tail = true)
     auto ell_offsets = [&](const int *width, int *off, int nslices, int64_t &total) -> int {
         launch_mul64(width, h->tmp_a.as<int>(), nslices, s);
         scan_exclusive(h->tmp_a.as<int>(), off, nslices, h->tmp_scan.as<int>(), s);
-        int t = 0;
-        RC_HIP(hipMemcpyAsync(&t, off + nslices, sizeof(int), hipMemcpyDeviceToHost, s));
+        RC_HIP(hipMemcpyAsync(h->pin.p, off + nslices, sizeof(int), hipMemcpyDeviceToHost, s));
         RC_HIP(hipStreamSynchronize(s));
-        total = t;
+        total = *h->pin.as<int>(0);
         return RC_OK;
     };
     // grouped layout: width -> slice count in place, slice block sizes -> offsets
-    auto sweep_offsets = [&](const int *ptr, int *slices, int *off, int64_t &total) -> int {
+    auto sweep_offsets = [&](const int *ptr, int *slices, int *off, int *total) -> hipError_t {
         launch_ell_width(nbulk, h->chunk_start.as<int>(), h->chunk_cnt.as<int>(), h->order.as<int>(), ns, ptr,
                          slices, s);
         launch_sweep_layout(nbulk, h->chunk_cnt.as<int>(), slices, slices, h->tmp_a.as<int>(), s);
         scan_exclusive(h->tmp_a.as<int>(), off, nbulk, h->tmp_scan.as<int>(), s);
-        int t = 0;
-        RC_HIP(hipMemcpyAsync(&t, off + nbulk, sizeof(int), hipMemcpyDeviceToHost, s));
-        RC_HIP(hipStreamSynchronize(s));
-        total = t;
-        return RC_OK;
+        return hipMemcpyAsync(total, off + nbulk, sizeof(int), hipMemcpyDeviceToHost, s);
     };
-    int rc = sweep_offsets(h->l_ptr.as<int>(), h->lf_width.as<int>(), h->lf_off.as<int>(), h->ell_l);
-    if (rc != RC_OK) return rc;
-    rc = sweep_offsets(h->lt_ptr.as<int>(), h->lb_width.as<int>(), h->lb_off.as<int>(), h->ell_u);
-    if (rc != RC_OK) return rc;
+    RC_HIP(sweep_offsets(h->l_ptr.as<int>(), h->lf_width.as<int>(), h->lf_off.as<int>(), h->pin.as<int>(0)));
+    RC_HIP(sweep_offsets(h->lt_ptr.as<int>(), h->lb_width.as<int>(), h->lb_off.as<int>(), h->pin.as<int>(4)));
+    RC_HIP(hipStreamSynchronize(s));
+    h->ell_l = *h->pin.as<int>(0);
+    h->ell_u = *h->pin.as<int>(4);
     // one more entry after the chunks: the zero slot (index ns, value 0)
     // that lanes without a slot load when the sweeps prefetch a chunk
     RC_HIP(h->lf_ind.ensure(((size_t)h->ell_l + 1) * sizeof(int)));
     RC_HIP(h->lf_val.ensure(((size_t)h->ell_l + 1) * sizeof(T)));
     RC_HIP(h->lb_ind.ensure(((size_t)h->ell_u + 1) * sizeof(int)));
     RC_HIP(h->lb_val.ensure(((size_t)h->ell_u + 1) * sizeof(T)));
-    {
-        const T zero_val = (T)0;
-        RC_HIP(hipMemcpyAsync(h->lf_ind.as<int>() + h->ell_l, &ns, sizeof(int), hipMemcpyHostToDevice, s));
-        RC_HIP(hipMemcpyAsync(h->lf_val.as<T>() + h->ell_l, &zero_val, sizeof(T), hipMemcpyHostToDevice, s));
-        RC_HIP(hipMemcpyAsync(h->lb_ind.as<int>() + h->ell_u, &ns, sizeof(int), hipMemcpyHostToDevice, s));
-        RC_HIP(hipMemcpyAsync(h->lb_val.as<T>() + h->ell_u, &zero_val, sizeof(T), hipMemcpyHostToDevice, s));
-        RC_HIP(hipStreamSynchronize(s));
-    }
+    launch_zero_slots<T>(ns, h->lf_ind.as<int>() + h->ell_l, h->lf_val.as<T>() + h->ell_l,
+                         h->lb_ind.as<int>() + h->ell_u, h->lb_val.as<T>() + h->ell_u, s);
     EllSrc fs{h->l_ptr.as<int>(), nullptr, h->lt_val.p, h->vals0.as<int>(), h->rowk.as<int>(), nullptr};
     launch_sweep_fill<T, T>(nbulk, h->chunk_start.as<int>(), h->chunk_cnt.as<int>(), h->order.as<int>(), fs,
                             h->lf_off.as<int>(), h->lf_width.as<int>(), ns, (T)0, h->lf_ind.as<int>(), h->lf_val.as<T>(),
@@ -1156,7 +1148,7 @@ static int assemble(rc_handle_t h, double *ms_out, bool tail = true)
         launch_tail_count<T>(tb, false, bs, cnt_b, flag, s);
         scan_exclusive(cnt_f, h->tf_ptr.as<int>(), tb.ntail, h->tmp_scan.as<int>(), s);
         scan_exclusive(cnt_b, h->tb_ptr.as<int>(), tb.ntail, h->tmp_scan.as<int>(), s);
-        int tot[3] = {0, 0, 0};
+        int *tot = h->pin.as<int>(0);
         RC_HIP(hipMemcpyAsync(&tot[0], h->tf_ptr.as<int>() + nt, sizeof(int), hipMemcpyDeviceToHost, s));
         RC_HIP(hipMemcpyAsync(&tot[1], h->tb_ptr.as<int>() + nt, sizeof(int), hipMemcpyDeviceToHost, s));
         RC_HIP(hipMemcpyAsync(&tot[2], flag, sizeof(int), hipMemcpyDeviceToHost, s));
@@ -1194,7 +1186,7 @@ static int assemble(rc_handle_t h, double *ms_out, bool tail = true)
     RC_HIP(h->a_width.ensure(tsz * sizeof(int)));
     RC_HIP(h->a_off.ensure(tsz * sizeof(int)));
     launch_ell_width(ntiles, nullptr, nullptr, h->order.as<int>(), ns, h->a_ptr.as<int>(), h->a_width.as<int>(), s);
-    rc = ell_offsets(h->a_width.as<int>(), h->a_off.as<int>(), ntiles, h->ell_a);
+    const int rc = ell_offsets(h->a_width.as<int>(), h->a_off.as<int>(), ntiles, h->ell_a);
     if (rc != RC_OK) return rc;
     RC_HIP(h->a_ell_ind.ensure((size_t)std::max<int64_t>(h->ell_a, 1) * sizeof(int)));
     RC_HIP(h->a_ell_val.ensure((size_t)std::max<int64_t>(h->ell_a, 1) * sizeof(double)));

@@ -44,6 +44,30 @@ struct DevVec {
     template <typename T> T *as() const { return static_cast<T *>(p); }
 };
 
+// Pinned host words that small results are copied into (grow-only): copies to
+// pageable memory go through the runtime's own buffers one at a time.
+struct PinnedVec {
+    void *p = nullptr;
+    size_t bytes = 0;
+    PinnedVec() = default;
+    PinnedVec(const PinnedVec &) = delete;
+    PinnedVec &operator=(const PinnedVec &) = delete;
+    ~PinnedVec() { if (p) (void)hipHostFree(p); }
+    hipError_t ensure(size_t b)
+    {
+        if (b <= bytes && p) return hipSuccess;
+        if (p) (void)hipHostFree(p);
+        p = nullptr;
+        bytes = 0;
+        b = (b + 4095) / 4096 * 4096;
+        const hipError_t e = hipHostMalloc(&p, b, hipHostMallocDefault);
+        if (e != hipSuccess) { p = nullptr; return e; }
+        bytes = b;
+        return hipSuccess;
+    }
+    template <typename T> T *as(size_t byte) const { return reinterpret_cast<T *>(static_cast<char *>(p) + byte); }
+};
+
 // Largest fill pool (records) and factor (off-diagonal entries) the int32
 // indices of the fill lists and of the CSR of L^T can address.
 constexpr long long kMaxPoolRecords = 2147483647LL;
@@ -106,6 +130,7 @@ struct rc_handle_s {
     int sweep_gmin = kSweepMinGroupDefault;   // fewest lanes per row in a sweep chunk (chunks of <= 256 / gmin rows)
     long long pool_cap = 0, out_cap = 0;
     int scratch_cap = 0;
+    PinnedVec pin;                    // read-backs of the factorization and the assembly
     int rounds = 0;
 
     // factor result: CSR of L^T in the factored numbering (export / dump)
