@@ -1595,19 +1595,21 @@ static int reduction_blocks(rc_handle_t h)
     return need < h->reduce_blocks ? need : h->reduce_blocks;
 }
 
-// Persistent sweep workgroups for `values` vector entries (rows x lanes): the
-// autotuner's choice, else one per CU, two from 1.5 M values, for many
-// right-hand sides four from 32 M.  More of them hold chunks far ahead of the front, and their polls
-// slow it down; wide levels want more in flight.  Forward / backward sweep, us,
-// at 256 / 512 / 1024 workgroups: 64^3 SDDM 231/225, 252/243, 285/289; 701x699
-// 130/119, 141/129, 156/154; 128^3 SDDM 611/625, 589/586, 663/679; 192^3
-// learned 993/951, 960/882, 1035/965; 47x48x45 x 5 318/317, 341/341, 356/359;
-// 385x384 x 64 280/305, 203/235, 203/243; 2048x1024 x 64 4365/4412, 2468/2470,
-// 2466/1594.
-static int sweep_grid(rc_handle_t h, double values, bool multi)
+// Persistent sweep workgroups for `rows` rows of k values: the autotuner's
+// choice, else one per CU, two from 1.5 M values, and four for many right-hand
+// sides from 32 M values, or from 6 M with 64 of them (a chunk is then a few
+// rows).  More of them hold chunks far ahead of the front, and their polls slow
+// it down; wide levels want more in flight.  Forward / backward sweep, us, at
+// 256 / 512 workgroups: 701x699 107/111, 115/119; 101x83x89 339/360, 353/372;
+// 128^3 SDDM 597/614, 564/573; 192^3 learned 980/932, 940/866.  Solves, ms, at
+// 512 / 1024: 385x384 x 32 18.7, 18.8, x 64 25.9, 24.9; 47x48x45 x 32 32.8, 33.6,
+// x 64 41.3, 40.8; 80x81x82 x 16 45.2, 46.0.
+static int sweep_grid(rc_handle_t h, int rows, int k)
 {
     if (h->sweep_blocks > 0) return h->sweep_blocks;
-    const int per_cu = values < 1.5e6 ? 1 : (multi && values > 3.2e7 ? 4 : 2);
+    const double values = (double)rows * k;
+    const bool four = k > 1 && (values > 3.2e7 || (k >= 64 && values > 6e6));
+    const int per_cu = values < 1.5e6 ? 1 : (four ? 4 : 2);
     return std::min(h->sweep_blocks_max, per_cu * h->cus);
 }
 
@@ -1649,7 +1651,7 @@ SolveArgs solve_args(rc_handle_t h)
     a.ctr_fwd = h->ctrs.as<unsigned int>();
     a.ctr_bwd = h->ctrs.as<unsigned int>() + kClaimQueues * kClaimStride;
     a.reduce_blocks = reduction_blocks(h);
-    a.sweep_blocks = sweep_grid(h, h->ns, false);
+    a.sweep_blocks = sweep_grid(h, h->ns, 1);
     a.bulk_chunks = h->bulk_chunks;
     a.tail_level = h->tail_level;
     a.tail_pos0 = h->tail_pos0;
@@ -1996,7 +1998,7 @@ static int multi_args(rc_handle_t h, int k, MultiArgs &a)
     a.ctr_fwd = h->ctrs.as<unsigned int>();
     a.ctr_bwd = h->ctrs.as<unsigned int>() + kClaimQueues * kClaimStride;
     a.reduce_blocks = h->reduce_blocks;
-    a.sweep_blocks = sweep_grid(h, (double)n * K, true);
+    a.sweep_blocks = sweep_grid(h, (int)n, (int)K);
     a.spin_ticks = h->spin_ticks;
     return RC_OK;
 }
@@ -2683,7 +2685,7 @@ static int rc_autotune_impl(rc_handle_t h, int reps, rc_tune_stats *st)
         *out = f + b;
         return rc;
     };
-    const int tail0 = h->tail_max_rows, grid0 = sweep_grid(h, h->ns, false);
+    const int tail0 = h->tail_max_rows, grid0 = sweep_grid(h, h->ns, 1);
     double base = 0.0;
     int rc = sweep_ms(&base);
     if (rc != RC_OK) return rc;
