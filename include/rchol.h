@@ -295,12 +295,12 @@ int rc_time_kernel(rc_handle_t h, int kernel, int reps, double *ms_per_launch, d
 /* ---------------- autotuner (no reference counterpart) ----------------
  * The reference's thread-block count is a command-line argument (driver.cu:
  * 2157).  rc_autotune times both triangular sweeps for every candidate launch
- * configuration (start of the dense tail: by estimate or by a level width
- * limit, x persistent sweep grid) on the factored structure and keeps the fastest for this handle
- * (later factors of the same handle reuse it).  Needs rc_factor and rc_set_rhs
+ * configuration (start of the dense tail, by estimate or by a level width
+ * limit, x persistent sweep grid) on the factored structure and keeps the
+ * fastest for this handle (later factors of the same handle reuse it).  Needs rc_factor and rc_set_rhs
  * first; the RHS and the factor are unchanged.  reps <= 0 means 5. */
 typedef struct {
-    int32_t tail_max_rows;    /* chosen tail width limit (0 = no tail, -1 = estimate)  */
+    int32_t tail_max_rows;    /* width limit of the chosen tail (0 = no tail)          */
     int32_t sweep_blocks;     /* chosen persistent sweep grid                          */
     int32_t configs_tried;
     double sweeps_ms_before;  /* forward + backward sweep before tuning                */
