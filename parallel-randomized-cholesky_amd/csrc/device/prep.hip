@@ -124,9 +124,9 @@ __global__ void k_trim_fill(int n, const int *ptr, const int *ind, const double 
     }
 }
 
-// lower slice and dependency counts, one wave per column: rows are sorted,
-// so the strict-lower entries of column j are a suffix; dep[j] counts the
-// rows above j (the pattern is symmetric: the lower entries in row j)
+// lower slice and dependency counts: rows are sorted, so the strict-lower
+// entries of column j are a suffix; dep[j] counts the rows above j (the pattern
+// is symmetric: the lower entries in row j)
 __device__ __forceinline__ int first_at_least(const int *ind, int b, int e, int r)
 {
     while (b < e) {
@@ -144,8 +144,7 @@ __global__ void k_lower_count(int n, const int *ptr, const int *ind, int *cnt, i
     for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += gridDim.x * blockDim.x) {
         const int b = ptr[j], e = ptr[j + 1];
         const int d = first_at_least(ind, b, e, j);
-        const int l = d < e && ind[d] == j ? d + 1 : d;
-        cnt[j] = e - l;
+        cnt[j] = e - first_at_least(ind, d, e, j + 1);      // triplets may repeat the diagonal too
         dep[j] = d - b;
     }
 }
