@@ -295,7 +295,6 @@ struct SolveArgs {
     const int *a_off, *a_width, *a_ind;
     const double *a_val;
     // level schedule (positions)
-    int nchunks;
     const int *chunk_start, *chunk_cnt;
     const int4 *cm_f, *cm_b;      // per chunk {start, cnt, ELL offset, slices} of the two sweeps
     // L rows (forward) and L^T rows (backward) in grouped sliced ELL per chunk
@@ -316,7 +315,7 @@ struct SolveArgs {
     int sweep_blocks;             // persistent sweep workgroups (occupancy-sized)
     // level split: chunks [0, bulk_chunks) belong to the wide levels and run
     // on the persistent grid; levels [tail_level, nlevels) form the tail
-    int bulk_chunks, tail_level, nlevels;
+    int nchunks, bulk_chunks, tail_level, nlevels;
     // tail (see launch_tail_*): rows [tail_pos0, n) in tail_nb blocks of
     // tail_m rows; CSR of the entries outside a row's block (absolute column
     // positions, tf_*: rows of L, tb_*: rows of L^T), the blocks' inverses by
@@ -394,14 +393,14 @@ struct MultiScalars {
 
 struct MultiArgs {
     int n, K, k;                  // rows, lane stride (pow2 >= k), right-hand sides
+    int nchunks;                  // chunks of the levels before the tail
     const int *a_ptr, *a_ind;     // CSR in position numbering
     const double *a_val;
     const int *row_ord;           // position of every input-numbered row (the SpMV's visiting order)
     const int *l_ptr, *l_ind, *lt_ptr, *lt_ind;
     const void *l_val, *lt_val, *diag;
-    // chunks of the levels before the tail, {first row, rows, first entry,
-    // entries} per sweep (launch_mchunk_fill)
-    int nchunks;
+    // per chunk {first row, rows, first entry, entries} of the two sweeps
+    // (launch_mchunk_fill)
     const int4 *cm_f, *cm_b;
     // tail: as in SolveArgs; tacc: tail_m x K; tail_part: kMTailParts partial
     // results of a block; tail_arrive: arrivals per row tile (zero between launches)

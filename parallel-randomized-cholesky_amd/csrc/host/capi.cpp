@@ -1615,7 +1615,7 @@ static int sweep_grid(rc_handle_t h, int rows, int k)
 
 SolveArgs solve_args(rc_handle_t h)
 {
-    SolveArgs a;
+    SolveArgs a{};
     a.n = h->ns;
     a.ntiles = h->ntiles;
     a.a_tile_ord = h->tile_ord.as<int>();
@@ -1689,7 +1689,7 @@ extern "C" {
 
 static BatchArgs batch_args(rc_handle_t h)
 {
-    BatchArgs b;
+    BatchArgs b{};
     b.nsys = h->nsys;
     b.nblk = h->nblk;
     batch_carve(b, h->bt_state.p);
@@ -2123,14 +2123,24 @@ static const int *run_done_flag(rc_handle_t h, int mode)
     return reinterpret_cast<const int *>(h->scal.as<char>() + offsetof(PcgScalars, done));
 }
 
-// The cached graph of a run of one handle: two iterations, rebuilt when the
-// buffers it was captured with change.
+// The cached graph of a run of one handle: two iterations, rebuilt when any
+// argument of their launches differs from the captured one (a buffer moved, also
+// by a run of the handle that did not use this graph; another number of
+// right-hand sides in the same lanes).
 static int run_graph(rc_handle_t h, int mode, const MultiArgs &ma, hipGraphExec_t *out)
 {
-    const void *key = mode == kRunMulti ? h->m_x.p : h->y.p;
+    RunArgs args{};
+    args.prec = h->prec;
+    args.nsys = h->nsys;
+    if (mode == kRunMulti) {
+        args.multi = ma;
+    } else {
+        args.single = solve_args(h);
+        if (h->nsys > 0) args.batch = batch_args(h);
+    }
     hipGraphExec_t *slot = mode == kRunMulti ? &h->m_graph : &h->graph;
-    const int kk = mode == kRunMulti ? ma.K : 0;
-    if (*slot && h->graph_key[mode] == key && h->graph_prec_of[mode] == h->prec && h->graph_K[mode] == kk) {
+    GraphArgs<RunArgs> &captured = mode == kRunMulti ? h->m_graph_args : h->graph_args;
+    if (*slot && captured.same(args)) {
         *out = *slot;
         return RC_OK;
     }
@@ -2146,9 +2156,7 @@ static int run_graph(rc_handle_t h, int mode, const MultiArgs &ma, hipGraphExec_
         *slot = nullptr;
         return fail(h, RC_ERR_HIP, std::string("hipGraphInstantiate: ") + hipGetErrorString(e));
     }
-    h->graph_key[mode] = key;
-    h->graph_prec_of[mode] = h->prec;
-    h->graph_K[mode] = kk;
+    captured.set(args);
     *out = *slot;
     return RC_OK;
 }

@@ -15,6 +15,7 @@
 
 #include "../../../include/rchol.h"
 #include "../device/kernels.h"
+#include "graph_args.hpp"
 #include "sparse.hpp"
 
 using namespace rc;
@@ -80,6 +81,15 @@ inline int64_t pow2_at_least(int64_t v)
     return p;
 }
 
+
+// Everything the iterations of a run are launched with: the solve's and (of a
+// batch) the systems' arguments, or the multi-RHS ones; the rest is zero.
+struct RunArgs {
+    SolveArgs single;
+    BatchArgs batch;
+    MultiArgs multi;
+    int prec, nsys;
+};
 
 struct rc_handle_s {
     rc_options opt{};
@@ -172,11 +182,9 @@ struct rc_handle_s {
     std::vector<double> xref;
     int rhs_mode = 0;               // last resident right-hand side: 1 rc_set_rhs, 2 rc_set_rhs_multi
     // captured iteration pairs: graph (single / batch run), m_graph (multi-RHS
-    // run); each is rebuilt when the buffers it was captured with change
+    // run), with the arguments they were captured with
     hipGraphExec_t graph = nullptr, m_graph = nullptr;
-    const void *graph_key[3] = {nullptr, nullptr, nullptr};
-    int graph_prec_of[3] = {0, 0, 0};
-    int graph_K[3] = {0, 0, 0};
+    GraphArgs<RunArgs> graph_args, m_graph_args;
 
     // ordering network: graph + activations of the loaded system
     bool gnn_ready = false, gnn_keep = false;
