@@ -61,7 +61,9 @@ __global__ void k_tail_count(TailBuild tb, int fwd, EllSrc src, int *cnt, int *f
 }
 
 // One wave per tail row: stable compaction of the outer entries; forward, the
-// block's own entries are written to its dense matrix.
+// block's own entries are written to its dense matrix.  A loaded factor may hold
+// an entry in several parts; they lie side by side (rows are sorted by column),
+// and the first one's lane adds them in order.
 template <typename T>
 __global__ void k_tail_split(TailBuild tb, int fwd, EllSrc src, const int *ptr, int *ind, T *val, double *D)
 {
@@ -83,7 +85,14 @@ __global__ void k_tail_split(TailBuild tb, int fwd, EllSrc src, const int *ptr, 
                 e = src.eidx ? src.eidx[b + t] : b + t;
                 pos = entry_pos(src, e);
                 outer = fwd ? pos < lo : pos >= hi;
-                if (fwd && !outer) drow[pos - lo] = (double)sval[e];
+                if (fwd && !outer) {
+                    auto part = [&](int u) { return src.eidx ? src.eidx[b + u] : b + u; };
+                    if (t == 0 || entry_pos(src, part(t - 1)) != pos) {
+                        double v = (double)sval[e];
+                        for (int u = t + 1; u < len && entry_pos(src, part(u)) == pos; ++u) v += (double)sval[part(u)];
+                        drow[pos - lo] = v;
+                    }
+                }
             }
             const uint64_t mo = ballot(outer);
             if (outer) {
