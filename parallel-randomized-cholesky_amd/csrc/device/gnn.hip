@@ -14,6 +14,8 @@
 // so gradients are deterministic.
 #include <hip/hip_bf16.h>
 
+#include <type_traits>
+
 #include "common.cuh"
 #include "kernels.h"
 
@@ -222,7 +224,8 @@ __device__ __forceinline__ void load_dz(int v, int c, const float *dH, const flo
 // tile t of an operand is made of the features 4 j + t.  A wave keeps all 64 x
 // 128 sums; the workgroup's waves are added through LDS in order.  (One thread
 // per output row and 250 rows one after the other took 567 us at 64k rows, this
-// 25 us.)
+// 25 us.)  The products add 0 times the input where dZ is zero, NaN where that
+// input is not finite: k_sum_partials mends it.
 // Layout of a partial: [Ws | Wn | b | wo | bo], as in the weights.
 constexpr int kWgLen = 2 * kH * kH + kH + kH + 1;
 template <bool kLast>
@@ -344,10 +347,11 @@ __global__ void __launch_bounds__(256) k_wgrad2(int n, int rows_per_wave, const 
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const float dv = vb + u < v1 ? d[u] : 0.f;
-            g[0] = fmaf(dv, bf16r(x[u].x), g[0]);
-            g[1] = fmaf(dv, bf16r(x[u].y), g[1]);
-            g[2] = fmaf(dv, bf16r(m[u].x), g[2]);
-            g[3] = fmaf(dv, bf16r(m[u].y), g[3]);
+            const bool on = dv != 0.f;                   // a zero takes nothing, also from an infinity
+            g[0] = fmaf(dv, on ? bf16r(x[u].x) : 0.f, g[0]);
+            g[1] = fmaf(dv, on ? bf16r(x[u].y) : 0.f, g[1]);
+            g[2] = fmaf(dv, on ? bf16r(m[u].x) : 0.f, g[2]);
+            g[3] = fmaf(dv, on ? bf16r(m[u].y) : 0.f, g[3]);
             g[4] += dv;
         }
     }
@@ -365,9 +369,19 @@ __global__ void __launch_bounds__(256) k_wgrad2(int n, int rows_per_wave, const 
     p[4 * kH + lane] = g[4];
 }
 
+// What the weight gradients of a 64-wide layer were formed from.
+struct WgradRows {
+    int n;
+    const float *dH, *H, *ds, *wo, *X, *M;
+};
+
 // Sum of nblocks partials into out[0..len), eight threads per output, each over
-// its share of the partials in order, then the eight in order.
-__global__ void __launch_bounds__(256) k_sum_partials(const float *part, int nblocks, int stride, int len,
+// its share of the partials in order, then the eight in order.  A row whose dZ
+// is zero contributes nothing, whatever its inputs hold: a weight's sum that is
+// not finite is formed again from the rows, zeros skipped.  (Watching for such
+// inputs in k_wgrad64 cost it its registers: 325 -> 331-350 us a gradient.)
+template <bool kLast>
+__global__ void __launch_bounds__(256) k_sum_partials(const float *part, int nblocks, int stride, int len, WgradRows w,
                                                       float *out)
 {
     __shared__ float red[8][32];
@@ -386,10 +400,29 @@ __global__ void __launch_bounds__(256) k_sum_partials(const float *part, int nbl
         }
     red[s][o] = t;
     __syncthreads();
-    if (s == 0 && i < len) {
-        for (int q = 1; q < 8; ++q) t += red[q][o];
-        out[i] = t;
+    t = red[0][o];
+    for (int q = 1; q < 8; ++q) t += red[q][o];
+    const bool again = w.H && i < 2 * kH * kH && !__builtin_isfinite(t);
+    if (__syncthreads_or(again)) {
+        if (again) {
+            const float *in = i < kH * kH ? w.X : w.M;
+            const int row = (i / kH) % kH, col = i % kH;
+            const float wl = kLast ? bf16r(w.wo[row]) : 0.f;
+            const int share = (w.n + 7) / 8, v1 = min(w.n, (s + 1) * share);
+            t = 0.f;
+            for (int v = s * share; v < v1; ++v) {
+                const float g = kLast ? w.ds[v] * wl : w.dH[(size_t)v * kH + row];
+                if (w.H[(size_t)v * kH + row] > 0.f && g != 0.f) t = fmaf(g, bf16r(in[(size_t)v * kH + col]), t);
+            }
+            red[s][o] = t;
+        }
+        __syncthreads();
+        if (again) {
+            t = red[0][o];
+            for (int q = 1; q < 8; ++q) t += red[q][o];
+        }
     }
+    if (s == 0 && i < len) out[i] = t;
 }
 
 // dX[v][i] = sum_o dZ[v][o] bf16(Ws[o][i]);  G[v][i] = sum_o dZ[v][o] bf16(Wn[o][i]):
@@ -491,15 +524,15 @@ void gnn_backward(const GnnArgs &g, const float *w, const float *ds, float *dw, 
     int rows = (n + 4 * kGnnPartials - 1) / (4 * kGnnPartials);
     rows = (rows + 7) / 8 * 8;
     const int nb = (n + 4 * rows - 1) / (4 * rows);
-    auto sum = [&](int stride, int len, float *out) {
-        hipLaunchKernelGGL(k_sum_partials, dim3((len + 31) / 32), dim3(256), 0, s, (const float *)g.part, nb, stride, len,
-                           out);
+    auto sum = [&](auto last, int stride, int len, const WgradRows &r, float *out) {
+        hipLaunchKernelGGL((k_sum_partials<decltype(last)::value>), dim3((len + 31) / 32), dim3(256), 0, s,
+                           (const float *)g.part, nb, stride, len, r, out);
     };
     float *dH = g.dA, *dX = g.dB, *G = g.dC;
     // layer 3 with the output layer (its gradients follow the layer's in dw)
     hipLaunchKernelGGL(k_wgrad64<true>, dim3(nb), dim3(256), 0, s, n, rows, (const float *)nullptr,
                        (const float *)g.H[2], ds, w + kGnnWo, (const float *)g.H[1], (const float *)g.M[2], g.part);
-    sum(kWgLen, kWgLen, dw + kGnnWs3);
+    sum(std::true_type(), kWgLen, kWgLen, WgradRows{n, nullptr, g.H[2], ds, w + kGnnWo, g.H[1], g.M[2]}, dw + kGnnWs3);
     hipLaunchKernelGGL(k_back_dense<true>, dim3(tile_grid(n)), dim3(256), 0, s, n, (const float *)nullptr,
                        (const float *)g.H[2], ds, w + kGnnWo, w + kGnnWs3, w + kGnnWn3, dH, G);
     hipLaunchKernelGGL(k_agg64<true>, dim3(ga), dim3(256), 0, s, n, g.ptr, g.ind, g.at, (const float *)G, dH);
@@ -507,7 +540,8 @@ void gnn_backward(const GnnArgs &g, const float *w, const float *ds, float *dw, 
     hipLaunchKernelGGL(k_wgrad64<false>, dim3(nb), dim3(256), 0, s, n, rows, (const float *)dH, (const float *)g.H[1],
                        (const float *)nullptr, (const float *)nullptr, (const float *)g.H[0], (const float *)g.M[1],
                        g.part);
-    sum(kWgLen, 2 * kH * kH + kH, dw + kGnnWs2);
+    sum(std::false_type(), kWgLen, 2 * kH * kH + kH, WgradRows{n, dH, g.H[1], nullptr, nullptr, g.H[0], g.M[1]},
+        dw + kGnnWs2);
     hipLaunchKernelGGL(k_back_dense<false>, dim3(tile_grid(n)), dim3(256), 0, s, n, (const float *)dH,
                        (const float *)g.H[1], (const float *)nullptr, (const float *)nullptr, w + kGnnWs2, w + kGnnWn2,
                        dX, G);
@@ -515,7 +549,7 @@ void gnn_backward(const GnnArgs &g, const float *w, const float *ds, float *dw, 
     // layer 1
     hipLaunchKernelGGL(k_wgrad2, dim3(nb), dim3(256), 0, s, n, rows, (const float *)dX, (const float *)g.H[0],
                        (const float *)g.H0, (const float *)g.M1, g.part);
-    sum(kWgLen2, kWgLen2, dw + kGnnWs1);
+    sum(std::false_type(), kWgLen2, kWgLen2, WgradRows{}, dw + kGnnWs1);
 }
 
 }  // namespace rc
