@@ -115,6 +115,8 @@ static int rc_create_impl(rc_handle_t *out, const rc_options *opt)
         if (nm) h->nap_max = std::max(1, std::min(64, std::atoi(nm)));
         const char *tr = std::getenv("RCHOL_TAIL_ROWS");        // tail level width limit (1: no tail)
         if (tr) h->tail_max_rows = std::max(1, std::min(kTailMaxRows + 1, std::atoi(tr)));
+        const char *tm = std::getenv("RCHOL_TAIL_BYTES");       // memory of its dense matrices at most
+        if (tm) h->tail_bytes_max = (size_t)std::strtoull(tm, nullptr, 10);
         const char *sc = std::getenv("RCHOL_LIST_SEG_CAP");     // ready-list segment capacity limit (>= 1)
         if (sc) h->seg_cap_limit = std::max(1, std::atoi(sc));
         const char *at = std::getenv("RCHOL_ASYNC_TAIL");       // 0: narrow rounds stay round kernels
@@ -890,6 +892,8 @@ static int assemble(rc_handle_t h, double *ms_out, bool tail = true)
 {
     h->multi_ready = false;
     h->m_chunk_K = 0;
+    if (!tail)              // memory of a tail that is not built now
+        for (DevVec *v : {&h->tail_wf, &h->tail_wb}) v->release();
     hipStream_t s = h->stream;
     hipEvent_t e0, e1;
     RC_HIP(hipEventCreate(&e0));
@@ -1136,12 +1140,34 @@ static int assemble(rc_handle_t h, double *ms_out, bool tail = true)
         tb.m = ((h->ntail + tb.nb - 1) / tb.nb + kTailTile - 1) / kTailTile * kTailTile;
         tb.order = h->order.as<int>();
         h->tail_m = tb.m;
-        const size_t nt = (size_t)tb.ntail, dense = (size_t)tb.nb * (size_t)tb.m * (size_t)tb.m;
-        RC_HIP(h->tacc.ensure((size_t)tb.m * sizeof(T)));
-        RC_HIP(h->tf_ptr.ensure((nt + 1) * sizeof(int)));
-        RC_HIP(h->tb_ptr.ensure((nt + 1) * sizeof(int)));
-        RC_HIP(h->tail_d.ensure(dense * sizeof(double)));
-        RC_HIP(h->tail_e.ensure(dense * sizeof(double)));
+        // FP64: the matrices D and E that the inversion works in are its result.
+        // FP32: it rounds them to W; they lie in the elimination's fill pool, idle
+        // from here to the next factorization, as many blocks at a time as fit.
+        const size_t nt = (size_t)tb.ntail, block = (size_t)tb.m * (size_t)tb.m;
+        const size_t dense = (size_t)tb.nb * block * sizeof(T), one = 2 * block * sizeof(double);
+        // without the memory the factor does without a tail, as it does where the
+        // inverses' entries are not bounded
+        auto without_tail = [&]() -> int {
+            (void)hipEventDestroy(e0);
+            (void)hipEventDestroy(e1);
+            return assemble<T>(h, ms_out, false);
+        };
+        bool fits = 2 * dense <= h->tail_bytes_max;
+        auto need = [&](DevVec &v, size_t bytes) -> hipError_t {
+            if (!fits) return hipSuccess;
+            const hipError_t e = v.ensure(bytes);
+            if (e != hipErrorOutOfMemory) return e;
+            (void)hipGetLastError();
+            fits = false;
+            return hipSuccess;
+        };
+        RC_HIP(need(h->tail_wf, dense));
+        RC_HIP(need(h->tail_wb, dense));
+        if (sizeof(T) == 4) RC_HIP(need(h->pool, (size_t)std::min(tb.nb, kTailBatch) * one));
+        RC_HIP(need(h->tacc, (size_t)tb.m * sizeof(T)));
+        RC_HIP(need(h->tf_ptr, (nt + 1) * sizeof(int)));
+        RC_HIP(need(h->tb_ptr, (nt + 1) * sizeof(int)));
+        if (!fits) return without_tail();
         int *cnt_f = h->tmp_a.as<int>(), *cnt_b = cnt_f + nt + 1, *flag = cnt_b + nt + 1;
         RC_HIP(hipMemsetAsync(flag, 0, sizeof(int), s));
         launch_tail_count<T>(tb, true, fs, cnt_f, flag, s);
@@ -1152,31 +1178,32 @@ static int assemble(rc_handle_t h, double *ms_out, bool tail = true)
         RC_HIP(hipMemcpyAsync(&tot[0], h->tf_ptr.as<int>() + nt, sizeof(int), hipMemcpyDeviceToHost, s));
         RC_HIP(hipMemcpyAsync(&tot[1], h->tb_ptr.as<int>() + nt, sizeof(int), hipMemcpyDeviceToHost, s));
         RC_HIP(hipMemcpyAsync(&tot[2], flag, sizeof(int), hipMemcpyDeviceToHost, s));
-        RC_HIP(hipMemsetAsync(h->tail_d.p, 0, dense * sizeof(double), s));
         RC_HIP(hipStreamSynchronize(s));
-        if (tot[2] != 0) {
-            // a loaded factor whose columns are not bounded: every level is
-            // solved by substitution
-            (void)hipEventDestroy(e0);
-            (void)hipEventDestroy(e1);
-            return assemble<T>(h, ms_out, false);
+        if (tot[2] != 0) return without_tail();      // a loaded factor whose columns are not bounded
+        RC_HIP(need(h->tf_ind, (size_t)std::max(tot[0], 1) * sizeof(int)));
+        RC_HIP(need(h->tf_val, (size_t)std::max(tot[0], 1) * sizeof(T)));
+        RC_HIP(need(h->tb_ind, (size_t)std::max(tot[1], 1) * sizeof(int)));
+        RC_HIP(need(h->tb_val, (size_t)std::max(tot[1], 1) * sizeof(T)));
+        if (!fits) return without_tail();
+        const int batch = sizeof(T) == 4 ? (int)std::min<size_t>((size_t)tb.nb, h->pool.bytes / one) : tb.nb;
+        double *D = sizeof(T) == 4 ? h->pool.as<double>() : h->tail_wf.as<double>();
+        double *E = sizeof(T) == 4 ? D + (size_t)batch * block : h->tail_wb.as<double>();
+        for (int b0 = 0; b0 < tb.nb; b0 += batch) {
+            TailBuild part = tb;
+            part.tp0 = tb.tp0 + b0 * tb.m;
+            part.nb = std::min(batch, tb.nb - b0);
+            part.ntail = std::min(tb.ntail - b0 * tb.m, part.nb * tb.m);
+            RC_HIP(hipMemsetAsync(D, 0, (size_t)part.nb * block * sizeof(double), s));
+            launch_tail_split<T>(part, true, fs, h->tf_ptr.as<int>() + b0 * tb.m, h->tf_ind.as<int>(), h->tf_val.as<T>(),
+                                 D, s);
+            launch_tail_invert(part, D, E, s);
+            if constexpr (sizeof(T) == 4)
+                launch_tail_store<T>(part, D, h->tail_wf.as<T>() + (size_t)b0 * block,
+                                     h->tail_wb.as<T>() + (size_t)b0 * block, s);
+            else
+                launch_tail_store<T>(part, D, nullptr, h->tail_wb.as<T>(), s);
         }
-        RC_HIP(h->tf_ind.ensure((size_t)std::max(tot[0], 1) * sizeof(int)));
-        RC_HIP(h->tf_val.ensure((size_t)std::max(tot[0], 1) * sizeof(T)));
-        RC_HIP(h->tb_ind.ensure((size_t)std::max(tot[1], 1) * sizeof(int)));
-        RC_HIP(h->tb_val.ensure((size_t)std::max(tot[1], 1) * sizeof(T)));
-        launch_tail_split<T>(tb, true, fs, h->tf_ptr.as<int>(), h->tf_ind.as<int>(), h->tf_val.as<T>(),
-                             h->tail_d.as<double>(), s);
-        launch_tail_split<T>(tb, false, bs, h->tb_ptr.as<int>(), h->tb_ind.as<int>(), h->tb_val.as<T>(),
-                             h->tail_d.as<double>(), s);
-        launch_tail_invert(tb, h->tail_d.as<double>(), h->tail_e.as<double>(), s);
-        if constexpr (sizeof(T) == 4) {
-            RC_HIP(h->tail_wf.ensure(dense * sizeof(T)));
-            RC_HIP(h->tail_wb.ensure(dense * sizeof(T)));
-            launch_tail_store<T>(tb, h->tail_d.as<double>(), h->tail_wf.as<T>(), h->tail_wb.as<T>(), s);
-        } else {
-            launch_tail_store<T>(tb, h->tail_d.as<double>(), nullptr, h->tail_e.as<T>(), s);
-        }
+        launch_tail_split<T>(tb, false, bs, h->tb_ptr.as<int>(), h->tb_ind.as<int>(), h->tb_val.as<T>(), D, s);
     }
 
     // 5. A in position numbering, sliced ELL over 64-position tiles
@@ -1664,8 +1691,8 @@ SolveArgs solve_args(rc_handle_t h)
     a.tb_ptr = h->tb_ptr.as<int>();
     a.tb_ind = h->tb_ind.as<int>();
     a.tb_val = h->tb_val.p;
-    a.tail_wf = h->prec == 32 ? h->tail_wf.p : h->tail_d.p;
-    a.tail_wb = h->prec == 32 ? h->tail_wb.p : h->tail_e.p;
+    a.tail_wf = h->tail_wf.p;
+    a.tail_wb = h->tail_wb.p;
     a.tacc = h->tacc.p;
     a.nlevels = h->nlevels;
     a.spin_ticks = h->spin_ticks;
@@ -1980,8 +2007,8 @@ static int multi_args(rc_handle_t h, int k, MultiArgs &a)
     a.tb_ptr = h->tb_ptr.as<int>();
     a.tb_ind = h->tb_ind.as<int>();
     a.tb_val = h->tb_val.p;
-    a.tail_wf = h->prec == 32 ? h->tail_wf.p : h->tail_d.p;
-    a.tail_wb = h->prec == 32 ? h->tail_wb.p : h->tail_e.p;
+    a.tail_wf = h->tail_wf.p;
+    a.tail_wb = h->tail_wb.p;
     a.tacc = h->m_tacc.p;
     a.tail_part = h->m_tpart.p;
     a.tail_arrive = h->m_tarr.as<unsigned int>();
