@@ -892,8 +892,10 @@ static int assemble(rc_handle_t h, double *ms_out, bool tail = true)
 {
     h->multi_ready = false;
     h->m_chunk_K = 0;
-    if (!tail)              // memory of a tail that is not built now
+    if (!tail) {            // of a tail that is not built now: its memory, its width
         for (DevVec *v : {&h->tail_wf, &h->tail_wb}) v->release();
+        h->tail_width = 0;
+    }
     hipStream_t s = h->stream;
     hipEvent_t e0, e1;
     RC_HIP(hipEventCreate(&e0));

@@ -48,6 +48,22 @@ def test_tail_without_memory(rc, wl, prec, monkeypatch):
         s.close()
 
 
+@pytest.mark.parametrize("limit,width", [(0, 0), (None, 1)])
+def test_autotune_reports_the_tail_that_is_there(rc, wl, limit, width, monkeypatch):
+    """tail_max_rows is 0 where every candidate's tail was left out."""
+    print(f"[gpu] autotune tail bytes={limit}", flush=True)
+    if limit is not None:
+        monkeypatch.setenv("RCHOL_TAIL_BYTES", str(limit))
+    s = rc.Solver(device=0, seed=5, precision=64)
+    s.set_triplets(*wl.grid_laplacian((40, 41), "uniform_0.5_2", seed=3))
+    s.order(rc.ORDER_NNZ_SORT, 1)
+    s.factor()
+    s.set_rhs(s.make_rhs(rc.RHS_NORMAL_PROJECTED, 3))
+    st = s.autotune(2)
+    assert min(st["tail_max_rows"], 1) == width
+    s.close()
+
+
 @pytest.mark.parametrize("dims", [(140, 150), (160, 204)], ids=lambda d: f"{d[0] * d[1]}")
 def test_many_blocks_inverted_in_parts(rc, orc, wl, dims, monkeypatch):
     """FP32: eleven and sixteen blocks, more than are inverted at a time; one
