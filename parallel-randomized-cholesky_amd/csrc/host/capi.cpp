@@ -1279,6 +1279,32 @@ static double factor_bytes(rc_handle_t h)
            s * (double)h->nf;
 }
 
+// A resident right-hand side (and the last solution) lies in the row order of the
+// factor it was set under.  Factors of one kind have one order; under another
+// kind's the vectors move: to the user's numbering before the assembly, to the new
+// positions after it.  (r is free between solves.)
+enum { kEliminated = 1, kIc0 = 2, kLoaded = 3 };
+static bool carry_out(rc_handle_t h, int kind)
+{
+    if (!h->rhs_set || (kind == h->factor_kind && kind != kLoaded)) return false;
+    if (!h->factored) {                  // the last assembly did not end: no order to move from
+        h->rhs_set = false;
+        return false;
+    }
+    launch_scatter(h->b.as<double>(), h->idx_user.as<int>(), h->bu.as<double>(), h->ns, h->stream);
+    launch_scatter(h->x.as<double>(), h->idx_user.as<int>(), h->r.as<double>(), h->ns, h->stream);
+    h->rhs_set = false;
+    return true;
+}
+static void carry_in(rc_handle_t h, int kind, bool carried)
+{
+    h->factor_kind = kind;
+    if (!carried) return;
+    launch_gather(h->bu.as<double>(), h->idx_user.as<int>(), h->b.as<double>(), h->ns, h->stream);
+    launch_gather(h->r.as<double>(), h->idx_user.as<int>(), h->x.as<double>(), h->ns, h->stream);
+    h->rhs_set = true;
+}
+
 static int rc_factor_impl(rc_handle_t h, rc_factor_stats *st)
 {
     RC_CHECK_HANDLE();
@@ -1291,6 +1317,7 @@ static int rc_factor_impl(rc_handle_t h, rc_factor_stats *st)
     std::memset(&h->fstats, 0, sizeof(h->fstats));
     double fms = 0.0, ams = 0.0;
     int regrow = 0;
+    const bool carried = carry_out(h, kEliminated);
     h->factored = false;
     h->m_solved = false;
     h->m_ran = false;
@@ -1300,6 +1327,7 @@ static int rc_factor_impl(rc_handle_t h, rc_factor_stats *st)
     h->prec = h->opt.factor_precision;
     rc = (h->prec == 32) ? assemble<float>(h, &ams) : assemble<double>(h, &ams);
     if (rc != RC_OK) return rc;
+    carry_in(h, kEliminated, carried);
     h->fstats.n = h->nf;
     h->fstats.nnz_lower = h->nnz_low;
     h->fstats.nlevels = h->nlevels;
@@ -1327,6 +1355,7 @@ static int rc_factor_ic0_impl(rc_handle_t h, rc_factor_stats *st)
     if (rc != RC_OK) return rc;
     const double prep_ms = had ? 0.0 : h->prepare_ms;
     std::memset(&h->fstats, 0, sizeof(h->fstats));
+    const bool carried = carry_out(h, kIc0);
     h->factored = false;
     h->m_solved = false;
     h->m_ran = false;
@@ -1400,6 +1429,7 @@ static int rc_factor_ic0_impl(rc_handle_t h, rc_factor_stats *st)
     double ams = 0.0;
     rc = (h->prec == 32) ? assemble<float>(h, &ams) : assemble<double>(h, &ams);
     if (rc != RC_OK) return rc;
+    carry_in(h, kIc0, carried);
     h->fstats.n = nf;
     h->fstats.nnz_lower = h->nnz_low;
     h->fstats.nnz_factor = h->nnz_low + nf;
@@ -1602,9 +1632,12 @@ static int rc_load_factor_impl(rc_handle_t h, const char *prefix)
     h->fstats.zero_pivots = zp;
     h->prec = h->opt.factor_precision;
     double ams = 0.0;
+    const bool carried = carry_out(h, kLoaded);
+    h->factored = false;
     invalidate_graph(h);
     rc = (h->prec == 32) ? assemble<float>(h, &ams) : assemble<double>(h, &ams);
     if (rc != RC_OK) return rc;
+    carry_in(h, kLoaded, carried);
     h->fstats.n = nf;
     h->fstats.nnz_lower = h->nnz_low;
     h->fstats.nlevels = h->nlevels;

@@ -145,6 +145,7 @@ struct rc_handle_s {
 
     // factor result: CSR of L^T in the factored numbering (export / dump)
     bool factored = false;
+    int factor_kind = 0;            // elimination, IC(0) or loaded: kinds differ in their row order
     int prec = 64;
     DevVec lt_ptr, lt_ind, lt_val, diagT;
     // solve layout: level-order positions, sliced ELL of L, L^T and A
