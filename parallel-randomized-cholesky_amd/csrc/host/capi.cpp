@@ -1634,6 +1634,8 @@ static int rc_load_factor_impl(rc_handle_t h, const char *prefix)
     double ams = 0.0;
     const bool carried = carry_out(h, kLoaded);
     h->factored = false;
+    h->m_solved = false;
+    h->m_ran = false;
     invalidate_graph(h);
     rc = (h->prec == 32) ? assemble<float>(h, &ams) : assemble<double>(h, &ams);
     if (rc != RC_OK) return rc;
