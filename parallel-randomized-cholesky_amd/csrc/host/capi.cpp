@@ -2000,6 +2000,7 @@ static int multi_args(rc_handle_t h, int k, MultiArgs &a)
         }
     }
     if (h->m_chunk_K != K) {              // chunks of the wide levels for this many right-hand sides
+        h->m_chunk_K = 0;                 // (an error below leaves none)
         const int L = K / multi_lane_rhs(K, (int)sz), ng = h->bulk_segs;
         const int *seg = h->seg_work.as<int>();
         RC_HIP(h->m_ccnt.ensure(((size_t)ng + 1) * sizeof(int)));
