@@ -1660,20 +1660,22 @@ static int reduction_blocks(rc_handle_t h)
 }
 
 // Persistent sweep workgroups for `rows` rows of k values: the autotuner's
-// choice, else one per CU, two from 1.5 M values, and four for many right-hand
-// sides from 32 M values, or from 6 M with 64 of them (a chunk is then a few
-// rows).  More of them hold chunks far ahead of the front, and their polls slow
-// it down; wide levels want more in flight.  Forward / backward sweep, us, at
-// 256 / 512 workgroups: 701x699 107/111, 115/119; 101x83x89 339/360, 353/372;
-// 128^3 SDDM 597/614, 564/573; 192^3 learned 980/932, 940/866.  Solves, ms, at
-// 512 / 1024: 385x384 x 32 18.7, 18.8, x 64 25.9, 24.9; 47x48x45 x 32 32.8, 33.6,
-// x 64 41.3, 40.8; 80x81x82 x 16 45.2, 46.0.
+// choice, else one per CU, two from 1.5 M values, and four from 9 M with several
+// right-hand sides.  More of them hold chunks far ahead of the front, and their
+// polls slow it down; wide levels want more in flight.  Forward / backward sweep,
+// us, at 256 / 512 workgroups: 701x699 107/111, 115/119; 101x83x89 339/360,
+// 353/372; 128^3 SDDM 597/614, 564/573; 192^3 learned 980/932, 940/866.  PCG of k
+// right-hand sides to 1e-8 (FP32 factor, without the copies), ms, at 512 / 1024:
+// 1 M values 250x256 x 16 12.3, 12.8; 4.7 M 385x384 x 32 17.9, 18.1; 6.4 M 317x316
+// x 64 19.8, 19.8 and 47x48x45 x 64 23.3, 23.2; 8 M 1000x1002 x 8 53.9, 47.8,
+// 700x702 x 16 30.9, 31.4, 500x504 x 32 27.9, 27.8, 80x81x82 x 16 41.8, 42.1;
+// 9.5 M 385x384 x 64 24.9, 24.0; 16 M 1000x1002 x 16 63.4, 57.9, 64x63x62 x 64 44.6,
+// 42.1; 32 M 1000x1002 x 32 111, 93, 80x81x82 x 64 84.0, 74.4.
 static int sweep_grid(rc_handle_t h, int rows, int k)
 {
     if (h->sweep_blocks > 0) return h->sweep_blocks;
     const double values = (double)rows * k;
-    const bool four = k > 1 && (values > 3.2e7 || (k >= 64 && values > 6e6));
-    const int per_cu = values < 1.5e6 ? 1 : (four ? 4 : 2);
+    const int per_cu = values < 1.5e6 ? 1 : (k > 1 && values > 9e6 ? 4 : 2);
     return std::min(h->sweep_blocks_max, per_cu * h->cus);
 }
 
