@@ -42,7 +42,7 @@ constexpr int kAqHead = 0, kAqTail = 32, kAqWords = 64;
 constexpr int kFillLists = 64;
 
 // Columns with more than the round kernel's LDS capacity (128 entries) are
-// deferred to a second kernel of the same round: kBigGrid one-wave workgroups
+// deferred to a second kernel of the same round: kBigGrid eight-wave workgroups
 // with kBigCap entries of LDS each.  A round of at most kBigGrid columns is
 // eliminated by that second kernel entirely.
 constexpr int kBigGrid = 256;
@@ -313,7 +313,7 @@ struct SolveArgs {
     double *partials;             // >= 2 * reduce blocks
     unsigned int *ctr_fwd, *ctr_bwd;
     int reduce_blocks;
-    int sweep_blocks;             // persistent sweep workgroups (occupancy-sized)
+    int sweep_blocks;             // persistent sweep workgroups
     // level split: chunks [0, bulk_chunks) belong to the wide levels and run
     // on the persistent grid; levels [tail_level, nlevels) form the tail
     int nchunks, bulk_chunks, tail_level, nlevels;

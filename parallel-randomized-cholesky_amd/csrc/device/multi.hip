@@ -344,7 +344,8 @@ __device__ __forceinline__ void row_update(const MultiArgs &a, size_t o, const d
 // level order, three ahead (the same protocol and the same argument against
 // deadlock as k_sweep_bulk); while chunk i is solved, chunk i + 1's descriptor,
 // row bounds and entries are loaded into registers, so a chunk costs one
-// gather round trip.  Entries go through LDS: all lanes of a row read them.
+// gather round trip and, as there, thread 0's claim.  Entries go through LDS: all
+// lanes of a row read them.
 template <typename T, bool kFwd, int V>
 __global__ void __launch_bounds__(kMSweepThreads) k_msweep(MultiArgs a, const double *p_cur, int update_rx)
 {

@@ -404,8 +404,10 @@ __device__ __forceinline__ void bwd_chunk(const SolveArgs &a, int4 m, int t, con
 // Claims run ahead of the work: while chunk i is processed, the workgroup
 // already holds chunk i+1's descriptor and its first kBulkPref index/value
 // slices (loaded before chunk i's dependency gathers, so both round trips
-// overlap), loads chunk i+2's descriptor, and thread 0 has the claim of chunk
-// i+3 in flight, so no round trip is exposed between chunks.  Holding claims
+// overlap) and loads chunk i+2's descriptor; after it, thread 0 takes the claim of
+// chunk i+3.  That claim is the round trip that remains between chunks: its
+// result is made a chunk number at once, so thread 0 waits for it before the
+// barrier, and its wave for the values it published.  Holding claims
 // ahead cannot deadlock: the smallest unfinished claimed chunk is always some
 // workgroup's current chunk, and its dependencies are all earlier chunks.
 template <typename T, bool kFwd>
@@ -479,11 +481,10 @@ __global__ void __launch_bounds__(kSweepThreads) k_sweep_bulk(SolveArgs a, const
         if (kFwd) fwd_chunk<T>(a, m_cur, t, alpha, p_cur, update_rx, j_cur, l_cur);
         else bwd_chunk<T>(a, m_cur, t, j_cur, l_cur);
         // made uniform before thread 0 issues new loads, so that waiting for
-        // it does not also wait for them
+        // it does not also wait for them (it does for the published values)
         const int4 m_nxt2_u = uniform(m_nxt2);
         if (t == 0) {
-            // publish the claim taken a chunk ago, take the next one; both
-            // this atomic and the status load complete during the next chunk
+            // publish the claim taken a chunk ago, take the next one
             s_claim[par] = c_pend;              // slots alternate, so one barrier suffices
             s_stop = (int)st_pend;
             c_pend = (int)atomicAdd(ctr, 1u) * nq + q;

@@ -166,7 +166,7 @@ struct rc_handle_s {
     int tail_max_rows = -1;         // width limit of its levels; -1: chosen by estimated time, 0: no tail
     size_t tail_bytes_max = (size_t)-1;   // RCHOL_TAIL_BYTES: a tail whose dense matrices take more is not built
     int tail_width = 0;             // widest tail level of the current factor + 1 (0: no tail)
-    int nap_max = 1;                // measured best: poll again after one s_sleep 2
+    int nap_max = 1;                // longest back-off between polls; 1: none, measured best
     int seg_cap_limit = 0;          // > 0: ready-list segments hold at most this many entries (exercises the overflow region)
     int tail_pos0 = 0, ntail = 0, tail_nb = 0, tail_m = 0;
     DevVec tf_ptr, tf_ind, tf_val, tb_ptr, tb_ind, tb_val, tacc, tail_wf, tail_wb;
