@@ -347,12 +347,24 @@ __global__ void __launch_bounds__(256) k_wgrad2(int n, int rows_per_wave, const 
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const float dv = vb + u < v1 ? d[u] : 0.f;
-            const bool on = dv != 0.f;                   // a zero takes nothing, also from an infinity
-            g[0] = fmaf(dv, on ? bf16r(x[u].x) : 0.f, g[0]);
-            g[1] = fmaf(dv, on ? bf16r(x[u].y) : 0.f, g[1]);
-            g[2] = fmaf(dv, on ? bf16r(m[u].x) : 0.f, g[2]);
-            g[3] = fmaf(dv, on ? bf16r(m[u].y) : 0.f, g[3]);
+            g[0] = fmaf(dv, bf16r(x[u].x), g[0]);
+            g[1] = fmaf(dv, bf16r(x[u].y), g[1]);
+            g[2] = fmaf(dv, bf16r(m[u].x), g[2]);
+            g[3] = fmaf(dv, bf16r(m[u].y), g[3]);
             g[4] += dv;
+        }
+    }
+    // 0 times an infinity is NaN: sums that are not finite are formed again, zeros
+    // skipped (selecting in the loop took 6 us)
+    if (!__builtin_isfinite(g[0]) || !__builtin_isfinite(g[1]) || !__builtin_isfinite(g[2]) || !__builtin_isfinite(g[3])) {
+        g[0] = g[1] = g[2] = g[3] = 0.f;
+        for (int v = v0; v < v1; ++v) {
+            const float d = H[(size_t)v * kH + lane] > 0.f ? dH[(size_t)v * kH + lane] : 0.f;
+            if (d == 0.f) continue;
+            g[0] = fmaf(d, bf16r(X[(size_t)v * 2]), g[0]);
+            g[1] = fmaf(d, bf16r(X[(size_t)v * 2 + 1]), g[1]);
+            g[2] = fmaf(d, bf16r(M[(size_t)v * 2]), g[2]);
+            g[3] = fmaf(d, bf16r(M[(size_t)v * 2 + 1]), g[3]);
         }
     }
 #pragma unroll
@@ -379,7 +391,7 @@ struct WgradRows {
 // its share of the partials in order, then the eight in order.  A row whose dZ
 // is zero contributes nothing, whatever its inputs hold: a weight's sum that is
 // not finite is formed again from the rows, zeros skipped.  (Watching for such
-// inputs in k_wgrad64 cost it its registers: 325 -> 331-350 us a gradient.)
+// inputs in k_wgrad64 cost it its registers: 321 -> 331-350 us a gradient.)
 template <bool kLast>
 __global__ void __launch_bounds__(256) k_sum_partials(const float *part, int nblocks, int stride, int len, WgradRows w,
                                                       float *out)
@@ -400,27 +412,25 @@ __global__ void __launch_bounds__(256) k_sum_partials(const float *part, int nbl
         }
     red[s][o] = t;
     __syncthreads();
+    if (threadIdx.x >= kWave) return;
     t = red[0][o];
     for (int q = 1; q < 8; ++q) t += red[q][o];
     const bool again = w.H && i < 2 * kH * kH && !__builtin_isfinite(t);
-    if (__syncthreads_or(again)) {
+    if (ballot(again)) {                                 // the wave's halves take half of the rows each
+        float r = 0.f;
         if (again) {
             const float *in = i < kH * kH ? w.X : w.M;
             const int row = (i / kH) % kH, col = i % kH;
             const float wl = kLast ? bf16r(w.wo[row]) : 0.f;
-            const int share = (w.n + 7) / 8, v1 = min(w.n, (s + 1) * share);
-            t = 0.f;
-            for (int v = s * share; v < v1; ++v) {
+            const int half = w.n / 2, v1 = s == 0 ? half : w.n;
+#pragma unroll 4
+            for (int v = s == 0 ? 0 : half; v < v1; ++v) {
                 const float g = kLast ? w.ds[v] * wl : w.dH[(size_t)v * kH + row];
-                if (w.H[(size_t)v * kH + row] > 0.f && g != 0.f) t = fmaf(g, bf16r(in[(size_t)v * kH + col]), t);
+                if (w.H[(size_t)v * kH + row] > 0.f && g != 0.f) r = fmaf(g, bf16r(in[(size_t)v * kH + col]), r);
             }
-            red[s][o] = t;
         }
-        __syncthreads();
-        if (again) {
-            t = red[0][o];
-            for (int q = 1; q < 8; ++q) t += red[q][o];
-        }
+        r += __shfl_xor(r, 32, kWave);
+        if (again) t = r;
     }
     if (s == 0 && i < len) out[i] = t;
 }
