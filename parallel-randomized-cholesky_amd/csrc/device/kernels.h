@@ -235,7 +235,8 @@ void launch_sweep_layout(int nchunks, const int *cnt, const int *width, int *sli
 constexpr int kTailBlock = 2048;
 constexpr int kTailTile = 64;               // base block of the inversion; m is a multiple of it
 constexpr int kTailMaxRows = 16 * kTailBlock;
-constexpr int kTailBatch = 8;               // FP32: blocks inverted at a time at least (or all of them)
+constexpr int kTailBatch = 4;               // FP32: blocks inverted at a time at least (or all of them); the
+                                            // default grid's fill pool holds that many without growing
 struct TailBuild {
     int ntail, tp0, m, nb;                  // rows, first position, rows per block, blocks
     const int *order;
